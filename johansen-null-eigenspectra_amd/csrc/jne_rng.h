@@ -61,21 +61,24 @@ __device__ __forceinline__ u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_
 // (e ln2_lo + lnm), lnm = f + f^2 Q(f), f = m - 1 (exact; Horner in float32
 // with fixed coefficients).  Positive normal floats order as their bit
 // patterns and adding k 2^23 to a pattern scales the value by 2^k, so u in
-// (2C 2^(e-1), 2C 2^e] gives -e = floor((bits(2C) - bits(u)) / 2^23) (one
-// subtraction, one shift) and m = u 2^-e (v_ldexp_f32): the (m, e) of the
-// split by frexp (mant in [1/2, 1); m = 2 mant, e = exp - 1 when mant <= C)
-// for every u of the range.  The return value is 2L computed at twice the
-// scale: h = 2f = 2m - 2, Horner in h with coefficients c_k 2^(-k-1) (= Q/2,
+// (2C 2^(e-1), 2C 2^e] gives -e = floor((bits(2C) - bits(u)) / 2^23): one
+// subtraction, and the low 23 bits masked off leave -e 2^23, which added to
+// the pattern of u is that of m, and whose float conversion is -e scaled by
+// 2^23 (the constants of the ln 2 terms carry 2^-23).  That is the (m, e) of
+// the split by frexp (mant in [1/2, 1); m = 2 mant, e = exp - 1 when mant <= C)
+// for every u of the range.  The mask and the integer add issue at twice the
+// rate of a shift with v_ldexp_f32.  The return value is 2L computed at twice
+// the scale: h = 2f = 2m - 2, Horner in h with coefficients c_k 2^(-k-1) (= Q/2,
 // every partial sum exactly 2^(-k-1) times the one in f), 2 lnm = h + h^2 Q/2
 // and the ln 2 terms doubled, -e entering with their signs turned.  Scaling
 // by a power of two commutes with rounding (no partial result is subnormal),
 // so this is exactly 2L, +0 at u = 1, and -(2L) is bit for bit -2 * L.
 __device__ __forceinline__ float two_ln(float u) {
 #pragma clang fp contract(off)
-  const int32_t ub = (int32_t)__float_as_uint(u);
-  const int32_t ne = ((int32_t)0x3FB504F3 - ub) >> 23;  // 0x3FB504F3 = bits(2C); ne = -e
-  const float m = __builtin_amdgcn_ldexpf(u, ne);  // exact: m is a normal float
-  const float h = __builtin_fmaf(m, 2.0f, -2.0f);  // 2f, exact
+  const uint32_t ub = __float_as_uint(u);
+  const uint32_t ne23 = (0x3FB504F3u - ub) & 0xFF800000u;  // 0x3FB504F3 = bits(2C); -e 2^23
+  const float m = __uint_as_float(ub + ne23);              // exact: m is a normal float
+  const float h = __builtin_fmaf(m, 2.0f, -2.0f);          // 2f, exact
   float q = 0x1.15425cp-14f;
   q = __builtin_fmaf(q, h, -0x1.d962f2p-13f);
   q = __builtin_fmaf(q, h, 0x1.e3d33ap-12f);
@@ -88,24 +91,27 @@ __device__ __forceinline__ float two_ln(float u) {
   q = __builtin_fmaf(q, h, -0x1p-2f);
   const float h2 = h * h;
   const float lnm2 = __builtin_fmaf(h2, q, h);
-  const float nef = (float)ne;
-  return __builtin_fmaf(nef, -0x1.62e43p+0f, __builtin_fmaf(nef, 0x1.05c61p-28f, lnm2));
+  const float nef = (float)(int32_t)ne23;  // exact: at most 33 * 2^23
+  return __builtin_fmaf(nef, -0x1.62e43p-23f, __builtin_fmaf(nef, 0x1.05c61p-51f, lnm2));
 }
 
-// Correctly rounded sqrt(y) for y = +-0 or y in [2^-96, 2^126]: v_sqrt_f32
-// (within 1 ulp) and one correction step to the neighbour whose residual
-// has the right sign.  A general sqrtf adds scaling for tiny inputs and a
-// special-value check, neither needed on this range.
+// Correctly rounded sqrt(y) for y = -0 or y = -two_ln(u1) of the stream:
+// g = y rsq(y) and one Newton step, g + (y - g^2) rsq(y)/2 (Markstein's final
+// step), whose error is about 1.5 times the square of v_rsq_f32's.  That does
+// not prove the last bit by itself: it was compared, on the GPU, with the
+// neighbour-residual form (v_sqrt_f32, then the neighbour whose residual has
+// the right sign) and with sqrt in double for every radius word (all 2^32):
+// no difference.  6 instructions instead of 9, without the half-rate compares
+// and selects (an instruction's issue measured 2.6 SIMD cycles at the full and
+// 4.4 at the half rate, 8.4 for v_sqrt_f32 and v_rsq_f32): with the exponent
+// split above, the stream alone went from 428 to 404 SIMD cycles per Philox
+// call at 4 waves per SIMD.  The clamp keeps
+// rsq(0) finite: y = -0 gives g = -0, the residual -0 and the result -0.
 __device__ __forceinline__ float sqrt_cr(float y) {
 #pragma clang fp contract(off)
-  const float s = __builtin_amdgcn_sqrtf(y);
-  const float dn = __uint_as_float(__float_as_uint(s) - 1u);
-  const float up = __uint_as_float(__float_as_uint(s) + 1u);
-  const float rdn = __builtin_fmaf(-dn, s, y);
-  const float rup = __builtin_fmaf(-up, s, y);
-  float r = rdn <= 0.0f ? dn : s;
-  r = rup > 0.0f ? up : r;
-  return r;
+  const float r = __builtin_amdgcn_rsqf(__builtin_fmaxf(y, 0x1p-30f));
+  const float g = y * r;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, y), 0.5f * r, g);
 }
 
 // Two Philox words -> two N(0,1) floats.
