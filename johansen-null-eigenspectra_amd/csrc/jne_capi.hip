@@ -88,6 +88,9 @@ struct jne_ctx {
   // device scratch: M = W^T W of one chunk for the two-kernel eigen solve
   double* d_m = nullptr;
   size_t m_bytes = 0;
+  // device scratch: the blocks' sums of batches split over their walks' blocks
+  double* d_part = nullptr;
+  size_t part_bytes = 0;
   // the scratch is shared by every call: a call on another stream than the
   // previous one first waits for the previous call's last use of it
   hipEvent_t scratch_free = nullptr;
@@ -225,23 +228,36 @@ bool auto_uses_mfma(int dim, uint32_t steps) {
   return false;
 }
 
+int resolve_precision(int dim, uint32_t steps, int precision) {
+  if (precision != JNE_PREC_AUTO) return precision;
+  return auto_uses_mfma(dim, steps) ? JNE_PREC_MFMA_FP16X2 : JNE_PREC_FP64;
+}
+
+// Scratch for splitting a launch of n walks over their blocks (0: not split).
+size_t part_doubles_for(int dim, uint32_t steps, int precision, size_t n) {
+  if (n == 0 || dim > jne::kMaxDim || resolve_precision(dim, steps, precision) != JNE_PREC_FP64) return 0;
+  return jne::fp64_part_doubles(dim, steps, (uint32_t)n);
+}
+
 // Enqueues the walk kernels for n walks on st, in chunks of at most `chunk`
-// walks over the scratch `acc` (chunk * moment_count(dim) doubles) and `mbuf`
-// (chunk * eigen_m_count(dim) doubles): per chunk one moment pass, then the
+// walks over the scratch `acc` (chunk * moment_count(dim) doubles), `mbuf`
+// (chunk * eigen_m_count(dim) doubles) and `part` (part_doubles; may be NULL,
+// see part_doubles_for): per chunk one moment pass, then the
 // eigen solve of each of the n_models models into its output (the moments of
 // a walk do not depend on the model).  timed: record the launches when
 // profiling is enabled.
 int launch_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_t steps, uint32_t rng_stream,
                  const uint32_t* d_seeds, const double* d_z, size_t n, int precision, double* const* d_outs,
-                 hipStream_t st, double* acc, double* mbuf, size_t chunk, bool timed) {
-  if (precision == JNE_PREC_AUTO) precision = auto_uses_mfma(dim, steps) ? JNE_PREC_MFMA_FP16X2 : JNE_PREC_FP64;
+                 hipStream_t st, double* acc, double* mbuf, double* part, size_t part_doubles, size_t chunk,
+                 bool timed) {
+  precision = resolve_precision(dim, steps, precision);
   for (size_t off = 0; off < n; off += chunk) {
     const uint32_t cn = (uint32_t)std::min(chunk, n - off);
     const uint32_t* s = d_seeds ? d_seeds + off : nullptr;
     const double* z = d_z ? d_z + off * (size_t)steps * dim : nullptr;
     auto moments = [&] {
       if (dim > jne::kMaxDim) return jne::launch_walk_moments_wide(dim, s, z, rng_stream, steps, cn, acc, cn, st);
-      if (precision == JNE_PREC_FP64) return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, st);
+      if (precision == JNE_PREC_FP64) return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
       return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, st);
     };
     if (timed)
@@ -274,11 +290,18 @@ int run_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_t s
   if (rc) return rc;
   rc = ensure(ctx, (void**)&ctx->d_m, &ctx->m_bytes, chunk * (size_t)jne::eigen_m_count(dim) * sizeof(double));
   if (rc) return rc;
+  // without room for the blocks' sums the launches are not split
+  const size_t part = std::max(part_doubles_for(dim, steps, precision, chunk),
+                               part_doubles_for(dim, steps, precision, n % chunk));
+  if (ensure(ctx, (void**)&ctx->d_part, &ctx->part_bytes, part * sizeof(double)) != JNE_OK) {
+    (void)hipGetLastError();
+    ctx->err.clear();
+  }
   if (!ctx->scratch_free) JNE_HIP_CHECK(ctx, hipEventCreateWithFlags(&ctx->scratch_free, hipEventDisableTiming));
   if (ctx->scratch_stream && ctx->scratch_stream != st)
     JNE_HIP_CHECK(ctx, hipStreamWaitEvent(st, ctx->scratch_free, 0));
   if ((rc = launch_walks(ctx, models, n_models, dim, steps, rng_stream, d_seeds, d_z, n, precision, d_outs, st,
-                         ctx->d_acc, ctx->d_m, chunk, true)))
+                         ctx->d_acc, ctx->d_m, ctx->d_part, ctx->part_bytes / sizeof(double), chunk, true)))
     return rc;
   JNE_HIP_CHECK(ctx, hipEventRecord(ctx->scratch_free, st));
   ctx->scratch_stream = st;
@@ -365,6 +388,7 @@ void jne_destroy(jne_ctx* ctx) {
   for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
   if (ctx->d_acc) (void)hipFree(ctx->d_acc);
   if (ctx->d_m) (void)hipFree(ctx->d_m);
+  if (ctx->d_part) (void)hipFree(ctx->d_part);
   if (ctx->scratch_free) (void)hipEventDestroy(ctx->scratch_free);
   if (ctx->d_in) (void)hipFree(ctx->d_in);
   if (ctx->d_out) (void)hipFree(ctx->d_out);
@@ -448,7 +472,8 @@ int jne_eigenvalues_by_seed_device_noalloc(jne_ctx* ctx, int model, int dim, uin
   if (!d_seeds || !d_out) return set_err(ctx, JNE_ERR_INVALID_ARG, "d_seeds/d_out must not be NULL");
   const size_t mc = (size_t)jne::moment_count(dim);
   const size_t per_walk = mc + (size_t)jne::eigen_m_count(dim);
-  const size_t cap = (JNE_NOALLOC_SCRATCH_BYTES / sizeof(double)) / per_walk;
+  const size_t cap_doubles = JNE_NOALLOC_SCRATCH_BYTES / sizeof(double);
+  const size_t cap = cap_doubles / per_walk;
   if (n > cap)
     return set_err(ctx, JNE_ERR_INVALID_ARG,
                    "jne_eigenvalues_by_seed_device_noalloc: %zu walks exceed the scratch of %zu walks at dim %d "
@@ -458,8 +483,10 @@ int jne_eigenvalues_by_seed_device_noalloc(jne_ctx* ctx, int model, int dim, uin
   JNE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   double* const acc = ctx->noalloc_scratch;
   double* const outs[1] = {d_out};
+  // what n leaves of the scratch takes the blocks' sums when it is enough
   return launch_walks(ctx, &model, 1, dim, steps, rng_stream, d_seeds, nullptr, n, precision, outs,
-                      stream_of(ctx, hip_stream), acc, acc + mc * n, n, false);
+                      stream_of(ctx, hip_stream), acc, acc + mc * n, acc + per_walk * n, (cap_doubles - per_walk * n), n,
+                      false);
 }
 
 int jne_eigenvalues_from_normals(jne_ctx* ctx, int model, int dim, uint32_t steps, const double* z, size_t n,

@@ -17,16 +17,18 @@ constexpr uint32_t kMaxSteps = 1u << 30;  // steps per walk accepted by the C AB
 static_assert((uint64_t)kMaxDim * kMaxSteps / 4 < (1ull << 32), "32-bit Philox counters");
 
 // Per-dim shape of the FP64 moment kernel: lanes per walk (L) and target
-// waves per SIMD (the register cap).  Measured on MI355X (model 4, T = 10^4).
-// Dims with L = 1 run the register-only kernel (its own wave targets); one
-// lane per walk at dims 7 and 8 would need a wave per SIMD and ran 11% and
-// 36% slower than the LDS-staged shapes.
+// waves per SIMD (the register cap).  Measured on MI355X at T = 4,000 to 10^4.
+// Dims with L = 1 run the register-only kernel (its own wave targets): at
+// dim 7 its 105 sums fit two waves per SIMD (131,072 walks at T = 10^4: 11.0
+// ms against 14.4 with seven lanes per walk); dim 8's 132 would not.
+// Alternatives within 2%: (2, 3) at dim 8, (3, 2) at dim 9; slower: (2, 2) at
+// dim 10 by 35%, (3, 2) at dims 11 and 12 by 8-11%.
 struct Fp64Shape {
   int lanes, waves;
 };
 #ifndef JNE_FP64_SHAPES
 #define JNE_FP64_SHAPES \
-  {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {7, 4}, {2, 2}, {9, 4}, {5, 3}, {4, 2}, {4, 2}
+  {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {2, 2}, {9, 4}, {5, 3}, {4, 2}, {4, 2}
 #endif
 constexpr Fp64Shape kFp64Shapes[12] = {JNE_FP64_SHAPES};
 constexpr int lanes_for_dim(int d) { return kFp64Shapes[d - 1].lanes; }
@@ -103,8 +105,14 @@ constexpr int moment_count(int d) { return 2 * d * d + 6 * d; }
 
 constexpr int num_eigenvalues(int model, int d) { return (model == 1 || model == 3) ? d + 1 : d; }
 
+// part: part_doubles of scratch for the blocks' sums of batches that are split
+// over their walks' blocks (jne_blocks.h); NULL or too small: not split (the
+// same bits)
 hipError_t launch_walk_moments_fp64(int d, const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                    uint32_t n, double* acc, size_t ld, hipStream_t st);
+                                    uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                    hipStream_t st);
+// doubles of that scratch for n walks: 0 where the batch is not split
+size_t fp64_part_doubles(int d, uint32_t T, uint32_t n);
 // the segment-split pass: the MFMA precisions and the compensated FP32 VALU check
 hipError_t launch_walk_moments_mfma(int d, int precision, const uint32_t* seeds, const double* zin,
                                     uint32_t rng_stream, uint32_t T, uint32_t n, double* acc, size_t ld,

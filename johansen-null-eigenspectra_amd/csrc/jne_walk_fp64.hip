@@ -17,6 +17,7 @@
 
 #include <type_traits>
 
+#include "jne_blocks.h"
 #include "jne_internal.h"
 #include "jne_rng.h"
 #include "jne_tridiag.h"
@@ -39,48 +40,72 @@
 #ifndef JNE_FP64_UNROLL_CALLS
 #define JNE_FP64_UNROLL_CALLS 1
 #endif
-// dims with one lane per walk: the register-only kernel (0: the LDS-staged one)
-#ifndef JNE_FP64_REG
-#define JNE_FP64_REG 1
-#endif
-
 
 namespace jne {
 
 // ---------------------------------------------------------------------------
-// Kernel 1: moments.
+// Kernel 1: moments (jne_blocks.h: block sums, added up with the walk's state).
 //
-// A walk is owned by a group of L lanes.  Every lane keeps the whole
-// state vector b (dim doubles, in a lane-specific rotated order) and
-// accumulates its share of the Gram entries:
-//   rows k < R of  sum e b^T               (R = DP/L, DP = dim padded to L)
-//   rows k < R, cyclic offsets 0..DP/2 of  sum b b^T
-//   rows k < R of  sum u^p b, sum u^p e    (p = 0, 1, 2)
+// A walk is owned by a group of L lanes.  Every lane keeps the block's whole
+// path state c (dim doubles, in a lane-specific rotated order) and
+// accumulates its share of the block's sums:
+//   rows k < R of  sum z c^T               (R = DP/L, DP = dim padded to L)
+//   rows k < R, cyclic offsets 0..DP/2 of  sum c c^T
+//   rows k < R of  S, A1, A2
 // Lane r's row k is component (r*R + k) mod DP, so the L lanes cover every
 // entry; register indices are compile-time constants.
 //
 // The walk advances in rounds of S steps.  The S*dim normals of a round are
-// S*dim/4 Philox calls, dealt round-robin to the group's lanes; each normal
-// is scaled by sqrt(1/T) once and stored to LDS as a double, twice per step
-// row (row = [w_0..w_{dim-1}, 0.., w_0..w_{dim-1}, 0..], 2*DP entries) so that
-// a lane's rotated read of DP entries is one base address plus immediates.
-// The walk index is the fastest LDS dimension (odd pitch) so that the lanes
-// of a wave read from different banks.
+// S*dim/4 Philox calls, dealt round-robin to the group's lanes and stored to
+// LDS as doubles, twice per step row (row = [z_0..z_{dim-1}, 0.., z_0..z_{dim-1},
+// 0..], 2*DP entries) so that a lane's rotated read of DP entries is one base
+// address plus immediates.  The walk index is the fastest LDS dimension (odd
+// pitch) so that the lanes of a wave read from different banks.
+//
+// SPLIT = false: the group takes its walk's blocks in turn and adds each to
+// the sums in acc (its own entries, written by the block before); the last
+// block scales them into the canonical layout.  SPLIT = true: block blockIdx.y
+// alone, its sums to acc[(blockIdx.y * block_moment_count + entry) * ld + walk]
+// for walk_blocks_add.
 // ---------------------------------------------------------------------------
-// FP64 Gram accumulator.
-struct GramAcc {
-  double s;
-  __device__ __forceinline__ void zero() { s = 0.0; }
-  __device__ __forceinline__ void add_prod(double a, double b) { s = fma(a, b, s); }
-  __device__ __forceinline__ void add(double x) { s += x; }
-  __device__ __forceinline__ double value() const { return s; }
-};
+__device__ __forceinline__ void keep_order() { asm volatile("" ::: "memory"); }
 
-template <int D, bool FROM_NORMALS>
+// A lane's sums over the blocks it takes in turn, between blocks: the first
+// NR of its slots in registers, the next NL in LDS, the rest in acc (at x,
+// where their last value goes).  The slots are compile-time constants once
+// the loops are unrolled.
+template <int NR, int NL>
+struct Totals {
+  double reg[NR > 0 ? NR : 1];
+  double (*lds)[64];
+  __device__ __forceinline__ double add(int slot, bool first, bool last, double* x, double t) {
+    if (slot < NR) return reg[slot] = (first ? 0.0 : reg[slot]) + t;
+    if (slot < NR + NL) {
+      double& y = lds[slot - NR][threadIdx.x];
+      return y = (first ? 0.0 : y) + t;
+    }
+    const double v = (first ? 0.0 : *x) + t;
+    if (!last) *x = v;
+    return v;
+  }
+};
+// by dim: the slots that fit beside the block's sums without spills, and the
+// LDS that leaves the kernel's waves resident.  With every slot in acc all the
+// waves of a round write at once, which cost 10% at dim 5 (35 us per block of
+// 131,072 walks); with all 60 slots on chip it does not show.
+#ifndef JNE_FP64_TOTALS
+#define JNE_FP64_TOTALS \
+  {8, 0}, {15, 0}, {5, 17}, {3, 21}, {25, 35}, {0, 34}, {0, 33}, {24, 0}, {8, 10}, {0, 6}, {0, 10}, {12, 10}
+#endif
+struct Fp64Totals {
+  int regs, lds;
+};
+constexpr Fp64Totals kFp64Totals[12] = {JNE_FP64_TOTALS};
+
+template <int D, bool FROM_NORMALS, bool SPLIT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(waves_for_dim(D), waves_for_dim(D))))
 void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
                        uint32_t T, uint32_t n_walks, double* __restrict__ acc, size_t ld) {
-  using Acc = GramAcc;
   using Sh = WalkShape<D>;
   constexpr int L = Sh::L;
   constexpr int DP = Sh::DP;
@@ -92,16 +117,22 @@ void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restr
   constexpr int IT = (C + L - 1) / L;
   constexpr int RW = 2 * DP;        // LDS row width per step
   constexpr int GP = GPW | 1;       // odd walk pitch: a wave's reads spread over the banks
+  static_assert(kBlockUnit % S == 0, "a block must be whole rounds");
   __shared__ double ws[S][RW][GP];
+  __shared__ double bs[DP][GP];  // the state at the block's start
+  constexpr int NR = SPLIT ? 0 : kFp64Totals[D - 1].regs, NL = SPLIT ? 0 : kFp64Totals[D - 1].lds;
+  __shared__ double tot_lds[NL > 0 ? NL : 1][64];
+  Totals<NR, NL> tot;
+  tot.lds = tot_lds;
 
   const int lane = threadIdx.x;
   // walk fastest across the lanes (lane = r * GPW + g): the 16 lanes of a
   // 64-bit LDS access group read the same row of 16 different walks (odd walk
   // pitch: distinct banks), and the output stores of a lane row go to
-  // consecutive walks.  One lane per walk: lane = walk.
-  const int r = L == 1 ? 0 : lane / GPW;
-  const int g = L == 1 ? lane : lane - r * GPW;
-  const bool in_group = L == 1 || r < L;
+  // consecutive walks.
+  const int r = lane / GPW;
+  const int g = lane - r * GPW;
+  const bool in_group = r < L;
   const int gs = in_group ? g : 0;
   const size_t walk = (size_t)blockIdx.x * GPW + gs;
   const bool valid = in_group && walk < n_walks;
@@ -112,161 +143,229 @@ void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restr
   const int rot = r * R;
   const CallPos<D> pos0(r);  // normals of this lane's first Philox call in a round
 
-  if constexpr (DP != D) {  // zero the padding columns once
-    if (in_group)
+  if (in_group) {
+    if constexpr (DP != D) {  // zero the padding columns once
       for (int s = 0; s < S; ++s)
         for (int i = D + r; i < DP; i += L) {
           ws[s][i][gs] = 0.0;
           ws[s][DP + i][gs] = 0.0;
         }
+    }
+    for (int i = r; i < DP; i += L) bs[i][gs] = 0.0;
   }
 
-  double b[DP];
-  Acc geb[R][DP];
-  Acc gbb[R][H + 1];
-  Acc mom[6][R];
+  const uint32_t bn = block_steps(T);
+  uint32_t ts = SPLIT ? blockIdx.y * bn : 0;
+  do {
+    const uint32_t n = T - ts < bn ? T - ts : bn;
+    double c[DP], ge[R][DP], gc[R][H + 1], s0[R], a1[R], a2[R];
 #pragma unroll
-  for (int m = 0; m < DP; ++m) b[m] = 0.0;
+    for (int m = 0; m < DP; ++m) c[m] = 0.0;
 #pragma unroll
-  for (int k = 0; k < R; ++k) {
+    for (int k = 0; k < R; ++k) {
 #pragma unroll
-    for (int m = 0; m < DP; ++m) geb[k][m].zero();
+      for (int m = 0; m < DP; ++m) ge[k][m] = 0.0;
 #pragma unroll
-    for (int m = 0; m <= H; ++m) gbb[k][m].zero();
-#pragma unroll
-    for (int p = 0; p < 6; ++p) mom[p][k].zero();
-  }
+      for (int m = 0; m <= H; ++m) gc[k][m] = 0.0;
+      s0[k] = a1[k] = a2[k] = 0.0;
+    }
 
-  // src/johansen_statistics.rs:70 and src/rng_matrix.rs:137: sqrt(1/steps)
-  const double dt = 1.0 / (double)T;
-  const double sqrt_dt = sqrt(dt);
-
-  for (uint32_t t0 = 0; t0 < T; t0 += S) {
-    // produce: this round's increments
-    if (in_group) {
-      const uint32_t q0 = (uint32_t)((uint64_t)t0 * D / 4);  // < 2^32: dim <= kMaxDim, steps <= kMaxSteps
-      CallPos<D> pos = pos0;
+    for (uint32_t t0 = ts; t0 < ts + n; t0 += S) {
+      // produce: this round's increments
+      if (in_group) {
+        const uint32_t q0 = (uint32_t)((uint64_t)t0 * D / 4);  // < 2^32: dim <= kMaxDim, steps <= kMaxSteps
+        CallPos<D> pos = pos0;
 #if JNE_FP64_UNROLL_CALLS
 #pragma unroll
 #else
 #pragma unroll 1
 #endif
-      for (int it = 0; it < IT; ++it) {
-        const int c = it * L + r;
-        if (IT * L == C || c < C) {
-          int sj[4], ij[4];
+        for (int it = 0; it < IT; ++it) {
+          const int call = it * L + r;
+          if (IT * L == C || call < C) {
+            int sj[4], ij[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) pos.at(j, sj[j], ij[j]);
-          double wv[4];
-          if constexpr (!FROM_NORMALS) {
-            float v[4];
-            normals4(q0 + c, seed, rng_stream, v);
+            for (int j = 0; j < 4; ++j) pos.at(j, sj[j], ij[j]);
+            double wv[4];
+            if constexpr (!FROM_NORMALS) {
+              float v[4];
+              normals4(q0 + call, seed, rng_stream, v);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = (double)v[j] * sqrt_dt;
-          } else {
+              for (int j = 0; j < 4; ++j) wv[j] = (double)v[j];
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const uint32_t t = t0 + sj[j];
+                wv[j] = t < T ? zw[(size_t)t * D + ij[j]] : 0.0;
+              }
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              const uint32_t t = t0 + sj[j];
-              wv[j] = t < T ? zw[(size_t)t * D + ij[j]] * sqrt_dt : 0.0;
+              ws[sj[j]][ij[j]][gs] = wv[j];
+              ws[sj[j]][DP + ij[j]][gs] = wv[j];
             }
           }
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            ws[sj[j]][ij[j]][gs] = wv[j];
-            ws[sj[j]][DP + ij[j]][gs] = wv[j];
-          }
+          pos.template advance<L>();
         }
-        pos.template advance<L>();
       }
-    }
-    __syncthreads();
-    // consume: advance the walk S steps
-    const int ns = (T - t0) < (uint32_t)S ? (int)(T - t0) : S;
+      __syncthreads();
+      // consume: advance the block's path S steps
+      const int ns = (ts + n - t0) < (uint32_t)S ? (int)(ts + n - t0) : S;
 #if JNE_FP64_UNROLL_STEPS
 #pragma unroll
 #else
 #pragma unroll 1
 #endif
-    for (int s = 0; s < S; ++s) {
-      if (s >= ns) break;
-      const double* w = &ws[s][rot][gs];
-      const uint32_t t = t0 + s;
-      const double u = (double)(t + 1) * dt;
-      const double u2 = u * u;
-      // only the lane's own rows need B_{t+1} before the Gram update; the
-      // other components are advanced in place afterwards
-      double bnk[R], e[R];
+      for (int s = 0; s < S; ++s) {
+        if (s >= ns) break;
+        const double* w = &ws[s][rot][gs];
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
-        bnk[k] = b[k] + w[k * GP];  // B_{t+1} = B_t + z*sqrt(dt) (rng_matrix.rs:138-140)
-        e[k] = bnk[k] - b[k];  // dbm = bm_current - bm_previous (johansen_statistics.rs:80-82)
+        for (int k = 0; k < R; ++k) {
+          const double wk = w[k * GP];
+#pragma unroll
+          for (int m = 0; m < DP; ++m) ge[k][m] = fma(wk, c[m], ge[k][m]);
+#pragma unroll
+          for (int dl = 0; dl <= H; ++dl) gc[k][dl] = fma(c[k], c[(k + dl) % DP], gc[k][dl]);
+          a2[k] += a1[k];
+          a1[k] += s0[k];
+          s0[k] += c[k];
+        }
+#pragma unroll
+        for (int m = 0; m < DP; ++m) c[m] += w[m * GP];
       }
-#pragma unroll
-      for (int k = 0; k < R; ++k) {
-#pragma unroll
-        for (int m = 0; m < DP; ++m) geb[k][m].add_prod(e[k], b[m]);
-#pragma unroll
-        for (int dl = 0; dl <= H; ++dl) gbb[k][dl].add_prod(b[k], b[(k + dl) % DP]);
-        mom[0][k].add(b[k]);
-        mom[1][k].add_prod(u, b[k]);
-        mom[2][k].add_prod(u2, b[k]);
-        mom[3][k].add(e[k]);
-        mom[4][k].add_prod(u, e[k]);
-        mom[5][k].add_prod(u2, e[k]);
-      }
-#pragma unroll
-      for (int k = 0; k < R; ++k) b[k] = bnk[k];
-#pragma unroll
-      for (int m = R; m < DP; ++m) b[m] = b[m] + w[m * GP];
+      __syncthreads();
     }
-    __syncthreads();
-  }
 
-  if (!valid) return;
-  // canonical layout, entry-major: [0, D^2) sum b b^T (full), [D^2, 2D^2)
-  // sum e b^T (row e, col b), then 6 moment vectors of length D.
+    if constexpr (SPLIT) {
+      if (!valid) return;
+      double* const o = acc + (size_t)blockIdx.y * block_moment_count(D) * ld + walk;
 #pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const int ci = (rot + k) % DP;
-    if (ci >= D) continue;
+      for (int k = 0; k < R; ++k) {
+        const int ci = (rot + k) % DP;
+        if (ci >= D) continue;
 #pragma unroll
-    for (int m = 0; m < DP; ++m) {
-      const int cj = (rot + m) % DP;
-      if (cj < D) acc[(size_t)(D * D + ci * D + cj) * ld + walk] = geb[k][m].value();
-    }
+        for (int m = 0; m < DP; ++m) {
+          const int cj = (rot + m) % DP;
+          if (cj < D) o[(size_t)blk_ge(D, ci, cj) * ld] = ge[k][m];
+        }
 #pragma unroll
-    for (int dl = 0; dl <= H; ++dl) {
-      const int cj = (rot + k + dl) % DP;
-      if (cj < D) {
-        acc[(size_t)(ci * D + cj) * ld + walk] = gbb[k][dl].value();
-        acc[(size_t)(cj * D + ci) * ld + walk] = gbb[k][dl].value();
+        for (int dl = 0; dl <= H; ++dl) {
+          const int cj = (rot + k + dl) % DP;
+          if (cj < D) o[(size_t)(ci < cj ? blk_gc(D, ci, cj) : blk_gc(D, cj, ci)) * ld] = gc[k][dl];
+        }
+        o[(size_t)blk_vec(D, 0, ci) * ld] = s0[k];
+        o[(size_t)blk_vec(D, 1, ci) * ld] = a1[k];
+        o[(size_t)blk_vec(D, 2, ci) * ld] = a2[k];
+        o[(size_t)blk_vec(D, 3, ci) * ld] = c[k];
       }
-    }
+      return;
+    } else {
+      // add the block to the walk's sums: the S of the other lanes' rows go
+      // through the round's LDS (its last reads came before the barrier above)
+      double(*const ss)[GP] = ws[0];
+      if (in_group) {
 #pragma unroll
-    for (int p = 0; p < 6; ++p) acc[(size_t)(2 * D * D + p * D + ci) * ld + walk] = mom[p][k].value();
-  }
+        for (int k = 0; k < R; ++k) ss[(rot + k) % DP][gs] = s0[k];
+      }
+      __syncthreads();
+      const bool first = ts == 0, last = ts + n >= T;
+      if (valid) {
+        const BlockConst bc = block_const(ts, n);
+        const MomentScale sc = moment_scale(T);
+        // opaque copies: the entries' addresses are formed here, not kept in
+        // registers across the block (keep_order bounds the loads in flight)
+        double* o = acc + walk;
+        size_t ld_ = ld;
+        int rot_ = rot;
+        asm volatile("" : "+v"(o), "+s"(ld_), "+v"(rot_));
+        int slot = 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          const int ci = (rot_ + k) % DP;
+          const bool has_i = DP == D || ci < D;
+          const double bi = bs[ci][gs];
+#pragma unroll
+          for (int m = 0; m < DP; ++m, ++slot) {
+            const int cj = (rot_ + m) % DP;
+            if (m % 4 == 0) keep_order();
+            if (!has_i || (DP != D && cj >= D)) continue;
+            double* const x = o + (size_t)(D * D + ci * D + cj) * ld_;
+            const double v = tot.add(slot, first, last, x, block_zb(c[k], bs[cj][gs], ge[k][m]));
+            if (last) *x = v * sc.dt;
+          }
+#pragma unroll
+          for (int dl = 0; dl <= H; ++dl, ++slot) {
+            const int cj = (rot_ + k + dl) % DP;
+            if (dl % 4 == 0) keep_order();
+            if (!has_i || (DP != D && cj >= D)) continue;
+            // at an even DP both owners of a pair at distance DP/2 hold it: the
+            // lower component's adds it
+            if (DP % 2 == 0 && dl == H && cj < ci) continue;
+            const bool up = ci < cj;
+            const double bj = bs[cj][gs], sj = ss[cj][gs];
+            double* const x = o + (size_t)(up ? ci * D + cj : cj * D + ci) * ld_;
+            const double v = tot.add(slot, first, last, x,
+                                     block_bb(bc, up ? bi : bj, up ? bj : bi, up ? s0[k] : sj, up ? sj : s0[k], gc[k][dl]));
+            if (last) {
+              *x = v * sc.dt;
+              o[(size_t)(up ? cj * D + ci : ci * D + cj) * ld_] = v * sc.dt;
+            }
+          }
+          if (has_i) {
+            double* const x = o + (size_t)(2 * D * D + ci) * ld_;
+            const double m0 = tot.add(slot, first, last, x, block_m0(bc, bi, s0[k]));
+            const double m1 = tot.add(slot + 1, first, last, x + (size_t)D * ld_, block_m1(bc, bi, s0[k], a1[k]));
+            const double m2 =
+                tot.add(slot + 2, first, last, x + (size_t)(2 * D) * ld_, block_m2(bc, bi, s0[k], a1[k], a2[k]));
+            if (last) store_vector_moments(sc, m0, m1, m2, bi + c[k], o, D, ci, ld_, 0);
+          }
+          slot += 3;
+        }
+      }
+      __syncthreads();
+      if (in_group) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) bs[(rot + k) % DP][gs] += c[k];
+      }
+      if constexpr (DP != D) {  // the padding columns that held S
+        if (in_group)
+          for (int i = D + r; i < DP; i += L) ss[i][gs] = 0.0;
+      }
+      __syncthreads();
+      ts += n;
+    }
+  } while (!SPLIT && ts < T);
 }
 
 // ---------------------------------------------------------------------------
-// Kernel 1, one lane per walk (the dims whose shape has L = 1): the same moments and the same
-// arithmetic, step by step, as walk_moments_fp64 with L = 1, with the
-// increments kept in registers instead of LDS.  A lane draws its walk's
-// Philox calls in batches of NB calls (kFp64RegCalls: three independent
-// calls in flight at dims 1-4 and 6, the five of a whole-step group at dim 5)
-// and consumes the batch's G = 4 NB / dim steps from registers: no LDS, no
-// barriers.
+// Kernel 1, one lane per walk (the dims whose shape has L = 1): the same sums
+// as walk_moments_fp64 with L = 1, with the increments kept in registers
+// instead of LDS.  A lane draws its walk's Philox calls in batches of NB calls
+// (kFp64RegCalls: three independent calls in flight at dims 1-4 and 6, the
+// five of a whole-step group at dim 5, seven at dim 7) and consumes the batch's
+// G = 4 NB / dim steps from registers: no LDS, no barriers inside a block.
+//
+// Bound by VALU issue: at dim 5 a wave-step issues 235 instructions in 722
+// cycles, 65 of them FP64 at 3.9 and 1.25 Philox calls of 357 cycles.  The
+// increments' moments, the powers of u and the scaling of each normal left the
+// step with the block sums.  262,144 walks at T = 10^4, before (every term
+// per step) and after: dim 1 2.86 and 2.12 ms, dim 3 8.94 and 7.4, dim 5 16.2
+// and 14.4, dim 6 20.1 and 17.4; dim 7 34.6 ms with seven lanes per walk
+// through LDS, 28.4 with the block sums there, 22 here.
 // ---------------------------------------------------------------------------
 // target waves per SIMD of the register-only kernel by dim (the register cap:
-// 512 / waves VGPRs per lane); it runs the dims whose shape has one lane per walk
+// 512 / waves VGPRs per lane); it runs the dims whose shape has one lane per walk.
+// One wave per SIMD reaches 88% of two waves' rate; 4 waves at dim 3 and 3 at
+// dim 4 are 3 and 4% faster than 3 and 2.
 #ifndef JNE_FP64_REG_WAVES
-#define JNE_FP64_REG_WAVES 4, 4, 3, 2, 2, 2, 2, 2, 2, 2, 2, 2
+#define JNE_FP64_REG_WAVES 4, 4, 4, 3, 2, 2, 2, 2, 2, 2, 2, 2
 #endif
 constexpr int kFp64RegWaves[12] = {JNE_FP64_REG_WAVES};
 
 // Philox calls per batch by dim (a multiple of the calls of one whole-step
 // group: 1, 1, 3, 1, 5, 3 at dims 1..6)
 #ifndef JNE_FP64_REG_CALLS
-#define JNE_FP64_REG_CALLS 3, 3, 3, 3, 5, 3, 3, 3, 3, 3, 3, 3
+#define JNE_FP64_REG_CALLS 3, 3, 3, 3, 5, 3, 7, 6, 9, 5, 11, 3
 #endif
 constexpr int kFp64RegCalls[12] = {JNE_FP64_REG_CALLS};
 
@@ -276,15 +375,17 @@ struct RegBatch {
   static constexpr int NB = kFp64RegCalls[D - 1];         // calls per batch
   static constexpr int G = 4 * NB / D;                     // steps per batch
   static_assert(NB % NC == 0, "a batch must be whole steps");
+  static_assert(kBlockUnit % G == 0, "a block must be whole batches");
 };
 
-template <int D, bool FROM_NORMALS>
+template <int D, bool FROM_NORMALS, bool SPLIT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFp64RegWaves[D - 1], kFp64RegWaves[D - 1])))
 void walk_moments_fp64_reg(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
                            uint32_t T, uint32_t n_walks, double* __restrict__ acc, size_t ld) {
-  using Acc = GramAcc;
-  constexpr int H = D / 2;
-  constexpr int NB = RegBatch<D>::NB, G = RegBatch<D>::G;
+  constexpr int G = RegBatch<D>::G;
+  // dim 7: a step's calls are drawn just before it (a whole batch's normals
+  // beside the 105 sums would spill)
+  constexpr bool kLazy = D >= 7 && !FROM_NORMALS;
   const size_t walk = (size_t)blockIdx.x * 64 + threadIdx.x;
   const bool valid = walk < n_walks;
   const size_t wc = valid ? walk : (size_t)(n_walks - 1);
@@ -292,100 +393,289 @@ void walk_moments_fp64_reg(const uint32_t* __restrict__ seeds, const double* __r
   if constexpr (!FROM_NORMALS) seed = seeds[wc];
   const double* zw = FROM_NORMALS ? zin + wc * (size_t)T * D : nullptr;
 
-  double b[D];
-  Acc geb[D][D];
-  Acc gbb[D][H + 1];
-  Acc mom[6][D];
+  const uint32_t bn = block_steps(T);
+  uint32_t ts = SPLIT ? blockIdx.y * bn : 0;
+  constexpr int NR = SPLIT ? 0 : kFp64Totals[D - 1].regs, NL = SPLIT ? 0 : kFp64Totals[D - 1].lds;
+  __shared__ double tot_lds[NL > 0 ? NL : 1][64];
+  Totals<NR, NL> tot;
+  tot.lds = tot_lds;
+  // the state at the block's start: needed between blocks only
+  __shared__ double bs_lds[SPLIT ? 1 : D][64];
+  auto bs = [&](int m) -> double& { return bs_lds[m][threadIdx.x]; };
+  if constexpr (!SPLIT) {
 #pragma unroll
-  for (int m = 0; m < D; ++m) b[m] = 0.0;
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-#pragma unroll
-    for (int m = 0; m < D; ++m) geb[k][m].zero();
-#pragma unroll
-    for (int m = 0; m <= H; ++m) gbb[k][m].zero();
-#pragma unroll
-    for (int p = 0; p < 6; ++p) mom[p][k].zero();
+    for (int m = 0; m < D; ++m) bs(m) = 0.0;
   }
-
-  // src/johansen_statistics.rs:70 and src/rng_matrix.rs:137: sqrt(1/steps)
-  const double dt = 1.0 / (double)T;
-  const double sqrt_dt = sqrt(dt);
-
-  // one step of the walk from its scaled increments w[0..D) (the moment
-  // updates of walk_moments_fp64 with one lane per walk)
-  auto step = [&](const double* w, uint32_t t) {
-    const double u = (double)(t + 1) * dt;
-    const double u2 = u * u;
-    double bn[D], e[D];
+  do {
+    const uint32_t n = T - ts < bn ? T - ts : bn;
+    double c[D], ge[D][D], gc[D * (D + 1) / 2], s0[D], a1[D], a2[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-      bn[k] = b[k] + w[k];  // B_{t+1} = B_t + z*sqrt(dt) (rng_matrix.rs:138-140)
-      e[k] = bn[k] - b[k];  // dbm = bm_current - bm_previous (johansen_statistics.rs:80-82)
+      c[k] = s0[k] = a1[k] = a2[k] = 0.0;
+#pragma unroll
+      for (int m = 0; m < D; ++m) ge[k][m] = 0.0;
     }
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-#pragma unroll
-      for (int m = 0; m < D; ++m) geb[k][m].add_prod(e[k], b[m]);
-#pragma unroll
-      for (int dl = 0; dl <= H; ++dl) gbb[k][dl].add_prod(b[k], b[(k + dl) % D]);
-      mom[0][k].add(b[k]);
-      mom[1][k].add_prod(u, b[k]);
-      mom[2][k].add_prod(u2, b[k]);
-      mom[3][k].add(e[k]);
-      mom[4][k].add_prod(u, e[k]);
-      mom[5][k].add_prod(u2, e[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < D; ++k) b[k] = bn[k];
-  };
+    for (int e = 0; e < D * (D + 1) / 2; ++e) gc[e] = 0.0;
 
-  // a batch: G steps from t0; tail batches mask the steps at or beyond T
-  auto batch = [&](uint32_t t0, auto tail_tag) {
-    constexpr bool tail = decltype(tail_tag)::value;
-    double w[G * D];
-    if constexpr (!FROM_NORMALS) {
+    // one step of the block's path from its increments w[0..D)
+    auto step = [&](const double* w) {
+      int e = 0;
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+#pragma unroll
+        for (int m = 0; m < D; ++m) ge[k][m] = fma(w[k], c[m], ge[k][m]);
+#pragma unroll
+        for (int m = k; m < D; ++m, ++e) gc[e] = fma(c[k], c[m], gc[e]);
+        a2[k] += a1[k];
+        a1[k] += s0[k];
+        s0[k] += c[k];
+      }
+#pragma unroll
+      for (int k = 0; k < D; ++k) c[k] += w[k];
+    };
+    // a batch: G steps from t0; the tail batch masks the steps past the block
+    auto batch = [&](uint32_t t0, auto tail_tag) {
+      constexpr bool tail = decltype(tail_tag)::value;
+      double w[G * D];
       const uint32_t q0 = (uint32_t)((uint64_t)t0 * D / 4);  // < 2^32: dim <= kMaxDim, steps <= kMaxSteps
+      // the calls that steps s < s1 still need, of the first `have`
+      auto draw = [&](int have, int s1) {
 #pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        float v[4];
-        normals4(q0 + c, seed, rng_stream, v);
+        for (int q = have; q < (s1 * D + 3) / 4; ++q) {
+          float v[4];
+          normals4(q0 + q, seed, rng_stream, v);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[4 * c + j] = (double)v[j] * sqrt_dt;
+          for (int j = 0; j < 4; ++j) w[4 * q + j] = (double)v[j];
+        }
+      };
+      if constexpr (FROM_NORMALS) {
+#pragma unroll
+        for (int e = 0; e < G * D; ++e) {
+          const uint32_t t = t0 + (uint32_t)(e / D);
+          w[e] = (!tail || t < T) ? zw[(size_t)t0 * D + e] : 0.0;
+        }
+      } else if constexpr (!kLazy) {
+        draw(0, G);
       }
-    } else {
 #pragma unroll
-      for (int n = 0; n < G * D; ++n) {
-        const uint32_t t = t0 + (uint32_t)(n / D);
-        w[n] = (!tail || t < T) ? zw[(size_t)t0 * D + n] * sqrt_dt : 0.0;
+      for (int s = 0; s < G; ++s) {
+        if constexpr (kLazy) {
+          draw((s * D + 3) / 4, s + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (tail && t0 + s >= T) break;
+        step(&w[s * D]);
       }
-    }
-#pragma unroll
-    for (int s = 0; s < G; ++s) {
-      if (tail && t0 + s >= T) break;
-      step(&w[s * D], t0 + s);
-    }
-  };
-  const uint32_t full = T / G;
-  for (uint32_t q = 0; q < full; ++q) batch(q * G, BoolTag<false>{});
-  if (full * G < T) batch(full * G, BoolTag<true>{});
+    };
+    const uint32_t full = n / G;
+    for (uint32_t q = 0; q < full; ++q) batch(ts + q * G, BoolTag<false>{});
+    if (full * G < n) batch(ts + full * G, BoolTag<true>{});  // the walk's last block only
 
-  if (!valid) return;
-  // canonical layout, entry-major: [0, D^2) sum b b^T (full), [D^2, 2D^2)
-  // sum e b^T (row e, col b), then 6 moment vectors of length D.
+    if constexpr (SPLIT) {
+      if (!valid) return;
+      double* const o = acc + (size_t)blockIdx.y * block_moment_count(D) * ld + walk;
 #pragma unroll
-  for (int k = 0; k < D; ++k) {
+      for (int k = 0; k < D; ++k) {
 #pragma unroll
-    for (int m = 0; m < D; ++m) acc[(size_t)(D * D + k * D + m) * ld + walk] = geb[k][m].value();
+        for (int m = 0; m < D; ++m) o[(size_t)blk_ge(D, k, m) * ld] = ge[k][m];
+        o[(size_t)blk_vec(D, 0, k) * ld] = s0[k];
+        o[(size_t)blk_vec(D, 1, k) * ld] = a1[k];
+        o[(size_t)blk_vec(D, 2, k) * ld] = a2[k];
+        o[(size_t)blk_vec(D, 3, k) * ld] = c[k];
+      }
 #pragma unroll
-    for (int dl = 0; dl <= H; ++dl) {
-      const int cj = (k + dl) % D;
-      acc[(size_t)(k * D + cj) * ld + walk] = gbb[k][dl].value();
-      acc[(size_t)(cj * D + k) * ld + walk] = gbb[k][dl].value();
+      for (int e = 0; e < D * (D + 1) / 2; ++e) o[(size_t)(D * D + e) * ld] = gc[e];
+      return;
+    } else {
+      const bool first = ts == 0, last = ts + n >= T;
+      if (valid) {
+        const BlockConst bc = block_const(ts, n);
+        const MomentScale sc = moment_scale(T);
+        double* o = acc + walk;  // opaque copies, as in walk_moments_fp64
+        size_t ld_ = ld;
+        asm volatile("" : "+v"(o), "+s"(ld_));
+        int e = 0, slot = 0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          keep_order();
+#pragma unroll
+          for (int m = 0; m < D; ++m, ++slot) {
+            if (D >= 7 && m % 2 == 0) keep_order();
+            double* const x = o + (size_t)(D * D + k * D + m) * ld_;
+            const double v = tot.add(slot, first, last, x, block_zb(c[k], bs(m), ge[k][m]));
+            if (last) *x = v * sc.dt;
+          }
+          keep_order();
+#pragma unroll
+          for (int m = k; m < D; ++m, ++e, ++slot) {
+            if (D >= 7 && m % 2 == 0) keep_order();
+            double* const x = o + (size_t)(k * D + m) * ld_;
+            const double v = tot.add(slot, first, last, x, block_bb(bc, bs(k), bs(m), s0[k], s0[m], gc[e]));
+            if (last) {
+              *x = v * sc.dt;
+              o[(size_t)(m * D + k) * ld_] = v * sc.dt;
+            }
+          }
+          double* const x = o + (size_t)(2 * D * D + k) * ld_;
+          const double m0 = tot.add(slot, first, last, x, block_m0(bc, bs(k), s0[k]));
+          const double m1 = tot.add(slot + 1, first, last, x + (size_t)D * ld_, block_m1(bc, bs(k), s0[k], a1[k]));
+          const double m2 =
+              tot.add(slot + 2, first, last, x + (size_t)(2 * D) * ld_, block_m2(bc, bs(k), s0[k], a1[k], a2[k]));
+          slot += 3;
+          if (last) store_vector_moments(sc, m0, m1, m2, bs(k) + c[k], o, D, k, ld_, 0);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < D; ++k) bs(k) += c[k];
+      ts += n;
     }
+  } while (!SPLIT && ts < T);
+}
+
+// ---------------------------------------------------------------------------
+// Kernel 1, one wave per block of a walk (blockIdx.x: the walk, blockIdx.y:
+// the block): the batches of a few walks, where latency counts.  Rounds of
+// kWaveRound steps: the wave draws the round's normals, lanes 0..dim-1 run
+// their component's path and S, A1, A2, and every lane adds its entries of
+// sum z c^T and of the upper triangle of sum c c^T over the round's steps.
+// Each sum takes its terms in the order of the other forms (the same bits).
+// ---------------------------------------------------------------------------
+constexpr int kWaveRound = 64;
+
+template <int D, bool FROM_NORMALS>
+__global__ __launch_bounds__(64) void walk_moments_fp64_wave(const uint32_t* __restrict__ seeds,
+                                                             const double* __restrict__ zin, uint32_t rng_stream,
+                                                             uint32_t T, double* __restrict__ part, size_t ld) {
+  constexpr int R = kWaveRound, NE = D * D + D * (D + 1) / 2, NQ = (NE + 63) / 64;
+  constexpr int C = R * D / 4;  // Philox calls per round
+  __shared__ __align__(16) double zs[R * D], cs[R * D];  // t-major
+  const int l = threadIdx.x;
+  const size_t walk = blockIdx.x;
+  uint32_t seed = 0;
+  if constexpr (!FROM_NORMALS) seed = seeds[walk];
+  const double* zw = FROM_NORMALS ? zin + walk * (size_t)T * D : nullptr;
+  const uint32_t bn = block_steps(T), ts = blockIdx.y * bn, n = T - ts < bn ? T - ts : bn;
+  // entry e = l + 64 q: the product of the components x[q], y[q] of z or c and c
+  const double* px[NQ];
+  const double* py[NQ];
+  double acc[NQ];
 #pragma unroll
-    for (int p = 0; p < 6; ++p) acc[(size_t)(2 * D * D + p * D + k) * ld + walk] = mom[p][k].value();
+  for (int q = 0; q < NQ; ++q) {
+    int e = l + 64 * q;
+    if (e >= NE) e = 0;
+    int i = e / D, j = e - (e / D) * D;
+    px[q] = zs + i;
+    if (e >= D * D) {
+      e -= D * D;
+      for (i = 0; e >= D - i; ++i) e -= D - i;
+      j = i + e;
+      px[q] = cs + i;
+    }
+    py[q] = cs + j;
+    acc[q] = 0.0;
   }
+  double c = 0.0, s0 = 0.0, a1 = 0.0, a2 = 0.0;
+  for (uint32_t t0 = 0; t0 < n; t0 += R) {
+    const int ns = n - t0 < (uint32_t)R ? (int)(n - t0) : R;
+    if constexpr (FROM_NORMALS) {
+      for (int e = l; e < ns * D; e += 64) zs[e] = zw[(size_t)(ts + t0) * D + e];
+    } else {
+      const uint32_t q0 = (uint32_t)((uint64_t)(ts + t0) * D / 4);
+      for (int q = l; q < C && 4 * q < ns * D; q += 64) {
+        float v[4];
+        normals4(q0 + q, seed, rng_stream, v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) zs[4 * q + j] = (double)v[j];
+      }
+    }
+    __syncthreads();
+    if (l < D) {
+#pragma unroll 8
+      for (int t = 0; t < ns; ++t) {
+        cs[t * D + l] = c;
+        a2 += a1;
+        a1 += s0;
+        s0 += c;
+        c += zs[t * D + l];
+      }
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int t = 0; t < ns; ++t) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[q] = fma(px[q][t * D], py[q][t * D], acc[q]);
+    }
+    __syncthreads();
+  }
+  double* const o = part + (size_t)blockIdx.y * block_moment_count(D) * ld + walk;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+    if (l + 64 * q < NE) o[(size_t)(l + 64 * q) * ld] = acc[q];
+  if (l < D) {
+    o[(size_t)blk_vec(D, 0, l) * ld] = s0;
+    o[(size_t)blk_vec(D, 1, l) * ld] = a1;
+    o[(size_t)blk_vec(D, 2, l) * ld] = a2;
+    o[(size_t)blk_vec(D, 3, l) * ld] = c;
+  }
+}
+
+// The walks' moments from their blocks' sums (part: n_walks per entry): a
+// workgroup takes 64 walks, its wave k row k of sum z c^T, the upper
+// triangle's row k of sum c c^T and component k's vector sums, adding the
+// blocks in order with the operations of the kernels that take them in turn.
+// Bound by its reads; the waves share the S and E they all read through L1.
+// Above dim 6 blockIdx.y halves the columns (no spills).
+template <int D>
+struct AddShape {
+  static constexpr int NH = D > 6 ? 2 : 1, JW = (D + NH - 1) / NH;
+};
+template <int D>
+__global__ __launch_bounds__(64 * D) void walk_blocks_add(uint32_t T, uint32_t n_walks, const double* __restrict__ part,
+                                                          double* __restrict__ acc, size_t ld) {
+  constexpr int JW = AddShape<D>::JW;
+  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j0 = blockIdx.y * JW;
+  const size_t walk = (size_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  if (walk >= n_walks) return;
+  const uint32_t bn = block_steps(T);
+  const MomentScale sc = moment_scale(T);
+  const double* p = part + walk;
+  double b[JW], ge[JW], gc[JW], m0 = 0.0, m1 = 0.0, m2 = 0.0, bk = 0.0;
+#pragma unroll
+  for (int q = 0; q < JW; ++q) b[q] = ge[q] = gc[q] = 0.0;
+  for (uint32_t ts = 0; ts < T; ts += bn, p += (size_t)block_moment_count(D) * n_walks) {
+    auto at = [&](int e) { return p[(size_t)e * n_walks]; };
+    const BlockConst bc = block_const(ts, T - ts < bn ? T - ts : bn);
+    const double sk = at(blk_vec(D, 0, k)), ek = at(blk_vec(D, 3, k));
+#pragma unroll
+    for (int q = 0; q < JW; ++q) {
+      const int j = j0 + q;
+      if (j >= D) break;
+      const double bj = b[q];
+      ge[q] += block_zb(ek, bj, at(blk_ge(D, k, j)));
+      if (j >= k) gc[q] += block_bb(bc, bk, bj, sk, at(blk_vec(D, 0, j)), at(blk_gc(D, k, j)));
+      b[q] = bj + at(blk_vec(D, 3, j));
+    }
+    if (j0 == 0) {
+      const double a1 = at(blk_vec(D, 1, k)), a2 = at(blk_vec(D, 2, k));
+      m0 += block_m0(bc, bk, sk);
+      m1 += block_m1(bc, bk, sk, a1);
+      m2 += block_m2(bc, bk, sk, a1, a2);
+    }
+    bk += ek;
+  }
+  double* const o = acc + walk;
+#pragma unroll
+  for (int q = 0; q < JW; ++q) {
+    const int j = j0 + q;
+    if (j >= D) break;
+    o[(size_t)(D * D + k * D + j) * ld] = ge[q] * sc.dt;
+    if (j >= k) {
+      o[(size_t)(k * D + j) * ld] = gc[q] * sc.dt;
+      o[(size_t)(j * D + k) * ld] = gc[q] * sc.dt;
+    }
+  }
+  if (j0 == 0) store_vector_moments(sc, m0, m1, m2, bk, o, D, k, ld, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -727,28 +1017,80 @@ __global__ __launch_bounds__(64) void walk_eigen_jacobi(const double* __restrict
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// The forms of a moment launch.  One lane group per walk fills the GPU (`slots`
+// waves resident at the kernel's occupancy) in whole rounds only; the walks of
+// the last, partial round are split over their blocks where a walk has
+// several.  Walks whose blocks (in units of kBlockUnit steps) number at most
+// kWaveForm get one wave per block, more get one lane group per block: the
+// line lies where the two take the same time, between T = 300 and 2,000 (ms,
+// group / wave form: dim 1, 2,000 units 0.024 / 0.019, 8,000 0.024 / 0.036;
+// dim 5, 9,000 0.140 / 0.114, 18,000 0.124 / 0.176; dim 12, 2,000 0.115 /
+// 0.061, 4,500 0.150 / 0.179).  A split walk also writes and reads its blocks'
+// sums (4 to 30% of the whole, more at the high dims and short blocks), so a
+// rest of ROUND_FILL of a round or more is not split.  100,000 walks at
+// T = 2,000, in turn and split: dim 1 0.232 and 0.171 ms, dim 5 1.52 and 1.22;
+// 10,000 walks at T = 8,000: dim 1 0.607 and 0.112, dim 5 3.62 and 0.59,
+// dim 12 3.60 and 1.85.
+constexpr uint32_t kSimds = 1024;
+#ifndef JNE_WAVE_FORM
+#define JNE_WAVE_FORM 3500, 5000, 7000, 10000, 13000, 15000, 11000, 8000, 3000, 3000, 4000, 3200
+#endif
+constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
+#ifndef JNE_ROUND_FILL
+#define JNE_ROUND_FILL 90  // percent of a round
+#endif
+
+// Walks of n whose blocks one lane group takes in turn (the rest are split).
+static uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
+  const uint32_t L = lanes_for_dim(d);
+  const uint32_t round = (64 / L) * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
+  const uint32_t rest = n % round;
+  if (block_count(T) == 1) return n > kWaveForm[d - 1] ? n : 0;
+  return (uint64_t)rest * 100 >= (uint64_t)round * JNE_ROUND_FILL ? n : n - rest;
+}
+
+size_t fp64_part_doubles(int d, uint32_t T, uint32_t n) {
+  return (size_t)block_count(T) * block_moment_count(d) * (n - fp64_turns(d, T, n));
+}
+
 template <int D>
 static hipError_t launch_moments_d(const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                   uint32_t n, double* acc, size_t ld, hipStream_t st) {
-  constexpr int GPW = WalkShape<D>::GPW;
-  const unsigned grid = (unsigned)((n + GPW - 1) / GPW);
-#if JNE_FP64_REG
-  if constexpr (WalkShape<D>::L == 1) {
-    if (zin != nullptr)
-      hipLaunchKernelGGL((walk_moments_fp64_reg<D, true>), dim3(grid), dim3(64), 0, st, seeds, zin, rng_stream, T, n,
-                         acc, ld);
+                                   uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                   hipStream_t st) {
+  constexpr bool kReg = WalkShape<D>::L == 1;
+  constexpr uint32_t GPW = WalkShape<D>::GPW;
+  auto go = [&](auto fn_tag, auto split_tag, const uint32_t* s, const double* z, uint32_t m, double* out, size_t ldo) {
+    constexpr bool FN = decltype(fn_tag)::value, SPLIT = decltype(split_tag)::value;
+    const dim3 grid((m + GPW - 1) / GPW, SPLIT ? block_count(T) : 1);
+    if constexpr (kReg)
+      hipLaunchKernelGGL((walk_moments_fp64_reg<D, FN, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out, ldo);
     else
-      hipLaunchKernelGGL((walk_moments_fp64_reg<D, false>), dim3(grid), dim3(64), 0, st, seeds, zin, rng_stream, T, n,
-                         acc, ld);
+      hipLaunchKernelGGL((walk_moments_fp64<D, FN, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out, ldo);
     return hipGetLastError();
+  };
+  uint32_t turns = fp64_turns(D, T, n);
+  if (part == nullptr || part_doubles < fp64_part_doubles(D, T, n)) turns = n;
+  hipError_t e = hipSuccess;
+  if (turns > 0)
+    e = zin ? go(BoolTag<true>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld)
+            : go(BoolTag<false>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld);
+  if (e != hipSuccess || turns == n) return e;
+  // the split rest
+  const uint32_t m = n - turns;
+  const uint32_t* s = seeds ? seeds + turns : nullptr;
+  const double* z = zin ? zin + (size_t)turns * T * D : nullptr;
+  if ((uint64_t)m * ((T + kBlockUnit - 1) / kBlockUnit) <= kWaveForm[D - 1]) {
+    const dim3 grid(m, block_count(T));
+    if (z)
+      hipLaunchKernelGGL((walk_moments_fp64_wave<D, true>), grid, dim3(64), 0, st, s, z, rng_stream, T, part, (size_t)m);
+    else
+      hipLaunchKernelGGL((walk_moments_fp64_wave<D, false>), grid, dim3(64), 0, st, s, z, rng_stream, T, part, (size_t)m);
+    e = hipGetLastError();
+  } else {
+    e = z ? go(BoolTag<true>{}, BoolTag<true>{}, s, z, m, part, m) : go(BoolTag<false>{}, BoolTag<true>{}, s, z, m, part, m);
   }
-#endif
-  if (zin != nullptr)
-    hipLaunchKernelGGL((walk_moments_fp64<D, true>), dim3(grid), dim3(64), 0, st, seeds, zin, rng_stream, T, n, acc,
-                       ld);
-  else
-    hipLaunchKernelGGL((walk_moments_fp64<D, false>), dim3(grid), dim3(64), 0, st, seeds, zin, rng_stream, T, n,
-                       acc, ld);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(walk_blocks_add<D>, dim3((m + 63) / 64, AddShape<D>::NH), dim3(64 * D), 0, st, T, m, part, acc + turns, ld);
   return hipGetLastError();
 }
 
@@ -770,11 +1112,12 @@ static hipError_t launch_eigen_md(const double* acc, size_t ld, uint32_t T, uint
 }
 
 hipError_t launch_walk_moments_fp64(int d, const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                    uint32_t n, double* acc, size_t ld, hipStream_t st) {
+                                    uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                    hipStream_t st) {
   switch (d) {
 #define JNE_CASE(DD) \
   case DD:           \
-    return launch_moments_d<DD>(seeds, zin, rng_stream, T, n, acc, ld, st);
+    return launch_moments_d<DD>(seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
     JNE_CASE(1) JNE_CASE(2) JNE_CASE(3) JNE_CASE(4) JNE_CASE(5) JNE_CASE(6)
     JNE_CASE(7) JNE_CASE(8) JNE_CASE(9) JNE_CASE(10) JNE_CASE(11) JNE_CASE(12)
 #undef JNE_CASE

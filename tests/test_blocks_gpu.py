@@ -1,0 +1,39 @@
+"""The FP64 moment pass's forms: a walk's blocks of steps taken in turn by one
+lane group (whole rounds of a batch that fills the GPU), one lane group per
+block, or one wave per block.  The blocks' sums and the order they are added
+in are the same in every form, so a batch, its pieces and single walks give
+the same bits; each length is also held to the C oracle at 1e-9."""
+import numpy as np
+import pytest
+
+from conftest import assert_eigs_close
+
+pytestmark = pytest.mark.gpu
+
+# one walk per lane up to dim 7 (64 per wave at 4, 4, 4, 3, 2, 2, 2 waves per SIMD), lane groups above
+ROUND = {1: 262144, 2: 262144, 3: 262144, 4: 196608, 5: 131072, 6: 131072, 7: 131072, 8: 65536, 9: 28672, 10: 36864,
+         11: 32768, 12: 32768}
+
+
+@pytest.mark.parametrize("dim,steps", [(1, 2)] + [(d, t) for d in range(1, 13) for t in (239, 241, 483)])
+def test_forms_give_the_same_bits(engine, O, dim, steps):
+    model = 0 if steps == 2 else dim % 5
+    n = ROUND[dim] + 9001  # a whole round (blocks in turn) and a split rest
+    seeds = np.arange(11, 11 + n, dtype=np.uint32)
+    full = engine.eigenvalues_by_seed(model, dim, steps, seeds)
+    for at, m in [(0, 20000), (n - 20000, 20000), (5, 100), (n - 1, 1)]:
+        part = engine.eigenvalues_by_seed(model, dim, steps, seeds[at:at + m])
+        assert np.array_equal(part, full[at:at + m]), (dim, steps, at, m)
+    ends = np.r_[0:3, n - 3:n]
+    assert_eigs_close(full[ends], O.walks_by_seed_c(model, dim, steps, seeds[ends]), 1e-9, f"dim {dim} steps {steps}")
+
+
+@pytest.mark.parametrize("dim", [1, 4, 7, 8, 12])
+def test_long_blocks(engine, O, dim):
+    """T > 3,840: blocks of more than 240 steps, the last one partial; from-normals and by-seed."""
+    steps, seeds = 7999, np.arange(1, 2501, dtype=np.uint32)
+    full = engine.eigenvalues_by_seed(4, dim, steps, seeds)
+    assert np.array_equal(full[7:9], engine.eigenvalues_by_seed(4, dim, steps, seeds[7:9]))
+    assert_eigs_close(full[:2], O.walks_by_seed_c(4, dim, steps, seeds[:2]), 1e-9, f"dim {dim}")
+    z = engine.walk_normals(dim, steps, seeds[:40]).astype(np.float64)
+    assert np.array_equal(engine.eigenvalues_from_normals(4, z), full[:40])
