@@ -49,9 +49,10 @@ constexpr int steps_per_round(int d, int L) {
   return first;
 }
 
-template <int D>
+// LW: lanes per walk
+template <int D, int LW = lanes_for_dim(D)>
 struct WalkShape {
-  static constexpr int L = lanes_for_dim(D);          // lanes per walk
+  static constexpr int L = LW;
   static constexpr int DP = ((D + L - 1) / L) * L;     // dim padded to L
   static constexpr int GPW = 64 / L;                   // walks per wave
   static constexpr int S = steps_per_round(D, L);      // steps per round
@@ -67,6 +68,11 @@ struct WalkShape {
 template <bool B>
 struct BoolTag {
   static constexpr bool value = B;
+};
+
+template <int N>
+struct IntTag {
+  static constexpr int value = N;
 };
 
 template <int D>

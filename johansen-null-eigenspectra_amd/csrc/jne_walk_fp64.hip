@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "jne_blocks.h"
@@ -70,6 +71,10 @@ namespace jne {
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void keep_order() { asm volatile("" ::: "memory"); }
 
+// waves per SIMD (the register cap) of a lane group of LW lanes: the dim's
+// own shape, or one row of the sums per lane (LW = D, at most 96 registers)
+constexpr int group_waves(int d, int lw) { return lw == lanes_for_dim(d) ? waves_for_dim(d) : 4; }
+
 // A lane's sums over the blocks it takes in turn, between blocks: the first
 // NR of its slots in registers, the next NL in LDS, the rest in acc (at x,
 // where their last value goes).  The slots are compile-time constants once
@@ -102,11 +107,11 @@ struct Fp64Totals {
 };
 constexpr Fp64Totals kFp64Totals[12] = {JNE_FP64_TOTALS};
 
-template <int D, bool FROM_NORMALS, bool SPLIT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(waves_for_dim(D), waves_for_dim(D))))
+template <int D, int LW, bool FROM_NORMALS, bool SPLIT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(group_waves(D, LW), group_waves(D, LW))))
 void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
                        uint32_t T, uint32_t n_walks, double* __restrict__ acc, size_t ld) {
-  using Sh = WalkShape<D>;
+  using Sh = WalkShape<D, LW>;
   constexpr int L = Sh::L;
   constexpr int DP = Sh::DP;
   constexpr int R = DP / L;
@@ -1017,25 +1022,33 @@ __global__ __launch_bounds__(64) void walk_eigen_jacobi(const double* __restrict
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// The forms of a moment launch.  One lane group per walk fills the GPU (`slots`
+// The forms of a moment launch.  One lane group per walk fills the GPU (the
 // waves resident at the kernel's occupancy) in whole rounds only; the walks of
-// the last, partial round are split over their blocks where a walk has
-// several.  Walks whose blocks (in units of kBlockUnit steps) number at most
-// kWaveForm get one wave per block, more get one lane group per block: the
-// line lies where the two take the same time, between T = 300 and 2,000 (ms,
-// group / wave form: dim 1, 2,000 units 0.024 / 0.019, 8,000 0.024 / 0.036;
-// dim 5, 9,000 0.140 / 0.114, 18,000 0.124 / 0.176; dim 12, 2,000 0.115 /
-// 0.061, 4,500 0.150 / 0.179).  A split walk also writes and reads its blocks'
-// sums (4 to 30% of the whole, more at the high dims and short blocks), so a
-// rest of ROUND_FILL of a round or more is not split.  100,000 walks at
-// T = 2,000, in turn and split: dim 1 0.232 and 0.171 ms, dim 5 1.52 and 1.22;
-// 10,000 walks at T = 8,000: dim 1 0.607 and 0.112, dim 5 3.62 and 0.59,
-// dim 12 3.60 and 1.85.
+// the last, partial round are split over their blocks, as are all walks of a
+// batch too small for one lane group each.  With units = walks x blocks of
+// kBlockUnit steps, the split walks get
+//   one wave per block          up to kWaveForm units,
+//   one lane per component      up to kRowForm units (walk_moments_fp64, L = dim),
+//   the dim's own lane group    above.
+// The lines lie where two forms take the same time (T = 150 to 2,000; own
+// group / row / wave form, ms): dim 3, T = 240: 4,000 units 0.065 / 0.045 /
+// 0.044, 8,000 0.065 / 0.048 / 0.075, 30,000 0.068 / 0.067 / 0.24; dim 7:
+// 2,000 0.156 / 0.049 / 0.048, 30,000 0.171 / 0.127 / 0.42, 60,000 0.183 /
+// 0.205 / 0.81; dim 12: 2,000 0.110 / 0.060 / 0.078, 16,000 0.128 / 0.155 /
+// 0.46.  A split walk also writes and reads its blocks' sums (4 to 30% of the
+// whole, more at the high dims and short blocks), so a rest of ROUND_FILL of a
+// round or more is not split.  100,000 walks at T = 2,000, in turn and split:
+// dim 1 0.232 and 0.171 ms, dim 5 1.52 and 1.22; 10,000 walks at T = 8,000:
+// dim 1 0.607 and 0.112, dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
 constexpr uint32_t kSimds = 1024;
 #ifndef JNE_WAVE_FORM
-#define JNE_WAVE_FORM 3500, 5000, 7000, 10000, 13000, 15000, 11000, 8000, 3000, 3000, 4000, 3200
+#define JNE_WAVE_FORM 3500, 4000, 5000, 4000, 4500, 4500, 2000, 1500, 1500, 1500, 1500, 1000
 #endif
 constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
+#ifndef JNE_ROW_FORM
+#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 45000, 24000, 0, 14000, 13000, 12000
+#endif
+constexpr uint32_t kRowForm[12] = {JNE_ROW_FORM};
 #ifndef JNE_ROUND_FILL
 #define JNE_ROUND_FILL 90  // percent of a round
 #endif
@@ -1045,7 +1058,7 @@ static uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   const uint32_t L = lanes_for_dim(d);
   const uint32_t round = (64 / L) * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
   const uint32_t rest = n % round;
-  if (block_count(T) == 1) return n > kWaveForm[d - 1] ? n : 0;
+  if (block_count(T) == 1) return n > std::max(kWaveForm[d - 1], kRowForm[d - 1]) ? n : 0;
   return (uint64_t)rest * 100 >= (uint64_t)round * JNE_ROUND_FILL ? n : n - rest;
 }
 
@@ -1057,40 +1070,53 @@ template <int D>
 static hipError_t launch_moments_d(const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
                                    uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
                                    hipStream_t st) {
-  constexpr bool kReg = WalkShape<D>::L == 1;
-  constexpr uint32_t GPW = WalkShape<D>::GPW;
-  auto go = [&](auto fn_tag, auto split_tag, const uint32_t* s, const double* z, uint32_t m, double* out, size_t ldo) {
-    constexpr bool FN = decltype(fn_tag)::value, SPLIT = decltype(split_tag)::value;
-    const dim3 grid((m + GPW - 1) / GPW, SPLIT ? block_count(T) : 1);
-    if constexpr (kReg)
-      hipLaunchKernelGGL((walk_moments_fp64_reg<D, FN, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out, ldo);
-    else
-      hipLaunchKernelGGL((walk_moments_fp64<D, FN, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out, ldo);
+  constexpr int L = WalkShape<D>::L;
+  // LW lanes per walk (0: one wave) for m walks into out
+  auto go = [&](auto lw_tag, auto split_tag, const uint32_t* s, const double* z, uint32_t m, double* out, size_t ldo) {
+    constexpr int LW = decltype(lw_tag)::value;
+    constexpr bool SPLIT = decltype(split_tag)::value;
+    const dim3 grid(LW == 0 ? m : (m + 64 / (LW ? LW : 1) - 1) / (64 / (LW ? LW : 1)), SPLIT ? block_count(T) : 1);
+    if constexpr (LW == 0) {
+      if (z)
+        hipLaunchKernelGGL((walk_moments_fp64_wave<D, true>), grid, dim3(64), 0, st, s, z, rng_stream, T, out, ldo);
+      else
+        hipLaunchKernelGGL((walk_moments_fp64_wave<D, false>), grid, dim3(64), 0, st, s, z, rng_stream, T, out, ldo);
+    } else if constexpr (LW == 1) {
+      if (z)
+        hipLaunchKernelGGL((walk_moments_fp64_reg<D, true, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out,
+                           ldo);
+      else
+        hipLaunchKernelGGL((walk_moments_fp64_reg<D, false, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out,
+                           ldo);
+    } else {
+      if (z)
+        hipLaunchKernelGGL((walk_moments_fp64<D, LW, true, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out,
+                           ldo);
+      else
+        hipLaunchKernelGGL((walk_moments_fp64<D, LW, false, SPLIT>), grid, dim3(64), 0, st, s, z, rng_stream, T, m, out,
+                           ldo);
+    }
     return hipGetLastError();
   };
   uint32_t turns = fp64_turns(D, T, n);
   if (part == nullptr || part_doubles < fp64_part_doubles(D, T, n)) turns = n;
   hipError_t e = hipSuccess;
-  if (turns > 0)
-    e = zin ? go(BoolTag<true>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld)
-            : go(BoolTag<false>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld);
+  if (turns > 0) e = go(IntTag<L>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld);
   if (e != hipSuccess || turns == n) return e;
   // the split rest
   const uint32_t m = n - turns;
   const uint32_t* s = seeds ? seeds + turns : nullptr;
   const double* z = zin ? zin + (size_t)turns * T * D : nullptr;
-  if ((uint64_t)m * ((T + kBlockUnit - 1) / kBlockUnit) <= kWaveForm[D - 1]) {
-    const dim3 grid(m, block_count(T));
-    if (z)
-      hipLaunchKernelGGL((walk_moments_fp64_wave<D, true>), grid, dim3(64), 0, st, s, z, rng_stream, T, part, (size_t)m);
-    else
-      hipLaunchKernelGGL((walk_moments_fp64_wave<D, false>), grid, dim3(64), 0, st, s, z, rng_stream, T, part, (size_t)m);
-    e = hipGetLastError();
-  } else {
-    e = z ? go(BoolTag<true>{}, BoolTag<true>{}, s, z, m, part, m) : go(BoolTag<false>{}, BoolTag<true>{}, s, z, m, part, m);
-  }
+  const uint64_t units = (uint64_t)m * ((T + kBlockUnit - 1) / kBlockUnit);
+  if (units <= kWaveForm[D - 1])
+    e = go(IntTag<0>{}, BoolTag<true>{}, s, z, m, part, m);
+  else if (units <= kRowForm[D - 1])
+    e = go(IntTag<D>{}, BoolTag<true>{}, s, z, m, part, m);
+  else
+    e = go(IntTag<L>{}, BoolTag<true>{}, s, z, m, part, m);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(walk_blocks_add<D>, dim3((m + 63) / 64, AddShape<D>::NH), dim3(64 * D), 0, st, T, m, part, acc + turns, ld);
+  hipLaunchKernelGGL(walk_blocks_add<D>, dim3((m + 63) / 64, AddShape<D>::NH), dim3(64 * D), 0, st, T, m, part,
+                     acc + turns, ld);
   return hipGetLastError();
 }
 
