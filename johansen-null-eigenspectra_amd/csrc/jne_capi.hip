@@ -235,7 +235,9 @@ int resolve_precision(int dim, uint32_t steps, int precision) {
 
 // Scratch for splitting a launch of n walks over their blocks (0: not split).
 size_t part_doubles_for(int dim, uint32_t steps, int precision, size_t n) {
-  if (n == 0 || dim > jne::kMaxDim || resolve_precision(dim, steps, precision) != JNE_PREC_FP64) return 0;
+  if (n == 0) return 0;
+  if (dim > jne::kMaxDim) return jne::wide_part_doubles(dim, steps, (uint32_t)n);
+  if (resolve_precision(dim, steps, precision) != JNE_PREC_FP64) return 0;
   return jne::fp64_part_doubles(dim, steps, (uint32_t)n);
 }
 
@@ -256,7 +258,8 @@ int launch_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_
     const uint32_t* s = d_seeds ? d_seeds + off : nullptr;
     const double* z = d_z ? d_z + off * (size_t)steps * dim : nullptr;
     auto moments = [&] {
-      if (dim > jne::kMaxDim) return jne::launch_walk_moments_wide(dim, s, z, rng_stream, steps, cn, acc, cn, st);
+      if (dim > jne::kMaxDim) 
+        return jne::launch_walk_moments_wide(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
       if (precision == JNE_PREC_FP64) return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
       return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, st);
     };

@@ -131,7 +131,9 @@ hipError_t launch_walk_eigen_fp64(int model, int d, const double* acc, size_t ld
                                   double* out, double* mbuf, hipStream_t st);
 // the runtime-dim FP64 path, dims kMaxDim+1 .. kMaxWideDim
 hipError_t launch_walk_moments_wide(int d, const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                    uint32_t n, double* acc, size_t ld, hipStream_t st);
+                                    uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                    hipStream_t st);
+size_t wide_part_doubles(int d, uint32_t T, uint32_t n);
 hipError_t launch_walk_eigen_wide(int model, int d, const double* acc, size_t ld, uint32_t T, uint32_t n, double* out,
                                   hipStream_t st);
 hipError_t launch_walk_normals(int d, const uint32_t* seeds, uint32_t rng_stream, uint32_t T, uint32_t n,

@@ -7,15 +7,13 @@
 // eigenproblem no longer fit one lane's registers, so here one wave owns one
 // walk and keeps both in registers spread over its lanes and in LDS:
 //
-//   walk_moments_wide  the same one-pass moments as walk_moments_fp64 (the
-//                      canonical entry-major layout of jne_internal.h): per
-//                      round of S steps the wave draws the S*dim normals
-//                      (Philox calls dealt over the lanes, the stream of
-//                      jne_rng.h), lanes 0..dim-1 run the FP64 recurrence
-//                      B_{t+1} = B_t + z sqrt(dt) of their component, and every
-//                      lane adds its tile of sum [b; e] b^T (components padded
-//                      to 16, 24 or 32) and one row of the moment vectors,
-//                      FP64 fma;
+//   walk_moments_wide  the block sums of jne_blocks.h (the canonical entry-major
+//                      layout of jne_internal.h): per round of R steps the wave
+//                      draws the R*dim normals (Philox calls dealt over the
+//                      lanes, the stream of jne_rng.h), lanes 0..dim-1 run their
+//                      component's path c, and the sums of [c; z] c^T over the
+//                      round go through the FP64 matrix instructions, 4 steps at
+//                      a time;
 //   walk_eigen_wide    model algebra (S11 and S01 as Schur complements on the
 //                      moments), Cholesky of S11, W = L^-1 S10, M = W^T W,
 //                      with lanes working on matrix entries, rows or columns
@@ -32,6 +30,7 @@
 
 #include <type_traits>
 
+#include "jne_blocks.h"
 #include "jne_internal.h"
 #include "jne_rng.h"
 #include "jne_tridiag.h"
@@ -40,161 +39,338 @@ namespace jne {
 
 namespace {
 
-constexpr int kPadDim = kMaxWideDim;            // components padded to 32
-constexpr int kRoundMax = 16;                   // most steps in one round (dim 13..16)
-static_assert(kPadDim + kRoundMax <= 64, "lanes past the components form the steps' u and u^2");
+// Steps per round: a multiple of 4 that divides kBlockUnit, with at most 128
+// Philox calls; of those the one that fills the 64-lane call iterations best,
+// the longer on a tie (dim 13..16: 16, 17..19: 24, 20..25: 20 to 24, 26..32: 16).
+__host__ __device__ constexpr int wide_round_steps(int d) {
+  int best = 4;
+  for (int r = 8; r <= 24; r += 4) {
+    const int calls = r * d / 4, old = best * d / 4;
+    if (calls > 128 || kBlockUnit % r != 0) continue;
+    // calls / lanes drawn against old / lanes drawn
+    if (calls * ((old + 63) / 64) >= old * ((calls + 63) / 64)) best = r;
+  }
+  return best;
+}
 
-// Steps per round: a multiple of 4 (whole Philox calls for any dim) with at
-// most 64 calls, so each lane draws at most one call per round.
-__host__ __device__ constexpr int wide_round_steps(int d) { return ((256 / d) & ~3) < 4 ? 4 : ((256 / d) & ~3); }
+typedef double d64x4 __attribute__((ext_vector_type(4)));
 
 }  // namespace
 
-// One wave per walk (blockIdx.x).  The components are padded to DP = 16, 24
-// or 32 (dims 13-16, 17-24, 25-32), and lane l owns an RB x CB tile of the
-// stacked rows y = [b (DP, zero-padded); e (DP)] against the columns b:
-// rows RB (l / NCB) .. + RB - 1, columns CB (l % NCB) .. + CB - 1, so that the
-// 64 tiles cover sum y b^T = [sum b b^T; sum e b^T] (DP = 16: 2 x 4 tiles,
-// 24: 3 x 6, 32: 8 x 4); lanes l < 2 DP also add sum y_l, sum u y_l and
-// sum u^2 y_l.
-template <int DP>
-struct WideTile {
-  static constexpr int CB = DP == 24 ? 6 : 4;             // columns per lane
-  static constexpr int NCB = DP / CB;                     // column blocks
-  static constexpr int RB = 2 * DP / (64 / NCB);          // rows per lane
-  static_assert((2 * DP / RB) * NCB == 64 && RB * (64 / NCB) == 2 * DP, "64 tiles");
+// The operand rows of a walk, 16 to a tile: positions 0..DB-1 the path c of the
+// components (zero from dim on), DB..2 DB-1 their normals z, DB = 4 NB.  A lane's
+// operand of tile q is X[position 16 q + l % 16][step 4 g + l / 16], as A (rows)
+// and B (columns) alike.
+template <int NB>
+struct WideShape {
+  static constexpr int DB = 4 * NB;
+  static constexpr int NT = (2 * NB + 3) / 4;               // tiles
+  static constexpr int NR = NB == 8 ? 2 : 1;                // row tiles taken by 16x16x4 products
+  static constexpr int NU = NB == 8 ? 0 : NB - 4;           // 4-row blocks past them: 4x4x4 products
+  static constexpr int NC = NB == 4 ? 1 : 2;                // tiles that hold path components
+  static constexpr int N16 = NB == 8 ? 2 * NT - 1 : NT;     // 16x16 accumulators
+  static constexpr int N4 = NU * (NT - 1);                  // 4x4 accumulators (4 blocks each)
+  static constexpr int ND = 4 * N16 + N4;                   // accumulator doubles per lane
+  static constexpr int waves = NB <= 6 ? 4 : 3;
+  // accumulator entry x of lane l: its row (a component) and column (a position)
+  static __device__ __forceinline__ void entry(int x, int l, int& row, int& col) {
+    if (x < 4 * N16) {
+      const int t = x / 4, r = x % 4;
+      row = l / 16 + 4 * r + (t >= NT ? 16 : 0);
+      col = 16 * (t >= NT ? t - NT + 1 : t) + l % 16;
+    } else {
+      const int y = x - 4 * N16;
+      row = 16 + 4 * (y / (NT - 1)) + l / 16;
+      col = 16 * (1 + y % (NT - 1)) + l % 16;
+    }
+  }
 };
 
-template <int DP, bool FROM_NORMALS>
-__global__ __launch_bounds__(64) void walk_moments_wide(const uint32_t* __restrict__ seeds,
-                                                        const double* __restrict__ zin, uint32_t rng_stream,
-                                                        uint32_t T, uint32_t n_walks, int D,
-                                                        double* __restrict__ acc, size_t ld) {
-  using Tl = WideTile<DP>;
-  constexpr int RB = Tl::RB, CB = Tl::CB, NCB = Tl::NCB;
-  __shared__ __align__(16) double ys[kRoundMax][2 * DP];  // per step of the round: b, then e
-  __shared__ double wz[kRoundMax * kPadDim];              // the round's increments z sqrt(dt), t-major
-  // u_t and u_t^2 of the round's steps, formed once per round by spare lanes
-  // at DP = 32 (3% faster there; at DP = 16 and 24, whose steps carry fewer
-  // FMAs, the extra LDS read per step costs more than the 3 VALU it saves)
-  constexpr bool kUTable = DP == 32;
-  __shared__ __align__(16) double us[kUTable ? kRoundMax : 1][2];
+// One wave per walk, taking its blocks in turn with the totals in registers, or
+// (SPLIT) per block blockIdx.y of a walk, its sums to acc for wide_blocks_add.
+//
+// Bound by the FP64 matrix instructions and the normals, which share the SIMD:
+// a 16x16x4 product takes 65 cycles (15.8 FMAs per cycle against 14.2 from
+// v_fma_f64) and 4x4x4 ones fill the rows past 16 where a 16-row tile would be
+// mostly padding.  Operands are read once per 4 steps (2 to 8 LDS reads per
+// lane); the VALU tiles that stood here read 8 to 13 doubles per lane and step
+// for 8 to 32 FMAs and were bound by LDS.  At dim 32 a step costs 218 cycles of
+// its SIMD, 112 of them in matrix instructions and 78 in the 25 VALU ones, most
+// of those the normals'.  Before and now, ms: 16,384 walks at T = 10^4, dim 32
+// 22.7 and 15.8 (eigen solve included); 12,288 walks at T = 4,000, dim 16 3.16
+// and 1.79, dim 20 4.36 and 2.90, dim 24 4.72 and 3.03; 500 walks there (split
+// over their blocks), dim 16 0.484 and 0.129, dim 32 0.879 and 0.251.  The
+// symmetric tile as three 4x4x4 products (50 cycles for 65) gained nothing:
+// its operands are two more LDS reads.
+template <int NB, bool FROM_NORMALS, bool SPLIT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WideShape<NB>::waves)))
+void walk_moments_wide(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
+                       uint32_t T, uint32_t n_walks, int D, double* __restrict__ acc, size_t ld) {
+  using Sh = WideShape<NB>;
+  constexpr int DB = Sh::DB, NT = Sh::NT, ND = Sh::ND;
+  extern __shared__ double wide_x[];  // X[tile][step][16], R steps (wide_moments_lds_bytes)
+  __shared__ double qv[16 * NT], bv[16 * NT], sv[32], a1v[32], a2v[32];
   const int l = threadIdx.x;
   const size_t walk = blockIdx.x;
   if (walk >= n_walks) return;  // whole wave exits together
-  const int S = wide_round_steps(D);
-  const int calls = S * D / 4;
+  const int R = wide_round_steps(D);
+  const int calls = R * D / 4;
   uint32_t seed = 0;
   if constexpr (!FROM_NORMALS) seed = seeds[walk];
   const double* zw = FROM_NORMALS ? zin + walk * (size_t)T * D : nullptr;
+  auto at = [&](int pos, int t) { return ((pos >> 4) * R + t) * 16 + (pos & 15); };
 
-  // padding rows and columns stay zero
-  for (int e = l; e < kRoundMax * 2 * DP; e += 64) (&ys[0][0])[e] = 0.0;
+  for (int e = l; e < NT * R * 16; e += 64) wide_x[e] = 0.0;  // the padding stays zero
+  // where the normals of this lane's calls l and l + 64 of a round go
+  int zo[2][4], zt[2];
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int n0 = 4 * (l + 64 * it);
+    int t = n0 / D, i = n0 - t * D;
+    zt[it] = t;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      zo[it][j] = at(DB + i, t);
+      if (++i == D) {
+        i = 0;
+        ++t;
+      }
+    }
+  }
   __syncthreads();
 
-  const int rb = l / NCB, cb = l % NCB;
-  double g[RB][CB];
+  double tot[SPLIT ? 1 : ND], m0 = 0.0, m1 = 0.0, m2 = 0.0, base = 0.0;  // base: the state at the block's start
+  if constexpr (!SPLIT) {
 #pragma unroll
-  for (int r = 0; r < RB; ++r)
+    for (int x = 0; x < ND; ++x) tot[x] = 0.0;
+  }
+  const uint32_t bn = block_steps(T);
+  uint32_t ts = SPLIT ? blockIdx.y * bn : 0;
+  do {
+    const uint32_t n = T - ts < bn ? T - ts : bn;
+    d64x4 g16[Sh::N16];
+    double g4[Sh::N4 > 0 ? Sh::N4 : 1], s[Sh::NC], a1[Sh::NC], a2[Sh::NC];
 #pragma unroll
-    for (int c = 0; c < CB; ++c) g[r][c] = 0.0;
-  double m0 = 0.0, m1 = 0.0, m2 = 0.0;  // sum y_l, sum u y_l, sum u^2 y_l (lanes l < 2 DP)
-  const int lm = l < 2 * DP ? l : 0;
+    for (int x = 0; x < Sh::N16; ++x) g16[x] = d64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int x = 0; x < Sh::N4; ++x) g4[x] = 0.0;
+#pragma unroll
+    for (int q = 0; q < Sh::NC; ++q) s[q] = a1[q] = a2[q] = 0.0;
+    double c = 0.0;                                  // the path of component l (lanes l < D)
+    double mk = (double)n - 1.0 - (double)(l >> 4);  // te - (t + 1) of this lane's step
 
-  // src/johansen_statistics.rs:70 and src/rng_matrix.rs:137: sqrt(1/steps)
-  const double dt = 1.0 / (double)T;
-  const double sqrt_dt = sqrt(dt);
-  double b = 0.0;  // B_t of component l (lanes l < D)
-
-  for (uint32_t t0 = 0; t0 < T; t0 += (uint32_t)S) {
-    const int ns = (T - t0) < (uint32_t)S ? (int)(T - t0) : S;
-    // this round's increments: call l draws normals 4l..4l+3 of the round
-    if (l < calls) {
-      float v[4];
-      if constexpr (!FROM_NORMALS) normals4((uint64_t)t0 * D / 4 + l, seed, rng_stream, v);
+    for (uint32_t t0 = 0; t0 < n; t0 += R) {
+      const int ns = n - t0 < (uint32_t)R ? (int)(n - t0) : R;
+      // the round's normals
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int q = 4 * l + j;  // = s*D + i
-        double w;
-        if constexpr (FROM_NORMALS) {
-          const uint32_t t = t0 + (uint32_t)(q / D);
-          w = t < T ? zw[(size_t)t0 * D + q] * sqrt_dt : 0.0;
-        } else {
-          w = (double)v[j] * sqrt_dt;
+      for (int it = 0; it < 2; ++it) {
+        const int q = l + 64 * it;
+        if (q < calls) {
+          float v[4];
+          if constexpr (!FROM_NORMALS) normals4((uint64_t)(ts + t0) * D / 4 + q, seed, rng_stream, v);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            double z;
+            if constexpr (FROM_NORMALS)
+              z = 4 * q + j < ns * D ? zw[(size_t)(ts + t0) * D + 4 * q + j] : 0.0;
+            else
+              z = (double)v[j];
+            wide_x[zo[it][j]] = z;
+          }
         }
-        wz[q] = w;
       }
-    }
-    __syncthreads();
-    // the recurrence of component l, with the reference's rounding:
-    // B_{t+1} = B_t + z sqrt(dt) (rng_matrix.rs:138-140), e = B_{t+1} - B_t
-    // (johansen_statistics.rs:80-82)
-    if (l < D) {
-      for (int s = 0; s < ns; ++s) {
-        const double bn = b + wz[s * D + l];
-        ys[s][l] = b;
-        ys[s][DP + l] = bn - b;
-        b = bn;
+      __syncthreads();
+      // component l's path; the steps past the walk's end (its last round) are zeroed
+      if (l < D) {
+        double* const xc = wide_x + at(l, 0);
+        double* const xz = wide_x + at(DB + l, 0);
+        for (int t = ns; t < R; ++t) xz[t * 16] = 0.0;
+        for (int t = 0; t < R; t += 4) {
+          double z[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) z[j] = xz[(t + j) * 16];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            xc[(t + j) * 16] = c;
+            c += z[j];
+          }
+        }
+        for (int t = ns; t < R; ++t) xc[t * 16] = 0.0;
       }
-    } else if (kUTable && l >= kPadDim && l - kPadDim < ns) {
-      // lanes 32.. (never a component's): u_t = (t+1)/T and u_t^2 of step
-      // l - 32, the same for every lane of the moment sums below
-      const int s = l - kPadDim;
-      const double u = (double)(t0 + (uint32_t)s + 1u) * dt;
-      us[s][0] = u;
-      us[s][1] = u * u;
-    }
-    __syncthreads();
-    for (int s = 0; s < ns; ++s) {
-      double y[RB], bb[CB];
+      __syncthreads();
+      const int groups = (ns + 3) / 4;
+      for (int g = 0; g < groups; ++g) {
+        double x[NT];
 #pragma unroll
-      for (int k = 0; k < RB; ++k) y[k] = ys[s][RB * rb + k];
+        for (int q = 0; q < NT; ++q) x[q] = wide_x[(q * R + 4 * g) * 16 + l];
+        const double h = 0.5 * mk, w2 = fma(h, mk, -h);  // m and m (m - 1)/2
 #pragma unroll
-      for (int k = 0; k < CB; ++k) bb[k] = ys[s][CB * cb + k];
+        for (int q = 0; q < Sh::NC; ++q) {
+          s[q] += x[q];
+          a1[q] = fma(mk, x[q], a1[q]);
+          a2[q] = fma(w2, x[q], a2[q]);
+        }
+        mk -= 4.0;
 #pragma unroll
-      for (int r = 0; r < RB; ++r)
+        for (int q = 0; q < NT; ++q) g16[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[0], x[q], g16[q], 0, 0, 0);
+        if constexpr (NB == 8) {
 #pragma unroll
-        for (int c = 0; c < CB; ++c) g[r][c] = fma(y[r], bb[c], g[r][c]);
-      double u, u2;
-      if constexpr (kUTable) {
-        u = us[s][0];
-        u2 = us[s][1];
-      } else {
-        u = (double)(t0 + (uint32_t)s + 1u) * dt;
-        u2 = u * u;
+          for (int q = 1; q < NT; ++q)
+            g16[NT + q - 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[1], x[q], g16[NT + q - 1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < Sh::NU; ++u) {
+          // components 16 + 4 u .. + 3 in each of the four 4-row slots
+          const double xu = wide_x[(R + 4 * g) * 16 + (l & 48) + 4 * u + (l & 3)];
+#pragma unroll
+          for (int q = 1; q < NT; ++q)
+            g4[u * (NT - 1) + q - 1] =
+                __builtin_amdgcn_mfma_f64_4x4x4f64(xu, x[q], g4[u * (NT - 1) + q - 1], 0, 0, 0);
+        }
       }
-      const double yl = ys[s][lm];
-      m0 += yl;
-      m1 = fma(u, yl, m1);
-      m2 = fma(u2, yl, m2);
+      __syncthreads();
     }
-    __syncthreads();
-  }
 
-  // canonical layout, entry-major: [0, D^2) sum b b^T, [D^2, 2D^2) sum e b^T
-  // (row e, column b), then sum b, sum u b, sum u^2 b, sum e, sum u e, sum u^2 e
+    // S, A1, A2 of position 16 q + l % 16: the four step groups' shares
 #pragma unroll
-  for (int r = 0; r < RB; ++r) {
-    const int row = RB * rb + r;
-    const bool is_e = row >= DP;
-    const int i = is_e ? row - DP : row;
-    if (i >= D) continue;
+    for (int q = 0; q < Sh::NC; ++q) {
 #pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      const int j = CB * cb + c;
-      if (j < D) acc[(size_t)((is_e ? D * D : 0) + i * D + j) * ld + walk] = g[r][c];
+      for (int o = 16; o <= 32; o <<= 1) {
+        s[q] += __shfl_xor(s[q], o);
+        a1[q] += __shfl_xor(a1[q], o);
+        a2[q] += __shfl_xor(a2[q], o);
+      }
+      if (l < 16) {
+        sv[16 * q + l] = s[q];
+        a1v[16 * q + l] = a1[q];
+        a2v[16 * q + l] = a2[q];
+      }
+    }
+    __syncthreads();
+    auto grams = [&](int x) { return x < 4 * Sh::N16 ? g16[x / 4][x % 4] : g4[x - 4 * Sh::N16]; };
+    if constexpr (SPLIT) {
+      double* const o = acc + (size_t)blockIdx.y * block_moment_count(D) * ld + walk;
+#pragma unroll
+      for (int x = 0; x < ND; ++x) {
+        int i, p;
+        Sh::entry(x, l, i, p);
+        if (p < DB) {
+          if (i <= p && p < D) o[(size_t)blk_gc(D, i, p) * ld] = grams(x);
+        } else if (i < D && p - DB < D) {
+          o[(size_t)blk_ge(D, p - DB, i) * ld] = grams(x);
+        }
+      }
+      if (l < D) {
+        o[(size_t)blk_vec(D, 0, l) * ld] = sv[l];
+        o[(size_t)blk_vec(D, 1, l) * ld] = a1v[l];
+        o[(size_t)blk_vec(D, 2, l) * ld] = a2v[l];
+        o[(size_t)blk_vec(D, 3, l) * ld] = c;
+      }
+      return;
+    } else {
+      // the block's terms: for row i and column j both are B_i q_j + (S_i b_j +
+      // sum), with q, b = n B + S, B on a path column and E, 0 on a normals'
+      const BlockConst bc = block_const(ts, n);
+      if (l < D) {
+        const double sl = sv[l];
+        bv[l] = base;
+        qv[l] = fma(bc.n, base, sl);
+        bv[DB + l] = 0.0;
+        qv[DB + l] = c;
+        m0 += block_m0(bc, base, sl);
+        m1 += block_m1(bc, base, sl, a1v[l]);
+        m2 += block_m2(bc, base, sl, a1v[l], a2v[l]);
+        base += c;
+      }
+      __syncthreads();
+      // an opaque copy: the entries' indices are formed here, not kept in
+      // registers across the block
+      int lf = l;
+      asm volatile("" : "+v"(lf));
+#pragma unroll
+      for (int x = 0; x < ND; ++x) {
+        int i, p;
+        Sh::entry(x, lf, i, p);
+        if (i < D && (p < DB ? p < D : p - DB < D)) tot[x] += fma(bv[i], qv[p], fma(sv[i], bv[p], grams(x)));
+      }
+      __syncthreads();
+      ts += n;
+    }
+  } while (!SPLIT && ts < T);
+
+  if constexpr (!SPLIT) {
+    const MomentScale sc = moment_scale(T);
+    double* const o = acc + walk;
+    int lf = l;
+    asm volatile("" : "+v"(lf));
+#pragma unroll
+    for (int x = 0; x < ND; ++x) {
+      int i, p;
+      Sh::entry(x, lf, i, p);
+      const double v = tot[x] * sc.dt;
+      if (p < DB) {
+        if (i <= p && p < D) {
+          o[(size_t)(i * D + p) * ld] = v;
+          o[(size_t)(p * D + i) * ld] = v;
+        }
+      } else if (i < D && p - DB < D) {
+        o[(size_t)(D * D + (p - DB) * D + i) * ld] = v;
+      }
+    }
+    if (l < D) store_vector_moments(sc, m0, m1, m2, base, o, D, l, ld, 0);
+  }
+}
+
+// The walks' moments from their blocks' sums (part: n_walks per entry), in the
+// order and with the operations of the kernel that takes the blocks in turn:
+// 64 walks per workgroup, wave w of it row 4 blockIdx.y + w, columns
+// 8 blockIdx.z .. + 7 of sum z c^T and sum c c^T.
+__global__ __launch_bounds__(256) void wide_blocks_add(int D, uint32_t T, uint32_t n_walks,
+                                                       const double* __restrict__ part, double* __restrict__ acc,
+                                                       size_t ld) {
+  constexpr int JW = 8;
+  const int k = __builtin_amdgcn_readfirstlane(4 * blockIdx.y + (threadIdx.x >> 6)), j0 = JW * blockIdx.z;
+  const size_t walk = (size_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  if (walk >= n_walks || k >= D) return;
+  const uint32_t bn = block_steps(T);
+  const MomentScale sc = moment_scale(T);
+  const double* p = part + walk;
+  double b[JW], ge[JW], gc[JW], m0 = 0.0, m1 = 0.0, m2 = 0.0, bk = 0.0;
+#pragma unroll
+  for (int q = 0; q < JW; ++q) b[q] = ge[q] = gc[q] = 0.0;
+  for (uint32_t ts = 0; ts < T; ts += bn, p += (size_t)block_moment_count(D) * n_walks) {
+    auto at = [&](int e) { return p[(size_t)e * n_walks]; };
+    const BlockConst bc = block_const(ts, T - ts < bn ? T - ts : bn);
+    const double sk = at(blk_vec(D, 0, k)), ek = at(blk_vec(D, 3, k));
+#pragma unroll
+    for (int q = 0; q < JW; ++q) {
+      const int j = j0 + q;
+      if (j >= D) break;
+      const double bj = b[q];
+      ge[q] += fma(bj, ek, fma(at(blk_vec(D, 0, j)), 0.0, at(blk_ge(D, k, j))));
+      if (j >= k) gc[q] += block_bb(bc, bk, bj, sk, at(blk_vec(D, 0, j)), at(blk_gc(D, k, j)));
+      b[q] = bj + at(blk_vec(D, 3, j));
+    }
+    if (j0 == 0) {
+      const double x1 = at(blk_vec(D, 1, k)), x2 = at(blk_vec(D, 2, k));
+      m0 += block_m0(bc, bk, sk);
+      m1 += block_m1(bc, bk, sk, x1);
+      m2 += block_m2(bc, bk, sk, x1, x2);
+    }
+    bk += ek;
+  }
+  double* const o = acc + walk;
+#pragma unroll
+  for (int q = 0; q < JW; ++q) {
+    const int j = j0 + q;
+    if (j >= D) break;
+    o[(size_t)(D * D + k * D + j) * ld] = ge[q] * sc.dt;
+    if (j >= k) {
+      o[(size_t)(k * D + j) * ld] = gc[q] * sc.dt;
+      o[(size_t)(j * D + k) * ld] = gc[q] * sc.dt;
     }
   }
-  if (l < 2 * DP) {
-    const bool is_e = l >= DP;
-    const int i = is_e ? l - DP : l;
-    if (i < D) {
-      const int base = 2 * D * D + (is_e ? 3 * D : 0) + i;
-      acc[(size_t)base * ld + walk] = m0;
-      acc[(size_t)(base + D) * ld + walk] = m1;
-      acc[(size_t)(base + 2 * D) * ld + walk] = m2;
-    }
-  }
+  if (j0 == 0) store_vector_moments(sc, m0, m1, m2, bk, o, D, k, ld, 0);
 }
 
 namespace {
@@ -519,24 +695,57 @@ __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const do
   if (l == 0 && NX > D) o[D] = pd ? 0.0 : nan;
 }
 
+// One wave per walk in whole rounds of the GPU's resident waves; the walks of
+// the last, partial round get a wave per block, as in the kernels of dims
+// 1..12 (a rest of 90% of a round is not split, for its sums' way through memory).
+static uint32_t wide_turns(int d, uint32_t T, uint32_t n) {
+  const int nb = (d + 3) / 4;
+  const uint32_t round = 1024u * (nb <= 6 ? 4 : 3), rest = n % round;
+  if (block_count(T) == 1) return n;
+  return (uint64_t)rest * 100 >= (uint64_t)round * 90 ? n : n - rest;
+}
+
+size_t wide_part_doubles(int d, uint32_t T, uint32_t n) {
+  return (size_t)block_count(T) * block_moment_count(d) * (n - wide_turns(d, T, n));
+}
+
 hipError_t launch_walk_moments_wide(int d, const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                    uint32_t n, double* acc, size_t ld, hipStream_t st) {
+                                    uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                    hipStream_t st) {
   if (d <= kMaxDim || d > kMaxWideDim) return hipErrorInvalidValue;
-  auto go = [&](auto dp_tag) {
-    constexpr int DP = decltype(dp_tag)::value;
-    if (zin != nullptr)
-      hipLaunchKernelGGL((walk_moments_wide<DP, true>), dim3(n), dim3(64), 0, st, seeds, zin, rng_stream, T, n, d, acc,
-                         ld);
+  auto go = [&](auto nb_tag, auto split_tag, const uint32_t* s, const double* z, uint32_t m, double* out, size_t ldo) {
+    constexpr int NB = decltype(nb_tag)::value;
+    constexpr bool SPLIT = decltype(split_tag)::value;
+    const dim3 grid(m, SPLIT ? block_count(T) : 1);
+    const size_t lds = sizeof(double) * WideShape<NB>::NT * 16 * (size_t)wide_round_steps(d);
+    if (z)
+      hipLaunchKernelGGL((walk_moments_wide<NB, true, SPLIT>), grid, dim3(64), lds, st, s, z, rng_stream, T, m, d, out,
+                         ldo);
     else
-      hipLaunchKernelGGL((walk_moments_wide<DP, false>), dim3(n), dim3(64), 0, st, seeds, zin, rng_stream, T, n, d,
-                         acc, ld);
+      hipLaunchKernelGGL((walk_moments_wide<NB, false, SPLIT>), grid, dim3(64), lds, st, s, z, rng_stream, T, m, d, out,
+                         ldo);
+    return hipGetLastError();
   };
-  if (d <= 16)
-    go(std::integral_constant<int, 16>{});
-  else if (d <= 24)
-    go(std::integral_constant<int, 24>{});
-  else
-    go(std::integral_constant<int, 32>{});
+  auto go_d = [&](auto split_tag, const uint32_t* s, const double* z, uint32_t m, double* out, size_t ldo) {
+    switch ((d + 3) / 4) {
+      case 4: return go(IntTag<4>{}, split_tag, s, z, m, out, ldo);
+      case 5: return go(IntTag<5>{}, split_tag, s, z, m, out, ldo);
+      case 6: return go(IntTag<6>{}, split_tag, s, z, m, out, ldo);
+      case 7: return go(IntTag<7>{}, split_tag, s, z, m, out, ldo);
+      default: return go(IntTag<8>{}, split_tag, s, z, m, out, ldo);
+    }
+  };
+  uint32_t turns = wide_turns(d, T, n);
+  if (part == nullptr || part_doubles < wide_part_doubles(d, T, n)) turns = n;
+  hipError_t e = hipSuccess;
+  if (turns > 0) e = go_d(BoolTag<false>{}, seeds, zin, turns, acc, ld);
+  if (e != hipSuccess || turns == n) return e;
+  const uint32_t m = n - turns;
+  if ((e = go_d(BoolTag<true>{}, seeds ? seeds + turns : nullptr, zin ? zin + (size_t)turns * T * d : nullptr, m, part,
+                m)) != hipSuccess)
+    return e;
+  hipLaunchKernelGGL(wide_blocks_add, dim3((m + 63) / 64, (d + 3) / 4, (d + 7) / 8), dim3(256), 0, st, d, T, m, part,
+                     acc + turns, ld);
   return hipGetLastError();
 }
 

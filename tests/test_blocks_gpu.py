@@ -37,3 +37,17 @@ def test_long_blocks(engine, O, dim):
     assert_eigs_close(full[:2], O.walks_by_seed_c(4, dim, steps, seeds[:2]), 1e-9, f"dim {dim}")
     z = engine.walk_normals(dim, steps, seeds[:40]).astype(np.float64)
     assert np.array_equal(engine.eigenvalues_from_normals(4, z), full[:40])
+
+
+@pytest.mark.parametrize("dim", [13, 16, 17, 20, 21, 24, 25, 28, 29, 32])
+@pytest.mark.parametrize("steps", [241, 503, 4999])
+def test_wide_forms_give_the_same_bits(engine, O, dim, steps):
+    """Dims 13..32: one wave per walk taking its blocks in turn, or one per block of a walk; every
+    padded class at both ends."""
+    n = (4100 if dim <= 24 else 3100) + 300
+    seeds = np.arange(5, 5 + n, dtype=np.uint32)
+    full = engine.eigenvalues_by_seed(dim % 5, dim, steps, seeds)
+    for at, m in [(0, 700), (n - 3, 3), (17, 1)]:
+        assert np.array_equal(engine.eigenvalues_by_seed(dim % 5, dim, steps, seeds[at:at + m]), full[at:at + m])
+    ends = np.r_[0:2, n - 2:n]
+    assert_eigs_close(full[ends], O.walks_by_seed_c(dim % 5, dim, steps, seeds[ends]), 1e-9, f"dim {dim} steps {steps}")
