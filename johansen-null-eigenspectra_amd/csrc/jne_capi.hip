@@ -237,7 +237,8 @@ int resolve_precision(int dim, uint32_t steps, int precision) {
 size_t part_doubles_for(int dim, uint32_t steps, int precision, size_t n) {
   if (n == 0) return 0;
   if (dim > jne::kMaxDim) return jne::wide_part_doubles(dim, steps, (uint32_t)n);
-  if (resolve_precision(dim, steps, precision) != JNE_PREC_FP64) return 0;
+  precision = resolve_precision(dim, steps, precision);
+  if (precision != JNE_PREC_FP64) return jne::mfma_part_doubles(dim, precision, steps, (uint32_t)n);
   return jne::fp64_part_doubles(dim, steps, (uint32_t)n);
 }
 
@@ -261,7 +262,7 @@ int launch_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_
       if (dim > jne::kMaxDim) 
         return jne::launch_walk_moments_wide(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
       if (precision == JNE_PREC_FP64) return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
-      return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, st);
+      return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
     };
     if (timed)
       JNE_HIP_CHECK(ctx, timed_launch(ctx, JNE_KERNEL_MOMENTS, cn, st, moments));

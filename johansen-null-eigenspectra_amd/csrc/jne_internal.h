@@ -122,7 +122,8 @@ size_t fp64_part_doubles(int d, uint32_t T, uint32_t n);
 // the segment-split pass: the MFMA precisions and the compensated FP32 VALU check
 hipError_t launch_walk_moments_mfma(int d, int precision, const uint32_t* seeds, const double* zin,
                                     uint32_t rng_stream, uint32_t T, uint32_t n, double* acc, size_t ld,
-                                    hipStream_t st);
+                                    double* part, size_t part_doubles, hipStream_t st);
+size_t mfma_part_doubles(int d, int precision, uint32_t T, uint32_t n);
 // mbuf: (eigen_m_count(d)) * ld doubles of scratch for the two-kernel form
 // (dims whose fused solve would hold fewer than 2 waves per SIMD)
 // (none for the runtime-dim path, whose solve keeps M in LDS)

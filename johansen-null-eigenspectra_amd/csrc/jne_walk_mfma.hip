@@ -49,6 +49,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/jne.h"
 #include "jne_internal.h"
 #include "jne_rng.h"
@@ -302,13 +304,16 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float x) {
 // Philox calls of a segment unrolled: by-seed form only (the from-normals
 // form has no Philox chains to overlap), whole iterations only, and not with
 // the three-way bf16 split, whose operands leave no registers for it.  The
-// fp16x2 pass with one walk per wave keeps three calls in flight (all of a
-// dim-12 segment's three iterations) within its 128 VGPRs; the other operand
-// splits and the packed waves (W walks) hold more registers and keep two.
-template <int D, int PREC, bool FROM_NORMALS, int W = 1>
+// fp16x2 pass keeps three calls in flight, all of a dim-12 segment's three
+// iterations: within its 128 VGPRs with one walk per wave; packed waves spill 6
+// registers at dims 3 and 6 and are still 24 and 12% faster than with two
+// (65,536 walks at T = 5,000: 1.74 to 1.33 ms and 2.97 to 2.61), whose third
+// iteration is a loop of its own.  The other operand splits hold more
+// registers and keep two.
+template <int D, int PREC, bool FROM_NORMALS>
 struct CallUnroll {
   static constexpr int U =
-      PREC == JNE_PREC_MFMA_FP16X2 && W == 1 ? JNE_MFMA_UNROLL_CALLS_FP16X2 : JNE_MFMA_UNROLL_CALLS;
+      PREC == JNE_PREC_MFMA_FP16X2 ? JNE_MFMA_UNROLL_CALLS_FP16X2 : JNE_MFMA_UNROLL_CALLS;
   static constexpr int value = (U > 1 && !FROM_NORMALS && PREC != JNE_PREC_MFMA_BF16X3 && MfmaShape<D>::CALLS % 64 == 0)
                                    ? (MfmaShape<D>::IT < U ? MfmaShape<D>::IT : U)
                                    : 1;
@@ -327,8 +332,55 @@ __device__ __forceinline__ uint32_t xcd_walk(uint32_t b, uint32_t n) {
   return x * q + (x < r ? x : r) + i;
 }
 
-// D: components of the wave (W walks of D / W each)
-template <int D, int PREC, bool FROM_NORMALS, int W = 1>
+// The per-segment FP64 terms, shared by the kernel that takes a walk's segments
+// in turn and the one that adds them up from memory (mfma_segments_add), so that
+// both perform the same operations.
+struct SegLen {
+  double n, a, s1, s2;  // steps, ts + 1, sum u, sum u^2 over the segment
+};
+__device__ __forceinline__ SegLen seg_len(uint32_t ts, uint32_t n, double dt, double dt2) {
+  // sum over the segment of u^p, u = (t+1)/T, in closed form:
+  // sum_{k<n} (A + k)^p with A = ts + 1, n <= 64:
+  // n A^p + p A^(p-1) n(n-1)/2 (+ n(n-1)(2n-1)/6 for p = 2).  Positive
+  // terms and exact integers: no division and no cancellation, unlike the
+  // difference of the two cubic prefix sums
+  SegLen v;
+  v.n = (double)n;
+  v.a = (double)ts + 1.0;
+  const double k1 = (double)(n * (n - 1) / 2), k2 = (double)(n * (n - 1) * (2 * n - 1) / 6);
+  v.s1 = (v.n * v.a + k1) * dt;
+  v.s2 = ((v.n * v.a) * v.a + (2.0 * v.a) * k1 + k2) * dt2;
+  return v;
+}
+__device__ __forceinline__ double seg_state(double b0, double s, double eps, float& m) {
+  m = (float)(0.5 * eps);
+  return b0 + s * (double)m;
+}
+__device__ __forceinline__ void seg_pq(SegVec& v, double n, double s, double sig) {
+  v.P = n * v.b + s * sig;
+  v.Q = s * sig;
+}
+// rows 24..26 hold sum x, sum k x, sum k(k-1)/2 x: added as sum x, sum u x,
+// sum u^2 x with u = (a + k)/T
+__device__ __forceinline__ void seg_det(double* g, double a, double dt, double dt2, double P0, double P1, double P2) {
+  g[0] += P0;
+  g[1] += (a * P0 + P1) * dt;
+  g[2] += ((a * a) * P0 + (2.0 * a + 1.0) * P1 + 2.0 * P2) * dt2;
+}
+
+// Split batches (SPLIT): a segment's Gram as FP32 values, as the MFMA leaves
+// them, and its FP64 eps, in memory: per wave and segment kSegFloats floats
+//   c columns: rows 0..23 (accumulator v of half h of column j at v 24 + 12 h + j),
+//   z columns: rows 12..23 at 288 + 12 (row - 12) + j,
+//   rows 24..26 at 432 + 24 (row - 24) + j of the c, + 12 + j of the z columns,
+// then 12 doubles.
+constexpr int kSegFloats = 504;
+constexpr int kSegDoubles = kSegFloats / 2 + 12;
+constexpr int kSplitSegs = 4;  // segments per wave: a carry period (4 CALLS is a multiple of 64)
+
+// D: components of the wave (W walks of D / W each).  SPLIT: segments
+// kSplitSegs blockIdx.y .. + 3 of the wave's walks, to acc (see kSegFloats).
+template <int D, int PREC, bool FROM_NORMALS, int W = 1, bool SPLIT = false>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(PREC == JNE_PREC_FP32_KAHAN ? 2 : JNE_MFMA_WAVES)))
 void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
@@ -372,7 +424,8 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   const int h = l >> 5;
   const uint32_t n_groups = (n_walks + W - 1) / W;
   if (blockIdx.x >= n_groups) return;  // whole wave exits together
-  const size_t walk = (size_t)xcd_walk(blockIdx.x, n_groups) * W;  // the wave's first walk
+  // the wave's first walk
+  const size_t walk = (size_t)(SPLIT ? blockIdx.x : xcd_walk(blockIdx.x, n_groups)) * W;
   uint32_t seed = 0;
   if constexpr (!FROM_NORMALS && W == 1) seed = seeds[walk];
   const double* zw = FROM_NORMALS ? zin + walk * (size_t)T * DW : nullptr;
@@ -457,7 +510,8 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   const double s = uniform_f64(sqrt(dt));
   const double dt2 = uniform_f64(dt * dt);
   const uint32_t rounds = (T + kSegSteps - 1) / kSegSteps;
-  uint32_t drawn = 0;  // calls drawn so far (carry form): a multiple of 64
+  const uint32_t r0 = SPLIT ? blockIdx.y * kSplitSegs : 0;
+  uint32_t drawn = r0 * (uint32_t)Sh::CALLS;  // calls drawn so far (carry form): a multiple of 64
 
   // one segment; the partial last segment (T not a multiple of 64) runs a copy
   // with the step masks, so the loop over full segments carries none of them
@@ -509,7 +563,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
     } else if constexpr (W > 1) {
       // call c: local call cl of walk w, whose normals 4 cl .. 4 cl + 3 are
       // (step, component) of that walk, component i -> row w DW + i
-#pragma unroll CallUnroll<D, PREC, FROM_NORMALS, W>::value
+#pragma unroll CallUnroll<D, PREC, FROM_NORMALS>::value
       for (int j = 0; j < Sh::IT; ++j) {
         const int c = l + 64 * j;
         const int w = c / (16 * DW), cl = c - w * (16 * DW);
@@ -588,7 +642,8 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
       double e = eps_part[0][si];
 #pragma unroll
       for (int p = 1; p < SP; ++p) e += eps_part[p][si];
-      const float m = (float)(0.5 * e);
+      float m;
+      const double bm = seg_state(SPLIT ? 0.0 : b0s[si], s, e, m);
       // running sum in FP64 (exact but for FP64 rounding): each c_t is then
       // rounded to FP32 once
       double c = -(double)m;
@@ -608,15 +663,18 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
       }
       if (sp == 0) {
         seg_eps[si] = e;
-        seg[si].b = b0s[si] + s * (double)m;
-        seg[si].E = s * e;
+        if constexpr (!SPLIT) {
+          seg[si].b = bm;
+          seg[si].E = s * e;
+        }
       }
     }
     __syncthreads();
 
     // ---- the segment's Gram of X: f[v] is element [8(v/4) + 4h + v%4][l%32]
     // (the 32x32 MFMA output layout)
-    double f[16];
+    using F = typename std::conditional<SPLIT, float, double>::type;
+    F f[16];
     if constexpr (kKahan) {
       // FP32 products in Kahan-compensated FP32 sums, then to LDS
       float ks[KS::NQ], kc[KS::NQ];
@@ -656,34 +714,46 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
       }
 #pragma unroll
       for (int v = 0; v < 16; ++v)
-        f[v] = (double)((kSym && v < 12) ? __builtin_fmaf(2.0f, accc[v], accm[v]) : accm[v] + accc[v]);
+        f[v] = (F)((kSym && v < 12) ? __builtin_fmaf(2.0f, accc[v], accm[v]) : accm[v] + accc[v]);
     }
+    if constexpr (SPLIT) {
+      static_assert(kSym, "the split layout is that of the symmetric form");
+      double* const od = acc + ((size_t)blockIdx.x * rounds + r) * kSegDoubles;
+      float* const o = reinterpret_cast<float*>(od);
+      const int j = is_c ? row - kRowC : row;
+      if (is_c) {
+#pragma unroll
+        for (int v = 0; v < 12; ++v) o[24 * v + 12 * h + j] = f[v];
+      }
+      if (is_z) {
+#pragma unroll
+        for (int v = 4; v < 12; ++v) {
+          const int rw = 8 * (v / 4) + 4 * h + v % 4;
+          if (rw >= kRowC) o[288 + 12 * (rw - kRowC) + j] = f[v];
+        }
+      }
+      if (det_lane) {
+#pragma unroll
+        for (int v = 12; v < 15; ++v) o[432 + 24 * (v - 12) + (is_c ? j : 12 + j)] = f[v];
+      }
+      if (l < D) od[kSegFloats / 2 + l] = seg_eps[l];
+      __syncthreads();
+      return;
+    } else {
 
     // ---- segment end
     // f[12] on the lower half is row 24 (the ones row): sum_seg x_col
-    const uint32_t te = tail ? T : ts + kSegSteps;
-    const double nseg = (double)(te - ts);
+    const SegLen sl = seg_len(ts, (tail ? T : ts + kSegSteps) - ts, dt, dt2);
     if (h == 0 && is_c) {
-      SegVec& v = seg[row - kRowC];
-      const double sig = f[12];
-      v.P = nseg * v.b + s * sig;
-      v.Q = s * sig;
+      seg_pq(seg[row - kRowC], sl.n, s, f[12]);
     }
     __syncthreads();
     {
-      // flush into the FP64 Gram.  Rows 24..26 (v = 12..14, lower half) hold
-      // sum x, sum k x, sum k(k-1)/2 x: stored as sum x, sum u x, sum u^2 x with
-      // u = (a + k)/T, a = ts + 1; on the z columns sum x is the FP64 eps.
-      const double a = (double)ts + 1.0;
+      // flush into the FP64 Gram; on the z columns sum x is the FP64 eps
       const double P0 = is_z ? seg_eps[row] : f[12];
-      const double P1 = f[13], P2 = f[14];
 #pragma unroll
       for (int v = 0; v < 12; ++v) g[v] += f[v];
-      if (det_lane) {
-        gdl[0] += P0;
-        gdl[1] += (a * P0 + P1) * dt;
-        gdl[2] += ((a * a) * P0 + (2.0 * a + 1.0) * P1 + 2.0 * P2) * dt2;
-      }
+      if (det_lane) seg_det(gdl, sl.a, dt, dt2, P0, f[13], f[14]);
     }
     // FP64 per-segment terms on the (i, j) grid
 #pragma unroll
@@ -696,26 +766,18 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
       }
     }
     if (l < 3 * D) {
-      // sum over the segment of u^p, u = (t+1)/T, in closed form:
-      // sum_{k<n} (A + k)^p with A = ts + 1, n = te - ts <= 64:
-      // n A^p + p A^(p-1) n(n-1)/2 (+ n(n-1)(2n-1)/6 for p = 2).  Positive
-      // terms and exact integers: no division and no cancellation, unlike the
-      // difference of the two cubic prefix sums
-      const uint32_t n = te - ts;
-      const double A = (double)ts + 1.0;
-      const double k1 = (double)(n * (n - 1) / 2), k2 = (double)(n * (n - 1) * (2 * n - 1) / 6);
-      const double s1 = (nseg * A + k1) * dt;
-      const double s2 = ((nseg * A) * A + (2.0 * A) * k1 + k2) * dt2;
-      const double up = mp == 0 ? nseg : mp == 1 ? s1 : s2;
-      mb[l] += seg[mi].b * up;
+      mb[l] += seg[mi].b * (mp == 0 ? sl.n : mp == 1 ? sl.s1 : sl.s2);
     }
     __syncthreads();
     // the next reads of b0s come two barriers into the next segment
     if (l < D) b0s[l] += s * seg_eps[l];
+    }
   };
   const uint32_t full = T / kSegSteps;
-  for (uint32_t r = 0; r < full; ++r) segment(r, BoolTag<false>{});
-  if (full < rounds) segment(full, BoolTag<true>{});
+  const uint32_t r1 = SPLIT && full > r0 + kSplitSegs ? r0 + kSplitSegs : full;
+  for (uint32_t r = r0; r < r1; ++r) segment(r, BoolTag<false>{});
+  if (r1 == full && full < rounds && (!SPLIT || full < r0 + kSplitSegs)) segment(full, BoolTag<true>{});
+  if constexpr (SPLIT) return;
 
   // Lane indices of the output, recomputed from an opaque copy of the lane id
   // (an empty asm statement: no instruction), so that the compiler does not
@@ -800,13 +862,120 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   }
 }
 
+// The moments of a split batch's walks from their segments: one workgroup per
+// wave of walks, thread e < D^2 entry (i, j) of sum b b^T and sum e b^T, the next
+// 3 D threads the vector moments; each adds the segments in order with the
+// operations of walk_moments_mfma's flush and output.
+template <int D, int W>
+__global__ __launch_bounds__(192) void mfma_segments_add(uint32_t T, uint32_t n_walks, const double* __restrict__ part,
+                                                         double* __restrict__ acc, size_t ld) {
+  constexpr int DW = D / W;
+  static_assert(D * D + 3 * D <= 192, "one thread per entry");
+  const int e = threadIdx.x;
+  if (e >= D * D + 3 * D) return;
+  const size_t walk = (size_t)blockIdx.x * W;
+  const uint32_t rounds = (T + kSegSteps - 1) / kSegSteps;
+  const double* const p0 = part + (size_t)blockIdx.x * rounds * kSegDoubles;
+  const double dt = 1.0 / (double)T, s = sqrt(dt), dt2 = dt * dt, s2 = s * s;
+  auto len = [&](uint32_t r) {
+    const uint32_t ts = r * kSegSteps;
+    return seg_len(ts, T - ts < (uint32_t)kSegSteps ? T - ts : (uint32_t)kSegSteps, dt, dt2);
+  };
+  // Gram row `rw` (0..23) of c column j, and c row i (0..11) of z column j
+  auto c_at = [](int rw, int j) { return 24 * (4 * (rw / 8) + rw % 4) + 12 * ((rw / 4) & 1) + j; };
+  auto z_at = [](int i, int j) { return 288 + 12 * i + j; };
+  if (e < D * D) {
+    const int i = e / D, j = e - (e / D) * D;
+    const int lo = i < j ? i : j, hi = i < j ? j : i;
+    const int o0 = c_at(kRowC + lo, hi), o1 = c_at(kRowC + hi, lo), o2 = c_at(i, j), o3 = z_at(j, i);
+    double g0 = 0.0, g1 = 0.0, g2 = 0.0, g3 = 0.0, bbA = 0.0, ebA = 0.0, bi = 0.0, bj = 0.0;
+#pragma unroll 4
+    for (uint32_t r = 0; r < rounds; ++r) {
+      const double* const eps = p0 + (size_t)r * kSegDoubles + kSegFloats / 2;
+      const float* const f = reinterpret_cast<const float*>(p0 + (size_t)r * kSegDoubles);
+      const double ei = eps[i], ej = eps[j];
+      const double n = len(r).n;
+      SegVec vi, vj;
+      float m;
+      vi.b = seg_state(bi, s, ei, m);
+      vi.E = s * ei;
+      seg_pq(vi, n, s, (double)f[432 + i]);
+      vj.b = seg_state(bj, s, ej, m);
+      seg_pq(vj, n, s, (double)f[432 + j]);
+      g0 += (double)f[o0];
+      g1 += (double)f[o1];
+      g2 += (double)f[o2];
+      g3 += (double)f[o3];
+      bbA = fma(vi.b, vj.P, fma(vi.Q, vj.b, bbA));
+      ebA = fma(vi.E, vj.b, ebA);
+      bi += s * ei;
+      bj += s * ej;
+    }
+    const int w = i / DW, iw = i - w * DW, jw = j - w * DW;
+    if (j / DW == w && walk + w < n_walks) {
+      acc[(size_t)(iw * DW + jw) * ld + walk + w] = bbA + s2 * (0.5 * (g0 + g1));
+      acc[(size_t)(DW * DW + iw * DW + jw) * ld + walk + w] = ebA + s2 * (0.5 * (g2 + g3));
+    }
+  } else {
+    const int q = e - D * D, xp = q / D, xi = q - xp * D;
+    double gc[3] = {0.0, 0.0, 0.0}, gz[3] = {0.0, 0.0, 0.0}, mb = 0.0, b0 = 0.0;
+#pragma unroll 4
+    for (uint32_t r = 0; r < rounds; ++r) {
+      const float* const f = reinterpret_cast<const float*>(p0 + (size_t)r * kSegDoubles) + 432 + xi;
+      const double eps = p0[(size_t)r * kSegDoubles + kSegFloats / 2 + xi];
+      const SegLen sl = len(r);
+      float m;
+      const double b = seg_state(b0, s, eps, m);
+      seg_det(gc, sl.a, dt, dt2, (double)f[0], (double)f[24], (double)f[48]);
+      seg_det(gz, sl.a, dt, dt2, eps, (double)f[12 + 24], (double)f[12 + 48]);
+      mb += b * (xp == 0 ? sl.n : xp == 1 ? sl.s1 : sl.s2);
+      b0 += s * eps;
+    }
+    const int w = xi / DW, iw = xi - w * DW;
+    if (walk + w < n_walks) {
+      acc[(size_t)(2 * DW * DW + xp * DW + iw) * ld + walk + w] = mb + s * (xp == 0 ? gc[0] : xp == 1 ? gc[1] : gc[2]);
+      acc[(size_t)(2 * DW * DW + (3 + xp) * DW + iw) * ld + walk + w] =
+          s * (xp == 0 ? gz[0] : xp == 1 ? gz[1] : gz[2]);
+    }
+  }
+}
+
+// fp16x2 batches by seed whose waves leave the GPU mostly idle are split over
+// their walks' segments: a segment then also writes and reads its 2.1 KB, as
+// long as its share of a full GPU's time, so the line lies where the two forms
+// meet (waves; in turn / split, ms): dim 12, T = 1,000: 400 0.039 / 0.026, 800
+// 0.040 / 0.043; T = 10^4: 1 0.307 / 0.06, 400 0.325 / 0.161, 800 0.330 / 0.267,
+// 1,200 0.387 / 0.417; dim 7, T = 400: 400 0.0196 / 0.0188, 800 0.0204 / 0.0218.
+static uint32_t mfma_wave_walks(int d) { return JNE_MFMA_PACK && 12 % d == 0 ? 12 / d : 1; }
+#ifndef JNE_MFMA_SPLIT_WAVES
+#define JNE_MFMA_SPLIT_WAVES 700
+#endif
+size_t mfma_part_doubles(int d, int precision, uint32_t T, uint32_t n) {
+  const uint32_t waves = (n + mfma_wave_walks(d) - 1) / mfma_wave_walks(d), rounds = (T + kSegSteps - 1) / kSegSteps;
+  if (precision != JNE_PREC_MFMA_FP16X2 || waves > JNE_MFMA_SPLIT_WAVES || rounds <= (uint32_t)kSplitSegs) return 0;
+  return (size_t)waves * rounds * kSegDoubles;
+}
+
 template <int D, int PREC>
 static hipError_t launch_mfma_dp(const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                 uint32_t n, double* acc, size_t ld, hipStream_t st) {
+                                 uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                 hipStream_t st) {
   // dims dividing 12: 12 / D walks per wave as one 12-component walk
   constexpr int W = (JNE_MFMA_PACK && 12 % D == 0) ? 12 / D : 1;
   constexpr int DS = D * W;
   const unsigned grid = (n + W - 1) / W;
+  if constexpr (PREC == JNE_PREC_MFMA_FP16X2) {
+    const size_t need = mfma_part_doubles(D, PREC, T, n);
+    if (zin == nullptr && part != nullptr && need > 0 && need <= part_doubles) {
+      const unsigned chunks = ((T + kSegSteps - 1) / kSegSteps + kSplitSegs - 1) / kSplitSegs;
+      hipLaunchKernelGGL((walk_moments_mfma<DS, PREC, false, W, true>), dim3(grid, chunks), dim3(64), 0, st, seeds, zin,
+                         rng_stream, T, n, part, ld);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL((mfma_segments_add<DS, W>), dim3(grid), dim3(192), 0, st, T, n, part, acc, ld);
+      return hipGetLastError();
+    }
+  }
   if (zin != nullptr)
     hipLaunchKernelGGL((walk_moments_mfma<DS, PREC, true, W>), dim3(grid), dim3(64), 0, st, seeds, zin, rng_stream, T,
                        n, acc, ld);
@@ -818,11 +987,12 @@ static hipError_t launch_mfma_dp(const uint32_t* seeds, const double* zin, uint3
 
 template <int PREC>
 static hipError_t launch_mfma_p(int d, const uint32_t* seeds, const double* zin, uint32_t rng_stream, uint32_t T,
-                                uint32_t n, double* acc, size_t ld, hipStream_t st) {
+                                uint32_t n, double* acc, size_t ld, double* part, size_t part_doubles,
+                                hipStream_t st) {
   switch (d) {
 #define JNE_CASE(DD) \
   case DD:           \
-    return launch_mfma_dp<DD, PREC>(seeds, zin, rng_stream, T, n, acc, ld, st);
+    return launch_mfma_dp<DD, PREC>(seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
     JNE_CASE(1) JNE_CASE(2) JNE_CASE(3) JNE_CASE(4) JNE_CASE(5) JNE_CASE(6)
     JNE_CASE(7) JNE_CASE(8) JNE_CASE(9) JNE_CASE(10) JNE_CASE(11) JNE_CASE(12)
 #undef JNE_CASE
@@ -833,13 +1003,18 @@ static hipError_t launch_mfma_p(int d, const uint32_t* seeds, const double* zin,
 
 hipError_t launch_walk_moments_mfma(int d, int precision, const uint32_t* seeds, const double* zin,
                                     uint32_t rng_stream, uint32_t T, uint32_t n, double* acc, size_t ld,
-                                    hipStream_t st) {
+                                    double* part, size_t part_doubles, hipStream_t st) {
   switch (precision) {
-    case JNE_PREC_MFMA_FP16X2: return launch_mfma_p<JNE_PREC_MFMA_FP16X2>(d, seeds, zin, rng_stream, T, n, acc, ld, st);
-    case JNE_PREC_MFMA_BF16X2: return launch_mfma_p<JNE_PREC_MFMA_BF16X2>(d, seeds, zin, rng_stream, T, n, acc, ld, st);
-    case JNE_PREC_MFMA_BF16X3: return launch_mfma_p<JNE_PREC_MFMA_BF16X3>(d, seeds, zin, rng_stream, T, n, acc, ld, st);
-    case JNE_PREC_MFMA_FP32: return launch_mfma_p<JNE_PREC_MFMA_FP32>(d, seeds, zin, rng_stream, T, n, acc, ld, st);
-    case JNE_PREC_FP32_KAHAN: return launch_mfma_p<JNE_PREC_FP32_KAHAN>(d, seeds, zin, rng_stream, T, n, acc, ld, st);
+    case JNE_PREC_MFMA_FP16X2: 
+      return launch_mfma_p<JNE_PREC_MFMA_FP16X2>(d, seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
+    case JNE_PREC_MFMA_BF16X2: 
+      return launch_mfma_p<JNE_PREC_MFMA_BF16X2>(d, seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
+    case JNE_PREC_MFMA_BF16X3: 
+      return launch_mfma_p<JNE_PREC_MFMA_BF16X3>(d, seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
+    case JNE_PREC_MFMA_FP32: 
+      return launch_mfma_p<JNE_PREC_MFMA_FP32>(d, seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
+    case JNE_PREC_FP32_KAHAN: 
+      return launch_mfma_p<JNE_PREC_FP32_KAHAN>(d, seeds, zin, rng_stream, T, n, acc, ld, part, part_doubles, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -51,3 +51,19 @@ def test_wide_forms_give_the_same_bits(engine, O, dim, steps):
         assert np.array_equal(engine.eigenvalues_by_seed(dim % 5, dim, steps, seeds[at:at + m]), full[at:at + m])
     ends = np.r_[0:2, n - 2:n]
     assert_eigs_close(full[ends], O.walks_by_seed_c(dim % 5, dim, steps, seeds[ends]), 1e-9, f"dim {dim} steps {steps}")
+
+
+@pytest.mark.parametrize("dim", range(1, 13))
+@pytest.mark.parametrize("steps", [257, 512, 1003])
+def test_mixed_split_gives_the_same_bits(engine, jne, dim, steps):
+    """The fp16x2 pass split over its walks' segments (batches of few waves) and taking them in turn;
+    from-normals always takes them in turn."""
+    p = jne.PRECISIONS["mfma_fp16x2"]
+    n = 1300 * (12 // dim if 12 % dim == 0 else 1)  # packed dims: 12 / dim walks per wave
+    seeds = np.arange(1, 1 + n, dtype=np.uint32)
+    full = engine.eigenvalues_by_seed(dim % 5, dim, steps, seeds, precision=p)
+    for at, m in [(0, n // 2), (3, 1), (n - 7, 7)]:
+        got = engine.eigenvalues_by_seed(dim % 5, dim, steps, seeds[at:at + m], precision=p)
+        assert np.array_equal(got, full[at:at + m]), (dim, steps, at, m)
+    z = engine.walk_normals(dim, steps, seeds[:9]).astype(np.float64)
+    assert np.array_equal(engine.eigenvalues_from_normals(dim % 5, z, precision=p), full[:9])
