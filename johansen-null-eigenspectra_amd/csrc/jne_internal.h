@@ -147,6 +147,7 @@ constexpr int kMaxArrays = 2;  // arrays of one call (the server's trace and max
 struct QuantileScratch {
   void* small = nullptr;  // histogram, selection state, gathered values, radix-select state
   size_t small_bytes = 0;
+  void* host = nullptr;   // pinned: the results
   ~QuantileScratch();
 };
 // out[a*np + i] = percentile p[i] (0 <= p[i] <= 1, np <= kMaxPercentiles) of

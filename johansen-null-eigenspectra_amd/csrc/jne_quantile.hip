@@ -6,7 +6,8 @@
 // order statistics at floor(rank) and ceil(rank) are needed, so instead of
 // sorting the whole array:
 //
-//   1. min, max and a NaN flag (one pass);
+//   1. min, max and a NaN flag per workgroup (one pass; it also clears the
+//      histogram);
 //   2. a histogram of kBuckets equal-width value buckets between min and max
 //      (one pass).  The bucket index floor((x - min) * scale) is monotone in
 //      x, so the k-th smallest value lies in the bucket where the cumulative
@@ -14,7 +15,17 @@
 //   3. one workgroup finds the bucket (and the rank inside it) of every needed
 //      order statistic;
 //   4. the values of those few buckets are gathered (one pass);
-//   5. one workgroup sorts them in LDS and reads the order statistics.
+//   5. one workgroup sorts them in LDS, reads the order statistics and writes
+//      the results to pinned host memory.
+//
+// An array of at most kMaxCand values is sorted in LDS at once.
+//
+// 10^6 values: 127 to 63 us a call.  Before, 1,024 workgroups met in atomics on
+// one min and max (27 us, now 6 with a min and max per workgroup), 512 added
+// their 8,192 counts (25 us, now 61 groups in 8), the select walked its scans
+// in one thread (26 us, now 8) and a copy brought the results back.  Ending a
+// pass in its last workgroup instead of a launch was slower: the fence that
+// makes the others' writes visible cost 70 us.
 //
 // When the gathered buckets hold more than kMaxCand values (heavy ties, or a
 // few extreme values stretching the bucket width), or min/max are not finite,
@@ -46,15 +57,13 @@ __device__ __forceinline__ uint64_t ord_key(double x) {
   return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
 }
 
-// Bucket selection state of one array, written by qs_select and read by
-// qs_gather/qs_finish.
+// Bucket selection state of one array, written by qs_hist and read by qs_gather.
 struct Sel {
   uint32_t status;  // kSelect, kRadix, kNan or kEqual
   uint32_t nb;      // distinct buckets holding needed order statistics
   uint32_t m;       // values gathered
   uint32_t bucket[kMaxRanks];
   uint32_t base[kMaxRanks];     // first slot of bucket j's values
-  uint32_t count[kMaxRanks];    // values in bucket j
   uint32_t fill[kMaxRanks];     // gather cursors
   uint32_t pos[kMaxRanks];      // slot of rank k among the sorted gathered values
 };
@@ -69,10 +78,20 @@ struct QsArgs {
   double prank[kMaxPercentiles];
 };
 
-// Per-array device scratch: mm[3] (min key, max key, NaN flag), the
-// histogram, the selection state and the gathered values; then the results.
+// Workgroups of a pass over an array: up to kMaxGroups, for the histogram (whose
+// LDS copy each group adds to the array's) of at least 16,384 values each.
+constexpr unsigned kMaxGroups = 256;
+unsigned pass_groups(uint64_t n, uint64_t per) {
+  const uint64_t g = (n + per - 1) / per;
+  return g < kMaxGroups ? (unsigned)g : kMaxGroups;
+}
+
+// Per-array device scratch: the min and max keys and NaN flags of the first
+// pass's workgroups, the histogram, the selection state and the gathered values.
 struct QsArray {
-  uint64_t mm[4];
+  uint64_t lo[kMaxGroups], hi[kMaxGroups];
+  uint32_t nan[kMaxGroups];
+  uint32_t groups;  // of the first pass
   uint32_t hist[kBuckets];
   Sel sel;
   double cand[kMaxCand];
@@ -82,49 +101,53 @@ struct QsResult {
   double out[kMaxPercentiles];
 };
 
-__global__ void qs_init(QsArray* arr) {
-  QsArray& a = arr[blockIdx.y];
-  const int t = threadIdx.x;
-  if (t == 0) {
-    a.mm[0] = ~0ull;
-    a.mm[1] = 0ull;
-    a.mm[2] = 0ull;
+constexpr int kThreads = 1024;
+
+// min and max key over a workgroup (every thread gets them)
+__device__ __forceinline__ void block_minmax(uint64_t& lo, uint64_t& hi, uint64_t (&smin)[16], uint64_t (&smax)[16]) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t a = __shfl_xor((unsigned long long)lo, o), b = __shfl_xor((unsigned long long)hi, o);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
   }
-  for (int b = t; b < kBuckets; b += blockDim.x) a.hist[b] = 0u;
+  const int t = threadIdx.x;
+  if ((t & 63) == 0) {
+    smin[t >> 6] = lo;
+    smax[t >> 6] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    lo = smin[w] < lo ? smin[w] : lo;
+    hi = smax[w] > hi ? smax[w] : hi;
+  }
 }
 
-__global__ __launch_bounds__(256) void qs_minmax(QsArgs args, QsArray* arr) {
-  __shared__ uint64_t smin[256], smax[256];
-  __shared__ int snan;
+__global__ __launch_bounds__(kThreads) void qs_minmax(QsArgs args, QsArray* arr) {
+  __shared__ uint64_t smin[16], smax[16];
   const double* __restrict__ x = args.x[blockIdx.y];
   QsArray& a = arr[blockIdx.y];
   const int t = threadIdx.x;
-  if (t == 0) snan = 0;
   uint64_t lo = ~0ull, hi = 0ull;
   bool nan = false;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + t; i < args.n; i += (uint64_t)gridDim.x * 256) {
+#pragma unroll 4
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + t; i < args.n; i += (uint64_t)gridDim.x * kThreads) {
     const double v = x[i];
     nan |= isnan(v);
     const uint64_t k = ord_key(v);
     lo = k < lo ? k : lo;
     hi = k > hi ? k : hi;
   }
-  smin[t] = lo;
-  smax[t] = hi;
-  __syncthreads();
-  if (nan) snan = 1;
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) {
-      smin[t] = smin[t + s] < smin[t] ? smin[t + s] : smin[t];
-      smax[t] = smax[t + s] > smax[t] ? smax[t + s] : smax[t];
-    }
-    __syncthreads();
-  }
+  block_minmax(lo, hi, smin, smax);
+  nan = __syncthreads_or(nan);
   if (t == 0) {
-    atomicMin((unsigned long long*)&a.mm[0], (unsigned long long)smin[0]);
-    atomicMax((unsigned long long*)&a.mm[1], (unsigned long long)smax[0]);
-    if (snan) atomicOr((unsigned long long*)&a.mm[2], 1ull);
+    a.lo[blockIdx.x] = lo;
+    a.hi[blockIdx.x] = hi;
+    a.nan[blockIdx.x] = nan;
   }
+  for (unsigned b = blockIdx.x * kThreads + t; b < (unsigned)kBuckets; b += gridDim.x * kThreads) a.hist[b] = 0u;
+  if (blockIdx.x == 0 && t == 0) a.groups = gridDim.x;
 }
 
 __device__ __forceinline__ double from_key(uint64_t k) {
@@ -132,134 +155,31 @@ __device__ __forceinline__ double from_key(uint64_t k) {
 }
 
 // The bucket grid of an array from its min and max: kSelect when it is
-// usable, else the reason (every thread of every kernel decides the same).
-__device__ __forceinline__ uint32_t grid_of(const QsArray& a, double& lo, double& scale) {
-  lo = from_key(a.mm[0]);
-  const double hi = from_key(a.mm[1]);
-  if (a.mm[2]) return kNan;
-  if (lo == hi) return kEqual;
-  const double width = hi - lo;
-  if (!(isfinite(lo) && isfinite(hi) && isfinite(width) && width > 0.0)) return kRadix;
-  scale = (double)kBuckets / width;
-  return kSelect;
+// usable, else the reason (every thread of every workgroup decides the same).
+struct Grid {
+  double lo, scale;
+  uint64_t min_key;
+  uint32_t status;
+};
+__device__ __forceinline__ Grid grid_of(const QsArray& a, uint64_t (&smin)[16], uint64_t (&smax)[16]) {
+  Grid g;
+  const unsigned t = threadIdx.x, n = a.groups;
+  uint64_t lo = t < n ? a.lo[t] : ~0ull, hi = t < n ? a.hi[t] : 0ull;
+  const bool nan = __syncthreads_or(t < n && a.nan[t] != 0);
+  block_minmax(lo, hi, smin, smax);
+  g.min_key = lo;
+  g.lo = from_key(lo);
+  const double top = from_key(hi), width = top - g.lo;
+  g.scale = (double)kBuckets / width;
+  g.status = nan ? kNan
+             : g.lo == top ? kEqual
+             : isfinite(g.lo) && isfinite(top) && isfinite(width) && width > 0.0 ? kSelect : kRadix;
+  return g;
 }
 
-__device__ __forceinline__ uint32_t bucket_of(double v, double lo, double scale) {
-  const double f = (v - lo) * scale;  // >= 0, monotone in v
+__device__ __forceinline__ uint32_t bucket_of(double v, const Grid& g) {
+  const double f = (v - g.lo) * g.scale;  // >= 0, monotone in v
   return f < (double)(kBuckets - 1) ? (uint32_t)f : (uint32_t)(kBuckets - 1);
-}
-
-__global__ __launch_bounds__(256) void qs_hist(QsArgs args, QsArray* arr) {
-  __shared__ uint32_t h[kBuckets];
-  const double* __restrict__ x = args.x[blockIdx.y];
-  QsArray& a = arr[blockIdx.y];
-  double lo, scale;
-  if (grid_of(a, lo, scale) != kSelect) return;  // the same for every thread
-  const int t = threadIdx.x;
-  for (int b = t; b < kBuckets; b += 256) h[b] = 0u;
-  __syncthreads();
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + t; i < args.n; i += (uint64_t)gridDim.x * 256)
-    atomicAdd(&h[bucket_of(x[i], lo, scale)], 1u);
-  __syncthreads();
-  for (int b = t; b < kBuckets; b += 256)
-    if (h[b]) atomicAdd(&a.hist[b], h[b]);
-}
-
-// One workgroup of 256 threads per array, each owning kBuckets/256
-// consecutive buckets.
-__global__ __launch_bounds__(256) void qs_select(QsArgs args, QsArray* arr) {
-  constexpr int kPer = kBuckets / 256;
-  __shared__ uint64_t part[256];
-  __shared__ uint32_t rb[kMaxRanks];  // bucket of rank k
-  __shared__ uint64_t rl[kMaxRanks];  // rank of k inside its bucket
-  QsArray& a = arr[blockIdx.y];
-  Sel* sel = &a.sel;
-  const int t = threadIdx.x;
-  const int nr = 2 * args.np;
-  double lo, scale;
-  const uint32_t g = grid_of(a, lo, scale);
-  if (g != kSelect) {
-    if (t == 0) sel->status = g;
-    return;
-  }
-  uint64_t s = 0;
-  for (int j = 0; j < kPer; ++j) s += a.hist[t * kPer + j];
-  part[t] = s;
-  __syncthreads();
-  if (t == 0) {  // exclusive prefix of the 256 chunk sums
-    uint64_t acc = 0;
-    for (int j = 0; j < 256; ++j) {
-      const uint64_t v = part[j];
-      part[j] = acc;
-      acc += v;
-    }
-  }
-  __syncthreads();
-  uint64_t cum = part[t];
-  for (int j = 0; j < kPer; ++j) {
-    const int b = t * kPer + j;
-    const uint64_t c = a.hist[b];
-    for (int k = 0; k < nr; ++k) {
-      if (args.ranks[k] >= cum && args.ranks[k] < cum + c) {
-        rb[k] = (uint32_t)b;
-        rl[k] = args.ranks[k] - cum;
-      }
-    }
-    cum += c;
-  }
-  __syncthreads();
-  if (t == 0) {
-    // distinct buckets in increasing order, their slots among the gathered values
-    uint32_t nb = 0, m = 0;
-    bool over = false;
-    for (int k = 0; k < nr; ++k) {
-      bool seen = false;
-      for (uint32_t j = 0; j < nb; ++j) seen |= sel->bucket[j] == rb[k];
-      if (!seen) sel->bucket[nb++] = rb[k];
-    }
-    for (uint32_t i = 1; i < nb; ++i)  // insertion sort, nb <= kMaxRanks
-      for (uint32_t j = i; j > 0 && sel->bucket[j - 1] > sel->bucket[j]; --j) {
-        const uint32_t tmp = sel->bucket[j];
-        sel->bucket[j] = sel->bucket[j - 1];
-        sel->bucket[j - 1] = tmp;
-      }
-    for (uint32_t j = 0; j < nb; ++j) {
-      const uint32_t c = a.hist[sel->bucket[j]];
-      sel->base[j] = m;
-      sel->count[j] = c;
-      sel->fill[j] = 0u;
-      over |= (uint64_t)m + c > (uint64_t)kMaxCand;
-      m += over ? 0u : c;
-    }
-    for (int k = 0; k < nr; ++k)
-      for (uint32_t j = 0; j < nb; ++j)
-        if (sel->bucket[j] == rb[k]) sel->pos[k] = sel->base[j] + (uint32_t)rl[k];
-    sel->nb = nb;
-    sel->m = m;
-    sel->status = over ? kRadix : kSelect;
-  }
-}
-
-__global__ __launch_bounds__(256) void qs_gather(QsArgs args, QsArray* arr) {
-  __shared__ uint32_t bk[kMaxRanks];
-  const double* __restrict__ x = args.x[blockIdx.y];
-  QsArray& a = arr[blockIdx.y];
-  Sel* sel = &a.sel;
-  if (sel->status != kSelect) return;  // the same for every thread
-  double lo, scale;
-  (void)grid_of(a, lo, scale);
-  const uint32_t nb = sel->nb;
-  if (threadIdx.x < nb) bk[threadIdx.x] = sel->bucket[threadIdx.x];
-  __syncthreads();
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < args.n; i += (uint64_t)gridDim.x * 256) {
-    const double v = x[i];
-    const uint32_t b = bucket_of(v, lo, scale);
-    for (uint32_t j = 0; j < nb; ++j)
-      if (b == bk[j]) {
-        const uint32_t slot = atomicAdd(&sel->fill[j], 1u);
-        a.cand[sel->base[j] + slot] = v;
-      }
-  }
 }
 
 // The interpolation of get_percentile_value on the order statistics s(lo), s(hi).
@@ -269,44 +189,185 @@ __device__ __forceinline__ double interp(double rank, uint64_t lo, uint64_t hi, 
   return slo * (1.0 - w) + shi * w;
 }
 
-// One workgroup per array: bitonic sort of the m <= kMaxCand gathered values
-// in LDS, then the percentiles; the status and values into res.
-__global__ __launch_bounds__(1024) void qs_finish(QsArgs args, const QsArray* arr, QsResult* res) {
-  __shared__ double v[kMaxCand];
-  const QsArray& a = arr[blockIdx.y];
-  const Sel& sel = a.sel;
-  QsResult& r = res[blockIdx.y];
+__global__ __launch_bounds__(kThreads) void qs_hist(QsArgs args, QsArray* arr, QsResult* res) {
+  __shared__ uint32_t h[kBuckets];
+  __shared__ uint64_t smin[16], smax[16];
+  const double* __restrict__ x = args.x[blockIdx.y];
+  QsArray& a = arr[blockIdx.y];
   const int t = threadIdx.x;
-  const uint32_t status = sel.status;
-  if (t == 0) r.status = status;
-  if (status == kEqual) {  // every order statistic is the minimum
-    if (t < args.np) r.out[t] = from_key(a.mm[0]);
-    return;
+  const Grid g = grid_of(a, smin, smax);
+  if (blockIdx.x == 0) {
+    QsResult& r = res[blockIdx.y];
+    if (t == 0) a.sel.status = r.status = g.status;
+    if (g.status == kEqual && t < args.np) r.out[t] = from_key(g.min_key);  // every order statistic is the minimum
   }
-  if (status != kSelect) return;  // the same for every thread
-  const uint32_t m = sel.m;
-  uint32_t len = 1;
-  while (len < m) len <<= 1;
-  for (uint32_t i = t; i < len; i += blockDim.x) v[i] = i < m ? a.cand[i] : INFINITY;
+  if (g.status != kSelect) return;  // the same for every workgroup
+  for (int b = t; b < kBuckets; b += kThreads) h[b] = 0u;
   __syncthreads();
+#pragma unroll 4
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + t; i < args.n; i += (uint64_t)gridDim.x * kThreads)
+    atomicAdd(&h[bucket_of(x[i], g)], 1u);
+  __syncthreads();
+  for (int b = t; b < kBuckets; b += kThreads)
+    if (h[b]) atomicAdd(&a.hist[b], h[b]);
+}
+
+// One workgroup per array: the buckets of the needed ranks; thread t scans
+// buckets kPer t .. + kPer - 1.
+__global__ __launch_bounds__(kThreads) void qs_select(QsArgs args, QsArray* arr, QsResult* res) {
+  constexpr int kPer = kBuckets / kThreads;
+  __shared__ uint32_t wsum[16];
+  // of rank k: its bucket, the rank inside it and the bucket's count
+  __shared__ uint32_t rb[kMaxRanks], rl[kMaxRanks], rc[kMaxRanks];
+  QsArray& a = arr[blockIdx.y];
+  Sel* const sel = &a.sel;
+  const int t = threadIdx.x;
+  if (sel->status != kSelect) return;
+  const int nr = 2 * args.np;
+  uint32_t c[kPer], sum = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    c[j] = a.hist[kPer * t + j];
+    sum += c[j];
+  }
+  uint32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o);
+    if ((t & 63) >= o) incl += y;
+  }
+  if ((t & 63) == 63) wsum[t >> 6] = incl;
+  __syncthreads();
+  uint32_t cum = incl - sum;
+  for (int w = 0; w < (t >> 6); ++w) cum += wsum[w];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    for (int k = 0; k < nr; ++k) {
+      if (args.ranks[k] >= cum && args.ranks[k] < (uint64_t)cum + c[j]) {
+        rb[k] = (uint32_t)(kPer * t + j);
+        rl[k] = (uint32_t)args.ranks[k] - cum;
+        rc[k] = c[j];
+      }
+    }
+    cum += c[j];
+  }
+  __syncthreads();
+  // thread k: its bucket's place among the distinct ones in increasing order,
+  // and the slots of the gathered values before it
+  if (t < nr) {
+    uint32_t nb = 0, m = 0, at = 0, base = 0;
+    bool first = true;  // no earlier rank has this bucket
+    for (int j = 0; j < nr; ++j) {
+      bool fj = true;
+      for (int i = 0; i < j; ++i) fj &= rb[i] != rb[j];
+      if (j == t) first = fj;
+      if (!fj) continue;
+      ++nb;
+      m = m + rc[j] < m ? 0xFFFFFFFFu : m + rc[j];
+      if (rb[j] < rb[t]) {
+        ++at;
+        base += rc[j];
+      }
+    }
+    if (first) {
+      sel->bucket[at] = rb[t];
+      sel->base[at] = base;
+      sel->fill[at] = 0u;
+    }
+    sel->pos[t] = base + rl[t];
+    if (t == 0) {
+      sel->nb = nb;
+      sel->m = m;
+      if (m > (uint32_t)kMaxCand) sel->status = res[blockIdx.y].status = kRadix;
+    }
+  }
+}
+
+// Sorts v[0..len) of a workgroup by key (len a power of two).
+__device__ void sort_keys(uint64_t* v, uint32_t len) {
   for (uint32_t size = 2; size <= len; size <<= 1)
     for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-      for (uint32_t i = t; i < len; i += blockDim.x) {
-        const uint32_t j = i ^ stride;
-        if (j > i) {
-          const bool up = (i & size) == 0;
-          const double x0 = v[i], x1 = v[j];
-          if ((x0 > x1) == up) {
-            v[i] = x1;
-            v[j] = x0;
-          }
+      for (uint32_t i = threadIdx.x; i < len / 2; i += kThreads) {
+        const uint32_t lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
+        const uint64_t x0 = v[lo], x1 = v[hi];
+        if ((x0 > x1) == ((lo & size) == 0)) {
+          v[lo] = x1;
+          v[hi] = x0;
         }
       }
       __syncthreads();
     }
+}
+
+__global__ __launch_bounds__(kThreads) void qs_gather(QsArgs args, QsArray* arr) {
+  __shared__ uint64_t smin[16], smax[16];
+  __shared__ uint32_t bk[kMaxRanks];
+  const double* __restrict__ x = args.x[blockIdx.y];
+  QsArray& a = arr[blockIdx.y];
+  Sel* const sel = &a.sel;
+  if (sel->status != kSelect) return;  // the same for every thread
+  const Grid g = grid_of(a, smin, smax);
+  const uint32_t nb = sel->nb;
+  const int t = threadIdx.x;
+  if (t < (int)nb) bk[t] = sel->bucket[t];
+  __syncthreads();
+#pragma unroll 4
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + t; i < args.n; i += (uint64_t)gridDim.x * kThreads) {
+    const double xi = x[i];
+    const uint32_t b = bucket_of(xi, g);
+    for (uint32_t j = 0; j < nb; ++j)
+      if (b == bk[j]) {
+        const uint32_t slot = atomicAdd(&sel->fill[j], 1u);
+        a.cand[sel->base[j] + slot] = xi;
+      }
+  }
+}
+
+// One workgroup per array: the gathered values sorted in LDS, the percentiles.
+__global__ __launch_bounds__(kThreads) void qs_finish(QsArgs args, const QsArray* arr, QsResult* res) {
+  __shared__ uint64_t v[kMaxCand];
+  const QsArray& a = arr[blockIdx.y];
+  const Sel* const sel = &a.sel;
+  const int t = threadIdx.x;
+  if (sel->status != kSelect) return;  // the same for every thread
+  const uint32_t m = sel->m;
+  uint32_t len = 1;
+  while (len < m) len <<= 1;
+  for (uint32_t i = t; i < len; i += kThreads) v[i] = i < m ? ord_key(a.cand[i]) : ~0ull;
+  __syncthreads();
+  sort_keys(v, len);
+  QsResult& r = res[blockIdx.y];
   if (t < args.np)
-    r.out[t] = interp(args.prank[t], args.ranks[2 * t], args.ranks[2 * t + 1], v[sel.pos[2 * t]],
-                      v[sel.pos[2 * t + 1]]);
+    r.out[t] = interp(args.prank[t], args.ranks[2 * t], args.ranks[2 * t + 1], from_key(v[sel->pos[2 * t]]),
+                      from_key(v[sel->pos[2 * t + 1]]));
+}
+
+// n <= kMaxCand: the whole array in one workgroup's LDS.
+__global__ __launch_bounds__(kThreads) void qs_small(QsArgs args, QsResult* res) {
+  __shared__ uint64_t v[kMaxCand];
+  const double* __restrict__ x = args.x[blockIdx.y];
+  QsResult& r = res[blockIdx.y];
+  const uint32_t n = (uint32_t)args.n;
+  const int t = threadIdx.x;
+  uint32_t len = 1;
+  while (len < n) len <<= 1;
+  bool nan = false;
+  for (uint32_t i = t; i < len; i += kThreads) {
+    const double xi = i < n ? x[i] : 0.0;
+    nan |= isnan(xi);
+    v[i] = i < n ? ord_key(xi) : ~0ull;
+  }
+  nan = __syncthreads_or(nan);
+  if (t == 0) r.status = nan ? kNan : kSelect;
+  if (nan) return;
+  sort_keys(v, len);
+  if (t < args.np) {
+    const double lo = from_key(v[0]);
+    r.out[t] = lo == from_key(v[n - 1])
+                   ? lo
+                   : interp(args.prank[t], args.ranks[2 * t], args.ranks[2 * t + 1], from_key(v[args.ranks[2 * t]]),
+                            from_key(v[args.ranks[2 * t + 1]]));
+  }
 }
 
 // ---- the fallback: MSB-first radix select on the keys of ord_key.  Pass L
@@ -401,6 +462,7 @@ hipError_t grow(void** p, size_t* have, size_t need) {
 
 QuantileScratch::~QuantileScratch() {
   if (small) (void)hipFree(small);
+  if (host) (void)hipHostFree(host);
 }
 
 int quantile_select(QuantileScratch& sc, const double* const* xs, int nx, uint64_t n, const double* p, int np,
@@ -408,12 +470,16 @@ int quantile_select(QuantileScratch& sc, const double* const* xs, int nx, uint64
   if (used_fallback) *used_fallback = false;
   if (nx < 1 || nx > kMaxArrays || np < 1 || np > kMaxPercentiles || n < 1 || n > 0x7FFFFFFFull)
     return JNE_ERR_INVALID_ARG;
-  const size_t res_off = ((size_t)kMaxArrays * sizeof(QsArray) + 255) & ~size_t(255);
-  const size_t radix_off = (res_off + kMaxArrays * sizeof(QsResult) + 255) & ~size_t(255);
+  const size_t radix_off = ((size_t)kMaxArrays * sizeof(QsArray) + 255) & ~size_t(255);
   hipError_t e = grow(&sc.small, &sc.small_bytes, radix_off + kMaxArrays * sizeof(Radix));
   if (e != hipSuccess) return JNE_ERR_HIP;
+  // the results: pinned host memory that the kernels write
+  if (!sc.host && hipHostMalloc(&sc.host, kMaxArrays * sizeof(QsResult), hipHostMallocDefault) != hipSuccess) {
+    sc.host = nullptr;
+    return JNE_ERR_HIP;
+  }
   QsArray* arr = static_cast<QsArray*>(sc.small);
-  QsResult* d_res = reinterpret_cast<QsResult*>(static_cast<char*>(sc.small) + res_off);
+  QsResult* const res = static_cast<QsResult*>(sc.host);
   Radix* radix = reinterpret_cast<Radix*>(static_cast<char*>(sc.small) + radix_off);
 
   // ranks of the needed order statistics (get_percentile_value's rank)
@@ -426,18 +492,16 @@ int quantile_select(QuantileScratch& sc, const double* const* xs, int nx, uint64
     args.ranks[2 * i] = (uint64_t)floor(args.prank[i]);
     args.ranks[2 * i + 1] = (uint64_t)ceil(args.prank[i]);
   }
-  const unsigned grid = (unsigned)std::min<uint64_t>(1024, (n + 255) / 256);
-  hipLaunchKernelGGL(qs_init, dim3(1, nx), dim3(256), 0, st, arr);
-  hipLaunchKernelGGL(qs_minmax, dim3(grid, nx), dim3(256), 0, st, args, arr);
-  hipLaunchKernelGGL(qs_hist, dim3(std::min(grid, 512u), nx), dim3(256), 0, st, args, arr);
-  hipLaunchKernelGGL(qs_select, dim3(1, nx), dim3(256), 0, st, args, arr);
-  hipLaunchKernelGGL(qs_gather, dim3(grid, nx), dim3(256), 0, st, args, arr);
-  hipLaunchKernelGGL(qs_finish, dim3(1, nx), dim3(1024), 0, st, args, arr, d_res);
-  QsResult res[kMaxArrays];
-  if ((e = hipGetLastError()) != hipSuccess ||
-      (e = hipMemcpyAsync(res, d_res, nx * sizeof(QsResult), hipMemcpyDeviceToHost, st)) != hipSuccess ||
-      (e = hipStreamSynchronize(st)) != hipSuccess)
-    return JNE_ERR_HIP;
+  if (n <= (uint64_t)kMaxCand) {
+    hipLaunchKernelGGL(qs_small, dim3(1, nx), dim3(kThreads), 0, st, args, res);
+  } else {
+    hipLaunchKernelGGL(qs_minmax, dim3(pass_groups(n, 4 * kThreads), nx), dim3(kThreads), 0, st, args, arr);
+    hipLaunchKernelGGL(qs_hist, dim3(pass_groups(n, 16 * kThreads), nx), dim3(kThreads), 0, st, args, arr, res);
+    hipLaunchKernelGGL(qs_select, dim3(1, nx), dim3(kThreads), 0, st, args, arr, res);
+    hipLaunchKernelGGL(qs_gather, dim3(pass_groups(n, 4 * kThreads), nx), dim3(kThreads), 0, st, args, arr);
+    hipLaunchKernelGGL(qs_finish, dim3(1, nx), dim3(kThreads), 0, st, args, arr, res);
+  }
+  if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess) return JNE_ERR_HIP;
   for (int a = 0; a < nx; ++a)
     if (res[a].status == kNan) return JNE_ERR_NUMERIC;
   for (int a = 0; a < nx; ++a) {
@@ -450,17 +514,15 @@ int quantile_select(QuantileScratch& sc, const double* const* xs, int nx, uint64
     QsArgs one = args;
     one.x[0] = xs[a];
     Radix* const rx = radix + a;
+    const unsigned grid = (unsigned)std::min<uint64_t>(512, (n + 255) / 256);
     hipLaunchKernelGGL(qs_radix_init, dim3(1), dim3(256), 0, st, one, rx);
     for (int level = 0; level < kDigits; ++level) {
-      hipLaunchKernelGGL(qs_radix_hist, dim3(std::min(grid, 512u)), dim3(256), 0, st, one, rx, level);
+      hipLaunchKernelGGL(qs_radix_hist, dim3(grid), dim3(256), 0, st, one, rx, level);
       hipLaunchKernelGGL(qs_radix_pick, dim3(1), dim3(256), 0, st, one, rx);
     }
-    hipLaunchKernelGGL(qs_radix_finish, dim3(1), dim3(64), 0, st, one, rx, d_res + a);
-    if ((e = hipGetLastError()) != hipSuccess ||
-        (e = hipMemcpyAsync(out + (size_t)a * np, d_res[a].out, np * sizeof(double), hipMemcpyDeviceToHost, st)) !=
-            hipSuccess ||
-        (e = hipStreamSynchronize(st)) != hipSuccess)
-      return JNE_ERR_HIP;
+    hipLaunchKernelGGL(qs_radix_finish, dim3(1), dim3(64), 0, st, one, rx, res + a);
+    if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess) return JNE_ERR_HIP;
+    memcpy(out + (size_t)a * np, res[a].out, np * sizeof(double));
   }
   return 0;
 }
