@@ -30,7 +30,8 @@
 // One wave per walk.  A segment runs in three phases: the wave draws its
 // normals into LDS rows (64 Philox calls per iteration; where a segment's
 // calls are not whole iterations, the last one's spare lanes draw the next
-// segment's first calls); a scan lays the c rows beside them (lane (i, p)
+// segment's first calls, and the calls are stored whole, for the scan to lay
+// the rows from them); a scan lays the c rows beside them (lane (i, p)
 // takes a block of steps of component i, sums it in FP64 for eps and writes
 // each c_t as the FP32 rounding of an FP64 running sum); then lane l feeds
 // row l%32 of X for 8 of every 16 steps (half l/32), read straight from its
@@ -120,8 +121,16 @@ struct MfmaShape {
   static constexpr int OVF = CARRY ? 64 - gcd_int(CALLS, 64) : 1;
   static constexpr int ZP = kSegSteps + 4;              // LDS pitch of one row (floats)
   static constexpr int NG = (D * D + 63) / 64;          // (i, j) grid entries per lane
-  static constexpr int SP = D <= 8 ? 8 : 4;             // scan lanes per component
-  static constexpr int BS = kSegSteps / SP;             // steps per scan lane: whole 16-byte units
+  // scan: SP lanes per component, BS steps each (the last BL): as many lanes as
+  // the wave has for D components, up to 8 (a lane's offset takes SP - 1
+  // additions, so more lanes of fewer steps gain nothing).  Against four lanes
+  // of 16 steps, 100,000 walks at T = 10,000: dim 9 14.0 to 13.4 ms, dim 10
+  // 14.5 to 14.1, dim 11 15.3 to 15.2; five lanes of 13 steps at dim 12 gain
+  // nothing over four whose steps are whole 16-byte units (15.5 and 15.5 ms).
+  static constexpr int BS = D == 12 ? 16 : 64 / D < 8 ? (kSegSteps + 64 / D - 1) / (64 / D) : kSegSteps / 8;
+  static constexpr int SP = (kSegSteps + BS - 1) / BS;
+  static constexpr int BL = kSegSteps - (SP - 1) * BS;
+  static_assert(SP * D <= 64 && BL >= 1 && BL <= BS, "the scan lanes cover a segment");
   // LDS rows, each at its row index of X: z (0..D-1), c (12..12+D-1), 1, k,
   // k(k-1)/2 (24..26); the compact FP64 Gram takes the same bytes after the
   // last segment
@@ -404,18 +413,29 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   float(*const zbuf)[ZP] = xs;
   float(*const cbuf)[ZP] = xs + kRowC;
   double* const gram = reinterpret_cast<double*>(rows_raw);
-  __shared__ double eps_part[SP][D];
+  // sums of the scan blocks, block p of component i at [SP - 1 + p][i]: the SP - 1
+  // rows before a lane's own are those of the blocks before it and zeros
+  __shared__ __align__(16) double vecs[(2 * SP + 10) * D];  // one array: no padding between its parts
+  double(*const eps_part)[D] = reinterpret_cast<double(*)[D]>(vecs);
   // (not with the three-way bf16 split, whose operands leave no registers for it)
   constexpr bool kCarry = Sh::CARRY && !FROM_NORMALS && PREC != JNE_PREC_MFMA_BF16X3 && PREC != JNE_PREC_FP32_KAHAN;
   __shared__ float4 ovf[kCarry ? Sh::OVF : 1];  // calls drawn ahead for the next segment
-  __shared__ double seg_eps[D];
-  __shared__ double b0s[D];  // B at the segment start (FP64)
+  // the segment's calls in the order drawn (step-major: component i of step t at
+  // t D + i), in the c rows' bytes until the scan lays the z rows from it: one
+  // 16-byte store per call, where a call's four rows and steps, which change
+  // from call to call at these dims, took 112 of its 590 issue cycles (100,000
+  // walks at T = 10,000, dim 9: 14.7 to 14.0 ms)
+  static_assert(!kCarry || Sh::CALLS * 4 <= D * ZP, "a segment's calls fit the c rows");
+  float4* const zcall = reinterpret_cast<float4*>(&xs[kRowC][0]);
+  double* const seg_eps = vecs + (2 * SP - 1) * D;
+  double* const b0s = seg_eps + D;  // B at the segment start (FP64)
   // per component j of a segment: b = B0 + s m (the state the centred c rows
   // are relative to), P = n b + s sig, Q = s sig, E = s eps, so that the
   // segment adds b_i P_j + Q_i b_j to sum b b^T and E_i b_j to sum e b^T
   __shared__ SegVec seg[D];
-  __shared__ double mb[3 * D];   // sum over segments of B0' sum_seg u^p (lanes l < 3D)
-  __shared__ double gd[2 * D][3];  // Gram rows 24..26 of the c columns, then of the z columns
+  double* const mb = b0s + D;  // 3 D: sum over segments of B0' sum_seg u^p (lanes l < 3D)
+  // 2 D: Gram rows 24..26 of the c columns, then of the z columns
+  double(*const gd)[3] = reinterpret_cast<double(*)[3]>(mb + 3 * D);
   // the compensated check's per-segment Gram entries, [X row][X column]
   __shared__ double gk[kKahan ? kRowDet + 3 : 1][kKahan ? KS::COLS : 1];
 
@@ -503,6 +523,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   const int si = l % D, sp = l / D;
   const bool scan_lane = l < SP * D;
 
+  for (int e = l; e < (SP - 1) * D; e += 64) eps_part[e / D][e % D] = 0.0;
   if (l < D) b0s[l] = 0.0;
   if (l < 3 * D) mb[l] = 0.0;
   // walk constants: uniform, held in scalar registers
@@ -526,38 +547,18 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
     if constexpr (kCarry) {
       // calls [r CALLS, drawn) came with the previous segment's last iteration
       const int pending = (int)(drawn - r * (uint32_t)Sh::CALLS);
-      if (l < pending) {
-        const float4 q = ovf[l];
-        const float qv[4] = {q.x, q.y, q.z, q.w};
-        const CallPos<D> p(l);
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          int tl, i;
-          p.at(jj, tl, i);
-          zbuf[i][tl] = (!tail || ts + tl < T) ? qv[jj] : 0.0f;
-        }
-      }
+      if (l < pending) zcall[l] = ovf[l];
       // the rest, 64 calls per iteration; calls past the segment (spare lanes
       // of the last iteration) wait in ovf for the next one
       const uint32_t need = (r + 1) * (uint32_t)Sh::CALLS - drawn;
       const int nit = (int)((need + 63) / 64);
       int c = pending + l;  // this lane's call, counted from the segment's first
-      CallPos<D> pos(c);
       for (int j = 0; j < nit; ++j) {
         float v[4];
         normals4(drawn + 64u * j + l, seed, rng_stream, v);  // 32-bit counter (kMaxSteps)
-        if (c < Sh::CALLS) {
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            int tl, i;
-            pos.at(jj, tl, i);
-            zbuf[i][tl] = (!tail || ts + tl < T) ? v[jj] : 0.0f;
-          }
-        } else if (!tail) {
-          ovf[c - Sh::CALLS] = make_float4(v[0], v[1], v[2], v[3]);
-        }
+        float4* const dst = c < Sh::CALLS ? zcall + c : ovf + (c - Sh::CALLS);
+        *dst = make_float4(v[0], v[1], v[2], v[3]);
         c += 64;
-        pos.template advance<64>();
       }
       drawn += 64u * (uint32_t)nit;
     } else if constexpr (W > 1) {
@@ -614,23 +615,32 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
     // ---- scan, part 1: lane (si, sp) sums its block of component si in FP64:
     // the partial sums give the segment's eps, which drives the FP64 state,
     // and the offsets of the c rows in the blocks after it
-    // (128-bit LDS reads and writes: the 8 lanes of a read group cover
-    // distinct banks)
+    const auto block = [&](auto step) {  // step(j) for the steps sp BS + j of the lane's block
+#pragma unroll
+      for (int j = 0; j < Sh::BL; ++j) step(j);
+      if constexpr (Sh::BL < BS) {
+        if (sp < SP - 1) {
+#pragma unroll
+          for (int j = Sh::BL; j < BS; ++j) step(j);
+        }
+      }
+    };
     float zb[BS];
     if (scan_lane) {
-      const float4* const src = reinterpret_cast<const float4*>(&zbuf[si][sp * BS]);
-#pragma unroll
-      for (int q = 0; q < BS / 4; ++q) {
-        const float4 v = src[q];
-        zb[4 * q] = v.x;
-        zb[4 * q + 1] = v.y;
-        zb[4 * q + 2] = v.z;
-        zb[4 * q + 3] = v.w;
-      }
-      double e = (double)zb[0];  // (no 0.0 + first term: one add fewer)
-#pragma unroll
-      for (int j = 1; j < BS; ++j) e += (double)zb[j];
-      eps_part[sp][si] = e;
+      float* const zrow = &zbuf[si][sp * BS];
+      const float* const drawn_z = reinterpret_cast<const float*>(zcall) + sp * (BS * D) + si;
+      double e = 0.0;
+      block([&](int j) {
+        if constexpr (kCarry) {
+          const float z = drawn_z[j * D];
+          zb[j] = (!tail || ts + (uint32_t)(sp * BS + j) < T) ? z : 0.0f;
+          zrow[j] = zb[j];
+        } else {
+          zb[j] = zrow[j];
+        }
+        e = j ? e + (double)zb[j] : (double)zb[j];  // (no 0.0 + first term: one add fewer)
+      });
+      eps_part[SP - 1 + sp][si] = e;
     }
     __syncthreads();
 
@@ -639,28 +649,21 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
     // square, so the FP32 accumulation rounds less, and b_t = (B0 + s m) + s c_t.
     // Steps at or beyond T get c = 0 (their z are 0), so they add nothing.
     if (scan_lane) {
-      double e = eps_part[0][si];
+      double e = eps_part[SP - 1][si];
 #pragma unroll
-      for (int p = 1; p < SP; ++p) e += eps_part[p][si];
+      for (int p = 1; p < SP; ++p) e += eps_part[SP - 1 + p][si];
       float m;
       const double bm = seg_state(SPLIT ? 0.0 : b0s[si], s, e, m);
       // running sum in FP64 (exact but for FP64 rounding): each c_t is then
       // rounded to FP32 once
       double c = -(double)m;
 #pragma unroll
-      for (int p = 0; p < SP - 1; ++p) c += p < sp ? eps_part[p][si] : 0.0;
-      float4* const dst = reinterpret_cast<float4*>(&cbuf[si][sp * BS]);
-#pragma unroll
-      for (int q = 0; q < BS / 4; ++q) {
-        float cq[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t t = ts + (uint32_t)(sp * BS + 4 * q + k);
-          cq[k] = (!tail || t < T) ? (float)c : 0.0f;
-          c += (double)zb[4 * q + k];
-        }
-        dst[q] = make_float4(cq[0], cq[1], cq[2], cq[3]);
-      }
+      for (int p = 0; p < SP - 1; ++p) c += eps_part[sp + p][si];
+      float* const crow = &cbuf[si][sp * BS];
+      block([&](int j) {
+        crow[j] = (!tail || ts + (uint32_t)(sp * BS + j) < T) ? (float)c : 0.0f;
+        c += (double)zb[j];
+      });
       if (sp == 0) {
         seg_eps[si] = e;
         if constexpr (!SPLIT) {
