@@ -70,6 +70,19 @@ struct BoolTag {
   static constexpr bool value = B;
 };
 
+// Workgroups are dealt to the 8 XCDs round-robin by index, and each XCD has
+// its own L2.  With one walk per workgroup, walks b and b+1 would run on
+// different XCDs: their 8-byte stores into one sector of an entry-major array
+// would reach HBM as separate partial writes, and their loads would fetch every
+// line once per XCD.  This bijection gives XCD x the contiguous walk range
+// [start_x, start_x + count_x) instead, so neighbouring walks share an L2.
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t xcd_walk(uint32_t b, uint32_t n) {
+  const uint32_t q = n / kXcds, r = n % kXcds;
+  const uint32_t x = b % kXcds, i = b / kXcds;
+  return x * q + (x < r ? x : r) + i;
+}
+
 template <int N>
 struct IntTag {
   static constexpr int value = N;

@@ -21,6 +21,8 @@
 // ulp of the matrix norm.
 #pragma once
 
+#include <math.h>
+
 #if defined(__HIPCC__)
 #define JNE_TRI_HD __device__ __forceinline__
 #else
@@ -30,6 +32,17 @@
 namespace jne {
 
 constexpr int kQlMaxIter = 30;
+
+// High word of a double (its sign, exponent and leading bits).
+JNE_TRI_HD int tri_hi(double x) {
+#if defined(__HIPCC__)
+  return __double2hiint(x);
+#else
+  long long b;
+  __builtin_memcpy(&b, &x, sizeof b);
+  return (int)(b >> 32);
+#endif
+}
 
 // Packed upper triangle of an N x N symmetric matrix: a[tri_idx<N>(i, j)].
 template <int N>
@@ -180,20 +193,56 @@ JNE_TRI_HD void sturm_bounds(const double* d, const double* e2, int n, double& l
   hi = h + pad + 2.0 * pivmin;
 }
 
-// Number of eigenvalues of T below x.  Math::rcp(x) is 1/x to a few ulp.
-template <int NMAX, class Math>
-JNE_TRI_HD int sturm_count(const double* d, const double* e2, int n, double x, double pivmin) {
-  double q = d[0] - x;
-  bool neg = q <= pivmin;
-  int c = neg ? 1 : 0;
-  q = neg ? fmin(q, -pivmin) : q;
+// T scaled by a power of two s (returned) to |T| <= 1, its interval with it, for
+// sturm_count: squared off-diagonals below 2^-160 are raised to that, which moves
+// an eigenvalue by at most 2^-79 |T|, so that a zero term of the sequence is
+// followed by one that is not; the padding past n gets positive diagonal entries
+// of its own, which change no sign.
+template <int NMAX>
+JNE_TRI_HD double sturm_scale(double* d, double* e2, int n, double& lo, double& hi) {
+  const double tn = fmax(fabs(lo), fabs(hi));
+  int ex = 0;
+  if (tn > 0.0 && tn <= 0x1.fffffffffffffp+1023) (void)::frexp(tn, &ex);
+  const double s = ::ldexp(1.0, ex < -1022 ? 1022 : -ex);
 #pragma unroll
-  for (int i = 1; i < NMAX; ++i) {
-    if (i < n) {
-      q = fma(-e2[i - 1], Math::rcp(q), d[i] - x);
-      neg = q <= pivmin;
-      c += neg ? 1 : 0;
-      q = neg ? fmin(q, -pivmin) : q;
+  for (int i = 0; i < NMAX; ++i) {
+    d[i] = i < n ? d[i] * s : 4.0;
+    e2[i] = i + 1 < n ? fmax((e2[i] * s) * s, 0x1p-160) : 0.0;
+  }
+  lo *= s;
+  hi *= s;
+  return s;
+}
+
+// Number of eigenvalues of the scaled T below x: the sign changes of the
+// leading minors of T - x, p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, which
+// take three FP64 operations each where the ratios p_i / p_{i-1} take a
+// reciprocal (the same backward error, a few ulp of |T|).  A term grows at most
+// 5-fold, and two terms shrink at most 2^-201-fold, so eight steps from a pair of
+// size one neither overflow nor underflow.
+template <int NMAX>
+JNE_TRI_HD int sturm_count(const double* d, const double* e2, int n, double x) {
+  double p0 = 1.0, p1 = d[0] - x;
+  int h1 = tri_hi(p1);
+  int c = -(h1 >> 31);
+#pragma unroll
+  for (int b = 0; b < NMAX; b += 8) {
+    if (b < n) {
+#pragma unroll
+      for (int i = b > 0 ? b : 1; i < b + 8 && i < NMAX; ++i) {
+        const double p = fma(d[i] - x, p1, -(e2[i - 1] * p0));
+        const int h = tri_hi(p);
+        c -= (h ^ h1) >> 31;
+        h1 = h;
+        p0 = p1;
+        p1 = p;
+      }
+      if (b + 8 < NMAX) {
+        int ex;
+        (void)::frexp(fmax(fabs(p0), fabs(p1)), &ex);
+        p0 = ::ldexp(p0, -ex);
+        p1 = ::ldexp(p1, -ex);
+      }
     }
   }
   return c;
@@ -205,16 +254,22 @@ JNE_TRI_HD int sturm_count(const double* d, const double* e2, int n, double x, d
 // From the Gershgorin interval (width <= 2 |T|), 54 halvings leave a width of
 // at most 2^-53 |T|.
 template <int NMAX, class Math>
-JNE_TRI_HD double sturm_eigval(const double* d, const double* e2, int n, int k, double lo, double hi, double pivmin,
-                               int iters) {
+JNE_TRI_HD double sturm_eigval(const double* d_in, const double* e2_in, int n, int k, double lo, double hi,
+                               double /*pivmin*/, int iters) {
+  double d[NMAX], e2[NMAX];
+  for (int i = 0; i < NMAX; ++i) {
+    d[i] = i < n ? d_in[i] : 0.0;
+    e2[i] = i + 1 < n ? e2_in[i] : 0.0;
+  }
+  const double s = sturm_scale<NMAX>(d, e2, n, lo, hi);
   for (int it = 0; it < iters; ++it) {
     const double mid = 0.5 * (lo + hi);
-    if (sturm_count<NMAX, Math>(d, e2, n, mid, pivmin) > k)
+    if (sturm_count<NMAX>(d, e2, n, mid) > k)
       hi = mid;
     else
       lo = mid;
   }
-  return 0.5 * (lo + hi);
+  return 0.5 * (lo + hi) / s;
 }
 
 constexpr int kBisectIters = 54;

@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64) void walk_moments_fp64_wave(const uint32_t* __r
   constexpr int C = R * D / 4;  // Philox calls per round
   __shared__ __align__(16) double zs[R * D], cs[R * D];  // t-major
   const int l = threadIdx.x;
-  const size_t walk = blockIdx.x;
+  const size_t walk = xcd_walk(blockIdx.x, gridDim.x);
   uint32_t seed = 0;
   if constexpr (!FROM_NORMALS) seed = seeds[walk];
   const double* zw = FROM_NORMALS ? zin + walk * (size_t)T * D : nullptr;

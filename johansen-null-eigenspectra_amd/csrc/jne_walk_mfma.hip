@@ -328,19 +328,6 @@ struct CallUnroll {
                                    : 1;
 };
 
-// Workgroups are dealt to the 8 XCDs round-robin by index, and each XCD has
-// its own L2.  With one walk per workgroup, walks b and b+1 would run on
-// different XCDs and their 8-byte stores into one 32-byte sector of the
-// entry-major output would reach HBM as separate partial-sector writes.  This
-// bijection gives XCD x the contiguous walk range [start_x, start_x + count_x)
-// instead, so neighbouring walks share an L2 and their stores merge there.
-constexpr uint32_t kXcds = 8;
-__device__ __forceinline__ uint32_t xcd_walk(uint32_t b, uint32_t n) {
-  const uint32_t q = n / kXcds, r = n % kXcds;
-  const uint32_t x = b % kXcds, i = b / kXcds;
-  return x * q + (x < r ? x : r) + i;
-}
-
 // The per-segment FP64 terms, shared by the kernel that takes a walk's segments
 // in turn and the one that adds them up from memory (mfma_segments_add), so that
 // both perform the same operations.

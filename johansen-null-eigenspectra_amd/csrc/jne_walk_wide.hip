@@ -111,8 +111,8 @@ void walk_moments_wide(const uint32_t* __restrict__ seeds, const double* __restr
   extern __shared__ double wide_x[];  // X[tile][step][16], R steps (wide_moments_lds_bytes)
   __shared__ double qv[16 * NT], bv[16 * NT], sv[32], a1v[32], a2v[32];
   const int l = threadIdx.x;
-  const size_t walk = blockIdx.x;
-  if (walk >= n_walks) return;  // whole wave exits together
+  if (blockIdx.x >= n_walks) return;  // whole wave exits together
+  const size_t walk = xcd_walk(blockIdx.x, n_walks);
   const int R = wide_round_steps(D);
   const int calls = R * D / 4;
   uint32_t seed = 0;
@@ -373,19 +373,6 @@ __global__ __launch_bounds__(256) void wide_blocks_add(int D, uint32_t T, uint32
   if (j0 == 0) store_vector_moments(sc, m0, m1, m2, bk, o, D, k, ld, 0);
 }
 
-namespace {
-
-__device__ __forceinline__ double rcp_nr_w(double x) {
-  const double r = __builtin_amdgcn_rcp(x);
-  return fma(r, fma(-x, r, 1.0), r);
-}
-
-struct WideMath {
-  static __device__ __forceinline__ double rcp(double x) { return rcp_nr_w(x); }
-};
-
-}  // namespace
-
 // A row-major matrix in LDS with a runtime pitch: m[i][j].
 struct LdsMat {
   double* p;
@@ -393,42 +380,67 @@ struct LdsMat {
   __device__ __forceinline__ double* operator[](int i) const { return p + i * pitch; }
 };
 
-// LDS bytes of walk_eigen_wide for (model, dim): L (NX x (NX + 1)), W (NX x
-// (D + 1)) and P0, P1 (NX each), NX = D + 1 for models 1 and 3, else D.
+// LDS bytes of walk_eigen_wide for (model, dim): S11 (NX x (NX + 1)), S10 (NX x
+// (D + 1)), P0, P1 (NX each) and the vector moments (6 D), NX = D + 1 for models
+// 1 and 3, else D.
 size_t wide_eigen_lds_bytes(int model, int D) {
   const size_t nx = (model == 1 || model == 3) ? (size_t)D + 1 : (size_t)D;
-  return sizeof(double) * (nx * (nx + 1) + nx * ((size_t)D + 1) + 2 * nx);
+  return sizeof(double) * (nx * (nx + 1) + nx * ((size_t)D + 1) + 2 * nx + 6 * (size_t)D);
+}
+
+// Lane `from`'s value of x (from is wave-uniform).
+__device__ __forceinline__ double lane_f64(double x, int from) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), from),
+                          __builtin_amdgcn_readlane(__double2loint(x), from));
 }
 
 // One wave per walk: the model algebra of walk_eigen_fp64 (F = X - P Z with
 // P = (sum X Z^T)(sum Z Z^T)^-1 on the projected rows; models 0..4 as in
 // construct_f_matrix, src/johansen_statistics.rs:102-197), then the
 // generalized eigenproblem of src/johansen_statistics.rs:24-47 as the
-// symmetric one of M = W^T W, W = L^-1 S10, S11 = L L^T.
+// symmetric one of M = W^T W, W = L^-1 S10, S11 = L L^T.  16,384 walks at dims
+// 16, 24 and 32: 0.38, 0.77 and 1.47 ms with the walks dealt over the XCDs, the
+// algebra in LDS and ratio counts; now 0.28, 0.55 and 1.01 ms.
 template <int DP>
 __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const double* __restrict__ acc, size_t ld,
                                                       uint32_t T, uint32_t n_walks, double* __restrict__ out) {
   // LDS sized by the launch for this (model, dim) (wide_eigen_lds_bytes):
-  // S11 and then its Cholesky factor L (NX x NX, pitch NX + 1); S10 and then
-  // W (NX x D, pitch D + 1); the projections P0, P1.  Once W is formed the
-  // bytes of L hold M (D x D, pitch D + 1), which needs only W.
-  extern __shared__ double wide_lds[];
+  // sum b b^T and from it S11 (NX x NX, pitch NX + 1); sum e b^T and from it S10
+  // (NX x D, pitch D + 1); the projections P0, P1; the vector moments.  Once the
+  // rows of S11 and S10 are in registers, M (D x D, pitch D + 1) takes the
+  // bytes of S11 and the broadcast vectors those of S10.
+  extern __shared__ __align__(16) double wide_lds[];
   const int NX = (model == 1 || model == 3) ? D + 1 : D;
   const LdsMat Ls{wide_lds, NX + 1};
   const LdsMat Ws{wide_lds + NX * (NX + 1), D + 1};
   const LdsMat Ms{wide_lds, D + 1};
   double* const P0 = wide_lds + NX * (NX + 1) + NX * (D + 1);
   double* const P1 = P0 + NX;
+  double* const V = P1 + NX;
   const int l = threadIdx.x;
-  const size_t walk = blockIdx.x;
-  if (walk >= n_walks) return;
+  if (blockIdx.x >= n_walks) return;
+  const size_t walk = xcd_walk(blockIdx.x, n_walks);
   const int NB = (model == 2 || model == 4) ? D - 1 : D;
   const int NZ = model == 4 ? 2 : ((model == 2 || model == 3) ? 1 : 0);
   auto A = [&](int e) -> double { return acc[(size_t)e * ld + walk]; };
-  auto GBB = [&](int i, int j) { return A(i * D + j); };
-  auto GEB = [&](int k, int j) { return A(D * D + k * D + j); };
-  auto MB = [&](int p, int i) { return A(2 * D * D + p * D + i); };
-  auto ME = [&](int p, int k) { return A(2 * D * D + (3 + p) * D + k); };
+  // the walk's moments to LDS, many loads in flight (one after the other, as the
+  // algebra asks for them, they took 23 us of a walk's latency at dim 32)
+  const int hr = l >> 5, lc = l & 31;  // row (of two at a time) and column of this lane
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    if (l + 64 * q < 6 * D) V[l + 64 * q] = A(2 * D * D + l + 64 * q);
+  if (lc < D) {
+#pragma unroll 8
+    for (int i = hr; i < D; i += 2) {
+      Ws[lc][i] = A(D * D + i * D + lc);
+      if (lc <= i) Ls[i][lc] = A(i * D + lc);
+    }
+  }
+  __syncthreads();
+  auto GBB = [&](int i, int j) { return Ls[i][j]; };  // j <= i
+  auto GEB = [&](int k, int j) { return Ws[j][k]; };
+  auto MB = [&](int p, int i) { return V[p * D + i]; };
+  auto ME = [&](int p, int k) { return V[(3 + p) * D + k]; };
 
   const double Tn = (double)T;
   const double dt = 1.0 / Tn;
@@ -490,64 +502,78 @@ __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const do
     return 0.0;
   };
   // S11 (lower triangle) and S10 = S01raw^T: S01raw = eX - eZ ZZ^-1 ZX
-  for (int e = l; e < NX * NX; e += 64) {
-    const int i = e / NX, j = e - (e / NX) * NX;
-    if (j <= i) Ls[i][j] = (XX(i, j) - proj(i, j)) * dt;
-  }
-  for (int e = l; e < NX * D; e += 64) {
-    const int i = e / D, k = e - (e / D) * D;
-    double v = EX(k, i);
-    if (NZ > 0 && projected(i)) v -= NZ == 2 ? P0[i] * ME(0, k) + P1[i] * ME(1, k) : P0[i] * ME(0, k);
-    Ws[i][k] = v;
+  for (int i = hr; i < NX; i += 2) {
+    if (lc <= i) Ls[i][lc] = (XX(i, lc) - proj(i, lc)) * dt;
+    if (i == 32 && lc == 0) Ls[32][32] = (XX(32, 32) - proj(32, 32)) * dt;
+    if (lc < D) {
+      double v = EX(lc, i);
+      if (NZ > 0 && projected(i)) v -= NZ == 2 ? P0[i] * ME(0, lc) + P1[i] * ME(1, lc) : P0[i] * ME(0, lc);
+      Ws[i][lc] = v;
+    }
   }
   __syncthreads();
 
-  // Cholesky S11 = L L^T, one column at a time: every lane forms the pivot
-  // (the same value), lanes below it their entry of the column.  The
-  // reciprocal pivots go to P0's bytes (P0 and P1 are not read again) for the
-  // substitution below.
-  double* const dinv = P0;
+  // S11 = L L^T, W = L^-1 S10 and M = W^T W in one pass over L's columns: lane i
+  // < NX keeps row i of S11 (a, from the current column on) and of S10 (b), lane
+  // 63 - k row k of M (b).  Step j: lane j's pivot gives L_jj and W_j = S10_j /
+  // L_jj; the column L_ij and W_j are broadcast through LDS; then
+  //   S11_ik -= L_ij L_kj,   S10_i -= L_ij W_j,   M_k += W_j[k] W_j,
+  // the last two one FMA of every lane.  At dim 32 with NX = 33 the last row of
+  // S10 takes the lane of the last row of M: that row is the others' last
+  // column, its diagonal entry summed by every lane.  Bound by the LDS reads of
+  // the broadcasts (33 of 16 bytes per lane and step at dim 32).  In LDS, one
+  // triangular loop after the other, the three took 50 us of a walk's latency at
+  // dim 32 and now take 33; with the loads above, 16,384 walks 0.72 to 0.63 ms.
   bool pd = true;
-  for (int j = 0; j < NX; ++j) {
-    double s = Ls[j][j];
-    for (int k = 0; k < j; ++k) s -= Ls[j][k] * Ls[j][k];
-    pd = pd && (s > 0.0);
-    const double ljj = sqrt(s > 0.0 ? s : 1.0);
-    const double inv = 1.0 / ljj;
-    const int i = j + 1 + l;
-    double v = 0.0;
-    if (i < NX) {
-      v = Ls[i][j];
-      for (int k = 0; k < j; ++k) v -= Ls[i][k] * Ls[j][k];
+  {
+    double a[DP + 1], b[DP];
+    const int lr = l < NX ? l : 0;
+#pragma unroll
+    for (int m = 0; m <= DP; ++m) {
+      const double x = Ls[lr][m < NX ? m : 0];
+      a[m] = l < NX && m <= l ? x : 0.0;
+    }
+#pragma unroll
+    for (int m = 0; m < DP; ++m) {
+      const double x = Ws[lr][m < D ? m : 0];
+      b[m] = l < NX && m < D ? x : 0.0;
     }
     __syncthreads();
-    if (l == 0) {
-      Ls[j][j] = ljj;
-      dinv[j] = inv;
+    double* const Wj = wide_lds + NX * (NX + 1);  // W_j, DP entries
+    double* const Lj = Wj + DP;                      // column j from the diagonal on, 64 entries
+    const bool last = D + NX > 64;                   // a row of M has no lane
+    const int mk = 63 - l;                           // this lane's row of M
+    const bool m_lane = l >= NX && mk < D;
+    double dlast = 0.0;
+    for (int j = 0; j < NX; ++j) {
+      const double s = lane_f64(a[0], j);
+      pd = pd && (s > 0.0);
+      const double ljj = sqrt(s > 0.0 ? s : 1.0);
+      const double inv = 1.0 / ljj;
+      const double lij = l > j && l < NX ? a[0] * inv : 0.0;
+      if (l >= j) Lj[l - j] = lij;
+      if (l == j) {
+#pragma unroll
+        for (int m = 0; m < DP; ++m) Wj[m] = b[m] * inv;
+      }
+      __syncthreads();
+      const double cb = l < NX ? -lij : (m_lane ? Wj[m_lane ? mk : 0] : 0.0);
+      if (last) dlast = fma(Wj[D - 1], Wj[D - 1], dlast);
+#pragma unroll
+      for (int m = 0; m < DP; ++m) b[m] = fma(cb, Wj[m], b[m]);
+#pragma unroll
+      for (int m = 1; m <= DP; ++m) a[m - 1] = fma(-lij, Lj[m], a[m]);
+      __syncthreads();  // every lane has read the column before the next step writes its own
     }
-    if (i < NX) Ls[i][j] = v * inv;
+    if (m_lane) {
+#pragma unroll
+      for (int m = 0; m < DP; ++m)
+        if (m < D) Ms[mk][m] = b[m];
+      if (last) Ms[D - 1][mk] = b[DP - 1];  // D = DP = 32
+    }
+    if (last && l == 0) Ms[D - 1][D - 1] = dlast;
     __syncthreads();
   }
-
-  // W = L^-1 S10: lane k solves column k by forward substitution, in place
-  if (l < D) {
-    for (int i = 0; i < NX; ++i) {
-      double v = Ws[i][l];
-      for (int j = 0; j < i; ++j) v -= Ls[i][j] * Ws[j][l];
-      Ws[i][l] = v * dinv[i];
-    }
-  }
-  __syncthreads();
-  // M = W^T W (D x D, symmetric: both triangles)
-  for (int e = l; e < D * D; e += 64) {
-    const int k = e / D, m = e - (e / D) * D;
-    if (m < k) continue;
-    double v = 0.0;
-    for (int i = 0; i < NX; ++i) v = fma(Ws[i][k], Ws[i][m], v);
-    Ms[k][m] = v;
-    Ms[m][k] = v;
-  }
-  __syncthreads();
 
   // ---- Householder reduction of M to tridiagonal form: lane i keeps row i
   // of M in registers (columns padded to DP with zeros).  Step k broadcasts
@@ -635,9 +661,12 @@ __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const do
   // ---- eigenvalue g (ascending) of the tridiagonal matrix by the P = 64 / D
   // lanes g, g + D, .., g + (P - 1) D: from the Gershgorin interval, each round
   // lane g + jD takes the Sturm count at the (j+1)-th of P equally spaced
-  // interior points, the counts meet in LDS, and every lane of the group keeps
-  // the sub-interval whose upper point is the first count past g: (P + 1)-fold
-  // per round, where bisection halves (P = 2 at D = 22..32, 4 at D <= 16).
+  // interior points, the counts meet in a ballot, and every lane of the group
+  // keeps the sub-interval whose upper point is the first count past g: (P + 1)-fold
+  // per round, where bisection halves (P = 2 at D = 22..32, 4 at D <= 16).  Bound
+  // by the counts' FP64 operations: with a reciprocal per term (16,384 walks at
+  // dim 32) the rounds took 0.56 ms, with the minors themselves 0.24; one walk at
+  // dim 32: 64 to 24 us.
   double dg[DP], e2[DP];
 #pragma unroll
   for (int j = 0; j < DP; ++j) {
@@ -647,36 +676,24 @@ __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const do
   }
   double lo, hi, pivmin;
   sturm_bounds<DP>(dg, e2, D, lo, hi, pivmin);
+  const double scale = sturm_scale<DP>(dg, e2, D, lo, hi);
   const int P = 64 / D;  // >= 2 (D <= 32)
   const int grp = l % D, jp = l / D;  // lanes with jp >= P follow their group
   const double inv_sections = 1.0 / (double)(P + 1);
   int rounds = 0;  // (P + 1)^rounds >= 2^54: at most the width 54 halvings leave
   for (double w = 1.0; w > 0x1p-54; w *= inv_sections) ++rounds;
-  int* const cnt = reinterpret_cast<int*>(Xs);  // 64 ints over Xs, Ps (not read again)
   for (int it = 0; it < rounds; ++it) {
     const double step = (hi - lo) * inv_sections;
-    int c = 0;
-    if (jp < P) c = sturm_count<DP, WideMath>(dg, e2, D, lo + (double)(jp + 1) * step, pivmin);
-    cnt[l] = c;
-    __syncthreads();
-    double nlo = lo, nhi = hi;
-    bool found = false;
-    for (int q = 0; q < P; ++q) {
-      const double xq = lo + (double)(q + 1) * step;
-      if (!found) {
-        if (cnt[grp + D * q] > grp) {
-          nhi = xq;
-          found = true;
-        } else {
-          nlo = xq;
-        }
-      }
-    }
-    lo = nlo;
-    hi = nhi;
-    __syncthreads();  // every lane has read the counts before the next round writes them
+    bool past = false;
+    if (jp < P) past = sturm_count<DP>(dg, e2, D, lo + (double)(jp + 1) * step) > grp;
+    const unsigned long long mask = __ballot(past) >> grp;  // bit q D: the group's point q
+    int first = P;
+#pragma unroll
+    for (int q = 64 / (DP - (DP > 16 ? 7 : 3)) - 1; q >= 0; --q) first = (mask >> (q * D)) & 1ull ? q : first;
+    if (first < P) hi = lo + (double)(first + 1) * step;
+    if (first > 0) lo = lo + (double)first * step;
   }
-  const double lam = 0.5 * (lo + hi);
+  const double lam = 0.5 * (lo + hi) / scale;
 
   // |lambda| sorted descending (rank of each by lane), NX - D structural zeros
   if (l < D) EVs[l] = fabs(lam);
@@ -690,7 +707,7 @@ __global__ __launch_bounds__(64) void walk_eigen_wide(int model, int D, const do
       const double x = EVs[j];
       rank += (x > ev || (x == ev && j < l)) ? 1 : 0;
     }
-    o[rank] = pd ? ev : nan;
+    o[pd ? rank : l] = pd ? ev : nan;
   }
   if (l == 0 && NX > D) o[D] = pd ? 0.0 : nan;
 }
