@@ -16,6 +16,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "jne_blocks.h"
@@ -1025,8 +1026,8 @@ __global__ __launch_bounds__(64) void walk_eigen_jacobi(const double* __restrict
 // The forms of a moment launch.  One lane group per walk fills the GPU (the
 // waves resident at the kernel's occupancy) in whole rounds only; the walks of
 // the last, partial round are split over their blocks, as are all walks of a
-// batch too small for one lane group each.  With units = walks x blocks of
-// kBlockUnit steps, the split walks get
+// batch too small for one lane group each.  With units = the walks' steps in
+// blocks of kBlockUnit, the split walks get
 //   one wave per block          up to kWaveForm units,
 //   one lane per component      up to kRowForm units (walk_moments_fp64, L = dim),
 //   the dim's own lane group    above.
@@ -1035,31 +1036,46 @@ __global__ __launch_bounds__(64) void walk_eigen_jacobi(const double* __restrict
 // 0.044, 8,000 0.065 / 0.048 / 0.075, 30,000 0.068 / 0.067 / 0.24; dim 7:
 // 2,000 0.156 / 0.049 / 0.048, 30,000 0.171 / 0.127 / 0.42, 60,000 0.183 /
 // 0.205 / 0.81; dim 12: 2,000 0.110 / 0.060 / 0.078, 16,000 0.128 / 0.155 /
-// 0.46.  A split walk also writes and reads its blocks' sums (4 to 30% of the
-// whole, more at the high dims and short blocks), so a rest of ROUND_FILL of a
-// round or more is not split.  100,000 walks at T = 2,000, in turn and split:
-// dim 1 0.232 and 0.171 ms, dim 5 1.52 and 1.22; 10,000 walks at T = 8,000:
-// dim 1 0.607 and 0.112, dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
+// 0.46.  10,000 walks at T = 8,000, in turn and split: dim 1 0.607 and 0.112 ms,
+// dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
 constexpr uint32_t kSimds = 1024;
 #ifndef JNE_WAVE_FORM
 #define JNE_WAVE_FORM 3500, 4000, 5000, 4000, 4500, 4500, 2000, 1500, 1500, 1500, 1500, 1000
 #endif
 constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
 #ifndef JNE_ROW_FORM
-#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 45000, 24000, 0, 14000, 13000, 12000
+#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 52000, 24000, 0, 14000, 13000, 12000
 #endif
 constexpr uint32_t kRowForm[12] = {JNE_ROW_FORM};
-#ifndef JNE_ROUND_FILL
-#define JNE_ROUND_FILL 90  // percent of a round
-#endif
+
+// Steps of m walks in blocks of 240.
+static uint64_t split_units(uint32_t T, uint32_t m) { return ((uint64_t)m * T + kBlockUnit - 1) / kBlockUnit; }
 
 // Walks of n whose blocks one lane group takes in turn (the rest are split).
+// Whole rounds of the GPU's waves are taken in turn, and a rest of 90% of one with
+// them.  For the others both times are estimated, in steps of a SIMD with two
+// waves (one wave alone reaches 0.84 of its rate): in turn, the deepest SIMD's
+// waves of T steps (less what starts while the rounds before end); split, the
+// rest's steps spread evenly, but no less than the deepest SIMD's whole blocks,
+// and the sums' way through memory with their launches (130 steps behind whole
+// rounds; else 40 of the short steps below dim 7, nothing that shows above).  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8
+// steps): 65,536 walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536
+// 0.179 and 0.207, 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593,
+// 170,000 1.324 and 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 12, T =
+// 1,000, 16,384 0.368 and 0.481, 50,001 1.226 and 1.378.
 static uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
-  const uint32_t L = lanes_for_dim(d);
-  const uint32_t round = (64 / L) * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
-  const uint32_t rest = n % round;
-  if (block_count(T) == 1) return n > std::max(kWaveForm[d - 1], kRowForm[d - 1]) ? n : 0;
-  return (uint64_t)rest * 100 >= (uint64_t)round * JNE_ROUND_FILL ? n : n - rest;
+  const uint32_t L = lanes_for_dim(d), wave = 64 / L;  // walks per wave
+  const uint32_t round = wave * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
+  const uint32_t rest = n % round, bn = block_steps(T), small = std::max(kWaveForm[d - 1], kRowForm[d - 1]);
+  if (block_count(T) == 1) return n > small ? n : 0;
+  if (split_units(T, rest) <= small) return n - rest;
+  if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
+  const auto deep = [](double w) { return w <= 1.0 ? 1.0 / 0.84 : std::ceil(w); };
+  const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
+  const bool first = rest == n;
+  const double in_turn = first ? t * deep(w) : t * (std::ceil(w) - 0.145);
+  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 0.0);
+  return split < in_turn ? n - rest : n;
 }
 
 size_t fp64_part_doubles(int d, uint32_t T, uint32_t n) {
@@ -1107,7 +1123,7 @@ static hipError_t launch_moments_d(const uint32_t* seeds, const double* zin, uin
   const uint32_t m = n - turns;
   const uint32_t* s = seeds ? seeds + turns : nullptr;
   const double* z = zin ? zin + (size_t)turns * T * D : nullptr;
-  const uint64_t units = (uint64_t)m * ((T + kBlockUnit - 1) / kBlockUnit);
+  const uint64_t units = split_units(T, m);
   if (units <= kWaveForm[D - 1])
     e = go(IntTag<0>{}, BoolTag<true>{}, s, z, m, part, m);
   else if (units <= kRowForm[D - 1])
