@@ -343,7 +343,12 @@ int run_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_t s
   // without room for the blocks' sums the launches are not split
   const size_t part = std::max(part_doubles_for(dim, steps, precision, chunk),
                                part_doubles_for(dim, steps, precision, n % chunk));
-  if (ensure(ctx, (void**)&ctx->d_part, &ctx->part_bytes, part * sizeof(double)) != JNE_OK) {
+  // A captured call is not split: a smaller batch can need more room than a larger
+  // one did, so a later call may replace the block sums' buffer under the graph.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  if (!captured && ensure(ctx, (void**)&ctx->d_part, &ctx->part_bytes, part * sizeof(double)) != JNE_OK) {
     (void)hipGetLastError();
     ctx->err.clear();
   }
@@ -351,7 +356,8 @@ int run_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_t s
   if (ctx->scratch_stream && ctx->scratch_stream != st)
     JNE_HIP_CHECK(ctx, hipStreamWaitEvent(st, ctx->scratch_free, 0));
   if ((rc = launch_walks(ctx, models, n_models, dim, steps, rng_stream, d_seeds, d_z, n, precision, d_outs, st,
-                         ctx->d_acc, ctx->d_m, ctx->d_part, ctx->part_bytes / sizeof(double), chunk, true)))
+                         ctx->d_acc, ctx->d_m, captured ? nullptr : ctx->d_part,
+                         captured ? 0 : ctx->part_bytes / sizeof(double), chunk, true)))
     return rc;
   JNE_HIP_CHECK(ctx, hipEventRecord(ctx->scratch_free, st));
   ctx->scratch_stream = st;
