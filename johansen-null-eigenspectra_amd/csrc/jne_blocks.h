@@ -33,12 +33,10 @@
 namespace jne {
 
 // Steps per block: 240 (whole Philox calls and whole batches of every dim),
-// and at most 16 blocks per walk.  Up to 264 steps are one block: a second one
-// of at most 24 steps cost as much as 40 (12,000 to 50,001 walks at T = 250 and
-// 260, dims 9 to 12: up to 6% of the moment pass).
-constexpr uint32_t kBlockUnit = 240, kMaxBlocks = 16, kOneBlock = 264;
+// and at most 16 blocks per walk.
+constexpr uint32_t kBlockUnit = 240, kMaxBlocks = 16;
 __host__ __device__ constexpr uint32_t block_steps(uint32_t T) {
-  return T <= kOneBlock ? 2 * kBlockUnit : kBlockUnit * ((T + kBlockUnit * kMaxBlocks - 1) / (kBlockUnit * kMaxBlocks));
+  return kBlockUnit * ((T + kBlockUnit * kMaxBlocks - 1) / (kBlockUnit * kMaxBlocks));
 }
 __host__ __device__ constexpr uint32_t block_count(uint32_t T) { return (T + block_steps(T) - 1) / block_steps(T); }
 

@@ -1053,8 +1053,8 @@ static uint64_t split_units(uint32_t T, uint32_t m) { return ((uint64_t)m * T + 
 
 // Walks of n whose blocks one lane group takes in turn (the rest are split).
 // Whole rounds of the GPU's waves are taken in turn, and a rest of 90% of one with
-// them.  For the others both times are estimated, in steps of a SIMD with two
-// waves (one wave alone reaches 0.84 of its rate): in turn, the deepest SIMD's
+// them.  For the others both times are estimated, in steps of a SIMD with all
+// its waves (one alone reaches 0.84 of that rate): in turn, the deepest SIMD's
 // waves of T steps (less what starts while the rounds before end); split, the
 // rest's steps spread evenly, but no less than the deepest SIMD's whole blocks,
 // and the sums' way through memory with their launches (130 steps behind whole
@@ -1070,10 +1070,14 @@ static uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   if (block_count(T) == 1) return n > small ? n : 0;
   if (split_units(T, rest) <= small) return n - rest;
   if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
-  const auto deep = [](double w) { return w <= 1.0 ? 1.0 / 0.84 : std::ceil(w); };
+  const double full = L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d);
+  const auto deep = [full](double w) {  // time of ceil(w) waves: 0.84 of the full rate with one, linear between
+    const double k = std::max(1.0, std::ceil(w));
+    return k >= full ? k : k / (1.0 - 0.16 * (full - k) / (full - 1.0));
+  };
   const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
   const bool first = rest == n;
-  const double in_turn = first ? t * deep(w) : t * (std::ceil(w) - 0.145);
+  const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
   const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 0.0);
   return split < in_turn ? n - rest : n;
 }

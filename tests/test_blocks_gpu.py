@@ -72,8 +72,8 @@ def test_mixed_split_gives_the_same_bits(engine, jne, dim, steps):
 @pytest.mark.parametrize("dim,n", [(1, 70_000), (2, 90_000), (6, 66_000), (7, 52_500), (9, 20_000), (10, 40_000), (12, 20_000)])
 @pytest.mark.parametrize("steps", [264, 265, 333])
 def test_rounds_and_rests_give_the_same_bits(engine, O, dim, n, steps):
-    """The longest walk of one block and the shortest of two; whole rounds, rests taken in turn with
-    them and rests split, against the small batches' forms and the oracle."""
+    """Second blocks of 24, 25 and 93 steps; whole rounds, rests taken in turn with them and rests
+    split, against the small batches' forms and the oracle."""
     seeds = np.arange(9, 9 + n, dtype=np.uint32)
     full = engine.eigenvalues_by_seed(2, dim, steps, seeds)
     for at, m in [(0, 1), (n // 2, 700), (n - 2, 2)]:
