@@ -55,6 +55,7 @@
 #include "../../include/jne.h"
 #include "jne_internal.h"
 #include "jne_rng.h"
+#include "jne_segments.h"
 
 // Tuning: how many of a lane's Philox calls of a segment to unroll
 // (independent chains for the scheduler, at the cost of registers: 2 is the
@@ -93,7 +94,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kSegSteps = 64;  // steps per FP64 segment and per RNG round
 constexpr int kChunks = 4;     // 16-step MFMA chunks per segment
 constexpr int kRowC = 12;      // first row of the c block
 constexpr int kRowDet = 24;    // rows 24, 25, 26: 1, k, k(k-1)/2
@@ -364,18 +364,8 @@ __device__ __forceinline__ void seg_det(double* g, double a, double dt, double d
   g[2] += ((a * a) * P0 + (2.0 * a + 1.0) * P1 + 2.0 * P2) * dt2;
 }
 
-// Split batches (SPLIT): a segment's Gram as FP32 values, as the MFMA leaves
-// them, and its FP64 eps, in memory: per wave and segment kSegFloats floats
-//   c columns: rows 0..23 (accumulator v of half h of column j at v 24 + 12 h + j),
-//   z columns: rows 12..23 at 288 + 12 (row - 12) + j,
-//   rows 24..26 at 432 + 24 (row - 24) + j of the c, + 12 + j of the z columns,
-// then 12 doubles.
-constexpr int kSegFloats = 504;
-constexpr int kSegDoubles = kSegFloats / 2 + 12;
-constexpr int kSplitSegs = 4;  // segments per wave: a carry period (4 CALLS is a multiple of 64)
-
 // D: components of the wave (W walks of D / W each).  SPLIT: segments
-// kSplitSegs blockIdx.y .. + 3 of the wave's walks, to acc (see kSegFloats).
+// kSplitSegs blockIdx.y .. + 3 of the wave's walks, to acc (the layout at kSegFloats).
 template <int D, int PREC, bool FROM_NORMALS, int W = 1, bool SPLIT = false>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(PREC == JNE_PREC_FP32_KAHAN ? 2 : JNE_MFMA_WAVES)))
@@ -517,7 +507,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   const double dt = uniform_f64(1.0 / (double)T);
   const double s = uniform_f64(sqrt(dt));
   const double dt2 = uniform_f64(dt * dt);
-  const uint32_t rounds = (T + kSegSteps - 1) / kSegSteps;
+  const uint32_t rounds = segment_count(T);
   const uint32_t r0 = SPLIT ? blockIdx.y * kSplitSegs : 0;
   uint32_t drawn = r0 * (uint32_t)Sh::CALLS;  // calls drawn so far (carry form): a multiple of 64
 
@@ -864,7 +854,7 @@ __global__ __launch_bounds__(192) void mfma_segments_add(uint32_t T, uint32_t n_
   const int e = threadIdx.x;
   if (e >= D * D + 3 * D) return;
   const size_t walk = (size_t)blockIdx.x * W;
-  const uint32_t rounds = (T + kSegSteps - 1) / kSegSteps;
+  const uint32_t rounds = segment_count(T);
   const double* const p0 = part + (size_t)blockIdx.x * rounds * kSegDoubles;
   const double dt = 1.0 / (double)T, s = sqrt(dt), dt2 = dt * dt, s2 = s * s;
   auto len = [&](uint32_t r) {
@@ -930,20 +920,10 @@ __global__ __launch_bounds__(192) void mfma_segments_add(uint32_t T, uint32_t n_
   }
 }
 
-// fp16x2 batches by seed whose waves leave the GPU mostly idle are split over
-// their walks' segments: a segment then also writes and reads its 2.1 KB, as
-// long as its share of a full GPU's time, so the line lies where the two forms
-// meet (waves; in turn / split, ms): dim 12, T = 1,000: 400 0.039 / 0.026, 800
-// 0.040 / 0.043; T = 10^4: 1 0.307 / 0.06, 400 0.325 / 0.161, 800 0.330 / 0.267,
-// 1,200 0.387 / 0.417; dim 7, T = 400: 400 0.0196 / 0.0188, 800 0.0204 / 0.0218.
 static uint32_t mfma_wave_walks(int d) { return JNE_MFMA_PACK && 12 % d == 0 ? 12 / d : 1; }
-#ifndef JNE_MFMA_SPLIT_WAVES
-#define JNE_MFMA_SPLIT_WAVES 700
-#endif
 size_t mfma_part_doubles(int d, int precision, uint32_t T, uint32_t n) {
-  const uint32_t waves = (n + mfma_wave_walks(d) - 1) / mfma_wave_walks(d), rounds = (T + kSegSteps - 1) / kSegSteps;
-  if (precision != JNE_PREC_MFMA_FP16X2 || waves > JNE_MFMA_SPLIT_WAVES || rounds <= (uint32_t)kSplitSegs) return 0;
-  return (size_t)waves * rounds * kSegDoubles;
+  if (precision != JNE_PREC_MFMA_FP16X2) return 0;
+  return segment_split_doubles((n + mfma_wave_walks(d) - 1) / mfma_wave_walks(d), T);
 }
 
 template <int D, int PREC>
@@ -957,9 +937,8 @@ static hipError_t launch_mfma_dp(const uint32_t* seeds, const double* zin, uint3
   if constexpr (PREC == JNE_PREC_MFMA_FP16X2) {
     const size_t need = mfma_part_doubles(D, PREC, T, n);
     if (zin == nullptr && part != nullptr && need > 0 && need <= part_doubles) {
-      const unsigned chunks = ((T + kSegSteps - 1) / kSegSteps + kSplitSegs - 1) / kSplitSegs;
-      hipLaunchKernelGGL((walk_moments_mfma<DS, PREC, false, W, true>), dim3(grid, chunks), dim3(64), 0, st, seeds, zin,
-                         rng_stream, T, n, part, ld);
+      hipLaunchKernelGGL((walk_moments_mfma<DS, PREC, false, W, true>), dim3(grid, split_chunks(T)), dim3(64), 0, st,
+                         seeds, zin, rng_stream, T, n, part, ld);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL((mfma_segments_add<DS, W>), dim3(grid), dim3(192), 0, st, T, n, part, acc, ld);
