@@ -31,14 +31,18 @@ constexpr uint32_t split_chunks(uint32_t T) { return (segment_count(T) + kSplitS
 #ifndef JNE_MFMA_SPLIT_WAVES
 #define JNE_MFMA_SPLIT_WAVES 700
 #endif
+// The segments' sums grow with T (700 waves: 0.23 GB at T = 10^4, 23 GB at T =
+// 10^6) and stay with the context: a batch that needs more than this is not
+// split.  700 waves reach it at T = 11,585, one at T = 8.13 million.
+constexpr size_t kMaxSplitBytes = size_t(1) << 28;
 // A launch's chunks are its grid's y dimension, of which 65,535 are counted on.
-constexpr uint32_t kMaxSplitChunks = 65535;
+static_assert(kMaxSplitBytes / sizeof(double) / kSegDoubles / kSplitSegs < 65535, "one wave's chunks fit the grid");
 
 // Doubles of the segments' sums of a batch of `waves` waves (0: not split).
 constexpr size_t segment_split_doubles(uint32_t waves, uint32_t T) {
   if (waves > JNE_MFMA_SPLIT_WAVES || segment_count(T) <= (uint32_t)kSplitSegs) return 0;
-  if (split_chunks(T) > kMaxSplitChunks) return 0;
-  return (size_t)waves * segment_count(T) * kSegDoubles;
+  const size_t doubles = (size_t)waves * segment_count(T) * kSegDoubles;
+  return doubles <= kMaxSplitBytes / sizeof(double) ? doubles : 0;
 }
 
 }  // namespace jne

@@ -35,6 +35,13 @@ def test_chunks_fit_the_grid(rule):
                 assert 1 < rule.chunks(steps) <= 65_535, (waves, steps)
 
 
+def test_scratch_is_bounded(rule):
+    """The segments' sums grow with the walk's length and stay with the context: 256 MiB at most."""
+    for steps in STEPS:
+        for waves in WAVES:
+            assert 8 * rule.split_doubles(waves, steps) <= 1 << 28, (waves, steps)
+
+
 def test_small_batches_are_split(rule):
     assert rule.split_doubles(1, 256) == 0 and rule.split_doubles(1, 257) == 5 * 264
     assert rule.split_doubles(700, 10_000) == 700 * 157 * 264 and rule.split_doubles(701, 10_000) == 0
