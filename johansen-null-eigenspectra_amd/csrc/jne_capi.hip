@@ -279,12 +279,13 @@ int resolve_precision(int dim, uint32_t steps, int precision) {
   return auto_uses_mfma(dim, steps) ? JNE_PREC_MFMA_FP16X2 : JNE_PREC_FP64;
 }
 
-// Scratch for splitting a launch of n walks over their blocks (0: not split).
-size_t part_doubles_for(int dim, uint32_t steps, int precision, size_t n) {
+// Scratch for splitting a launch of n walks over their blocks (0: not split;
+// the reduced precisions split walks given by seed only).
+size_t part_doubles_for(int dim, uint32_t steps, int precision, bool by_seed, size_t n) {
   if (n == 0) return 0;
   if (dim > jne::kMaxDim) return jne::wide_part_doubles(dim, steps, (uint32_t)n);
   precision = resolve_precision(dim, steps, precision);
-  if (precision != JNE_PREC_FP64) return jne::mfma_part_doubles(dim, precision, steps, (uint32_t)n);
+  if (precision != JNE_PREC_FP64) return by_seed ? jne::mfma_part_doubles(dim, precision, steps, (uint32_t)n) : 0;
   return jne::fp64_part_doubles(dim, steps, (uint32_t)n);
 }
 
@@ -341,8 +342,8 @@ int run_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_t s
   rc = ensure(ctx, (void**)&ctx->d_m, &ctx->m_bytes, chunk * (size_t)jne::eigen_m_count(dim) * sizeof(double));
   if (rc) return rc;
   // without room for the blocks' sums the launches are not split
-  const size_t part = std::max(part_doubles_for(dim, steps, precision, chunk),
-                               part_doubles_for(dim, steps, precision, n % chunk));
+  const size_t part = std::max(part_doubles_for(dim, steps, precision, d_seeds != nullptr, chunk),
+                               part_doubles_for(dim, steps, precision, d_seeds != nullptr, n % chunk));
   // A captured call is not split: a smaller batch can need more room than a larger
   // one did, so a later call may replace the block sums' buffer under the graph.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

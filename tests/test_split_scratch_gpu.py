@@ -1,6 +1,7 @@
 """What a context's device memory grows by for a mixed batch split over its
 walks' segments: nothing past the split's bound, where the batch takes its
-segments in turn with the same bits."""
+segments in turn with the same bits, and nothing for walks from given normals,
+which are not split."""
 import ctypes
 
 import numpy as np
@@ -29,3 +30,13 @@ def test_a_batch_past_the_bound_is_not_split(jne):
             got = eng.eigenvalues_by_seed(4, dim, steps, seeds[at:at + m], precision=jne.PRECISIONS["mfma_fp16x2"])
             assert np.array_equal(got, full[at:at + m]), (at, m)
         assert before - free_bytes() < 1 << 27
+
+
+def test_given_normals_take_no_split_scratch(jne):
+    dim, n, steps = 12, 600, 1500  # split by seed: 30 MB
+    z = np.random.default_rng(3).standard_normal((n, steps, dim))
+    with jne.Engine(0) as eng:
+        eng.eigenvalues_from_normals(4, z, precision=jne.PRECISIONS["mfma_bf16x2"])  # the other scratch
+        before = free_bytes()
+        eng.eigenvalues_from_normals(4, z, precision=jne.PRECISIONS["mfma_fp16x2"])
+        assert before - free_bytes() < 1 << 23
