@@ -30,15 +30,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace jne {
+#include "jne_forms.h"
 
-// Steps per block: 240 (whole Philox calls and whole batches of every dim),
-// and at most 16 blocks per walk.
-constexpr uint32_t kBlockUnit = 240, kMaxBlocks = 16;
-__host__ __device__ constexpr uint32_t block_steps(uint32_t T) {
-  return kBlockUnit * ((T + kBlockUnit * kMaxBlocks - 1) / (kBlockUnit * kMaxBlocks));
-}
-__host__ __device__ constexpr uint32_t block_count(uint32_t T) { return (T + block_steps(T) - 1) / block_steps(T); }
+namespace jne {
 
 // Doubles of one block's sums: GE (d*d), GC (upper triangle), S, A1, A2, E.
 constexpr int block_moment_count(int d) { return d * d + d * (d + 1) / 2 + 4 * d; }

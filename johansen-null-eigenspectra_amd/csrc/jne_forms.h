@@ -1,0 +1,120 @@
+// jne_forms.h -- the shapes and forms of the FP64 moment passes: a walk's blocks of
+// steps, lanes per walk and waves by dim, and the rules by which a launch is
+// split.  Plain C++: the host tests of the rules build it without HIP.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <cmath>
+
+namespace jne {
+
+// Steps per block: 240 (whole Philox calls and whole batches of every dim),
+// and at most 16 blocks per walk.
+constexpr uint32_t kBlockUnit = 240, kMaxBlocks = 16;
+constexpr uint32_t block_steps(uint32_t T) {
+  return kBlockUnit * ((T + kBlockUnit * kMaxBlocks - 1) / (kBlockUnit * kMaxBlocks));
+}
+constexpr uint32_t block_count(uint32_t T) { return (T + block_steps(T) - 1) / block_steps(T); }
+
+// Per-dim shape of the FP64 moment kernel: lanes per walk (L) and target
+// waves per SIMD (the register cap).  Measured on MI355X at T = 4,000 to 10^4.
+// Dims with L = 1 run the register-only kernel (its own wave targets): at
+// dim 7 its 105 sums fit two waves per SIMD (131,072 walks at T = 10^4: 11.0
+// ms against 14.4 with seven lanes per walk); dim 8's 132 would not.
+// Alternatives within 2%: (2, 3) at dim 8, (3, 2) at dim 9; slower: (2, 2) at
+// dim 10 by 35%, (3, 2) at dims 11 and 12 by 8-11%.
+struct Fp64Shape {
+  int lanes, waves;
+};
+#ifndef JNE_FP64_SHAPES
+#define JNE_FP64_SHAPES \
+  {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {2, 2}, {9, 4}, {5, 3}, {4, 2}, {4, 2}
+#endif
+constexpr Fp64Shape kFp64Shapes[12] = {JNE_FP64_SHAPES};
+constexpr int lanes_for_dim(int d) { return kFp64Shapes[d - 1].lanes; }
+constexpr int waves_for_dim(int d) { return kFp64Shapes[d - 1].waves; }
+
+// target waves per SIMD of the register-only kernel by dim (the register cap:
+// 512 / waves VGPRs per lane); it runs the dims whose shape has one lane per walk.
+// One wave per SIMD reaches 88% of two waves' rate; 4 waves at dim 3 and 3 at
+// dim 4 are 3 and 4% faster than 3 and 2.
+#ifndef JNE_FP64_REG_WAVES
+#define JNE_FP64_REG_WAVES 4, 4, 4, 3, 2, 2, 2, 2, 2, 2, 2, 2
+#endif
+constexpr int kFp64RegWaves[12] = {JNE_FP64_REG_WAVES};
+
+// The forms of a moment launch.  One lane group per walk fills the GPU (the
+// waves resident at the kernel's occupancy) in whole rounds only; the walks of
+// the last, partial round are split over their blocks, as are all walks of a
+// batch too small for one lane group each.  With units = the walks' steps in
+// blocks of kBlockUnit, the split walks get
+//   one wave per block          up to kWaveForm units,
+//   one lane per component      up to kRowForm units (walk_moments_fp64, L = dim),
+//   the dim's own lane group    above.
+// The lines lie where two forms take the same time (T = 150 to 2,000; own
+// group / row / wave form, ms): dim 3, T = 240: 4,000 units 0.065 / 0.045 /
+// 0.044, 8,000 0.065 / 0.048 / 0.075, 30,000 0.068 / 0.067 / 0.24; dim 7:
+// 2,000 0.156 / 0.049 / 0.048, 30,000 0.171 / 0.127 / 0.42, 60,000 0.183 /
+// 0.205 / 0.81; dim 12: 2,000 0.110 / 0.060 / 0.078, 16,000 0.128 / 0.155 /
+// 0.46.  10,000 walks at T = 8,000, in turn and split: dim 1 0.607 and 0.112 ms,
+// dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
+constexpr uint32_t kSimds = 1024;
+#ifndef JNE_WAVE_FORM
+#define JNE_WAVE_FORM 3500, 4000, 5000, 4000, 4500, 4500, 2000, 1500, 1500, 1500, 1500, 1000
+#endif
+constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
+#ifndef JNE_ROW_FORM
+#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 52000, 24000, 0, 14000, 13000, 12000
+#endif
+constexpr uint32_t kRowForm[12] = {JNE_ROW_FORM};
+
+// Steps of m walks in blocks of 240.
+inline uint64_t split_units(uint32_t T, uint32_t m) { return ((uint64_t)m * T + kBlockUnit - 1) / kBlockUnit; }
+
+// Walks of n whose blocks one lane group takes in turn (the rest are split).
+// Whole rounds of the GPU's waves are taken in turn, and a rest of 90% of one with
+// them.  For the others both times are estimated, in steps of a SIMD with all
+// its waves (one alone reaches 0.84 of that rate): in turn, the deepest SIMD's
+// waves of T steps (less what starts while the rounds before end); split, the
+// rest's steps spread evenly, but no less than the deepest SIMD's whole blocks,
+// and the sums' way through memory with their launches (130 steps behind whole
+// rounds; else 40 of the short steps below dim 7, nothing that shows above).  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8
+// steps): 65,536 walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536
+// 0.179 and 0.207, 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593,
+// 170,000 1.324 and 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 12, T =
+// 1,000, 16,384 0.368 and 0.481, 50,001 1.226 and 1.378.
+inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
+  const uint32_t L = lanes_for_dim(d), wave = 64 / L;  // walks per wave
+  const uint32_t round = wave * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
+  const uint32_t rest = n % round, bn = block_steps(T), small = std::max(kWaveForm[d - 1], kRowForm[d - 1]);
+  if (block_count(T) == 1) return n > small ? n : 0;
+  if (split_units(T, rest) <= small) return n - rest;
+  if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
+  const double full = L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d);
+  const auto deep = [full](double w) {  // time of ceil(w) waves: 0.84 of the full rate with one, linear between
+    const double k = std::max(1.0, std::ceil(w));
+    return k >= full ? k : k / (1.0 - 0.16 * (full - k) / (full - 1.0));
+  };
+  const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
+  const bool first = rest == n;
+  const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
+  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 0.0);
+  return split < in_turn ? n - rest : n;
+}
+
+// Lanes per walk of a launch of n walks that is not split.  A lane per walk is
+// the better form at dim 7 once a wave per SIMD is nearly full, and again when
+// two are; fewer walks leave their chains exposed and run in groups of seven
+// lanes (ms in one lane / seven): T = 1,000: 1 walk 0.712 / 0.209, 12,000 0.736 /
+// 0.311, 55,000 0.796 / 0.700, 60,000 0.798 / 0.793, 65,000 0.802 / 0.871, 70,000
+// 1.209 / 0.909, 100,000 1.236 / 1.212; T = 240: 55,000 0.219 / 0.218, 70,000 0.336
+// / 0.278, 100,000 0.345 / 0.359.
+inline int fp64_turn_lanes(int d, uint32_t n) {
+  if (d == 7 && (n <= 55000 || (n > 64 * kSimds && n <= 95000))) return 7;
+  return lanes_for_dim(d);
+}
+
+}  // namespace jne

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "jne_forms.h"
+
 namespace jne {
 
 constexpr int kMaxDim = 12;      // the register-resident kernels (and the MFMA pass)
@@ -16,23 +18,6 @@ constexpr uint32_t kMaxSteps = 1u << 30;  // steps per walk accepted by the C AB
 // whose seed is wave-uniform on the scalar unit.
 static_assert((uint64_t)kMaxDim * kMaxSteps / 4 < (1ull << 32), "32-bit Philox counters");
 
-// Per-dim shape of the FP64 moment kernel: lanes per walk (L) and target
-// waves per SIMD (the register cap).  Measured on MI355X at T = 4,000 to 10^4.
-// Dims with L = 1 run the register-only kernel (its own wave targets): at
-// dim 7 its 105 sums fit two waves per SIMD (131,072 walks at T = 10^4: 11.0
-// ms against 14.4 with seven lanes per walk); dim 8's 132 would not.
-// Alternatives within 2%: (2, 3) at dim 8, (3, 2) at dim 9; slower: (2, 2) at
-// dim 10 by 35%, (3, 2) at dims 11 and 12 by 8-11%.
-struct Fp64Shape {
-  int lanes, waves;
-};
-#ifndef JNE_FP64_SHAPES
-#define JNE_FP64_SHAPES \
-  {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {1, 2}, {2, 2}, {9, 4}, {5, 3}, {4, 2}, {4, 2}
-#endif
-constexpr Fp64Shape kFp64Shapes[12] = {JNE_FP64_SHAPES};
-constexpr int lanes_for_dim(int d) { return kFp64Shapes[d - 1].lanes; }
-constexpr int waves_for_dim(int d) { return kFp64Shapes[d - 1].waves; }
 constexpr int gcd_int(int a, int b) { return b == 0 ? a : gcd_int(b, a % b); }
 
 // Steps per round of the FP64 moment kernel: a multiple of 4/gcd(d,4) (so a

@@ -15,8 +15,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 #include "jne_blocks.h"
@@ -107,6 +105,11 @@ struct Fp64Totals {
   int regs, lds;
 };
 constexpr Fp64Totals kFp64Totals[12] = {JNE_FP64_TOTALS};
+// of a lane group of LW lanes: the dim's own, or (a row of the sums per lane,
+// LW = D) all its slots in registers
+constexpr Fp64Totals group_totals(int d, int lw) {
+  return lw == lanes_for_dim(d) ? kFp64Totals[d - 1] : Fp64Totals{d + d / 2 + 4, 0};
+}
 
 template <int D, int LW, bool FROM_NORMALS, bool SPLIT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(group_waves(D, LW), group_waves(D, LW))))
@@ -126,7 +129,7 @@ void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restr
   static_assert(kBlockUnit % S == 0, "a block must be whole rounds");
   __shared__ double ws[S][RW][GP];
   __shared__ double bs[DP][GP];  // the state at the block's start
-  constexpr int NR = SPLIT ? 0 : kFp64Totals[D - 1].regs, NL = SPLIT ? 0 : kFp64Totals[D - 1].lds;
+  constexpr int NR = SPLIT ? 0 : group_totals(D, LW).regs, NL = SPLIT ? 0 : group_totals(D, LW).lds;
   __shared__ double tot_lds[NL > 0 ? NL : 1][64];
   Totals<NR, NL> tot;
   tot.lds = tot_lds;
@@ -359,15 +362,6 @@ void walk_moments_fp64(const uint32_t* __restrict__ seeds, const double* __restr
 // and 14.4, dim 6 20.1 and 17.4; dim 7 34.6 ms with seven lanes per walk
 // through LDS, 28.4 with the block sums there, 22 here.
 // ---------------------------------------------------------------------------
-// target waves per SIMD of the register-only kernel by dim (the register cap:
-// 512 / waves VGPRs per lane); it runs the dims whose shape has one lane per walk.
-// One wave per SIMD reaches 88% of two waves' rate; 4 waves at dim 3 and 3 at
-// dim 4 are 3 and 4% faster than 3 and 2.
-#ifndef JNE_FP64_REG_WAVES
-#define JNE_FP64_REG_WAVES 4, 4, 4, 3, 2, 2, 2, 2, 2, 2, 2, 2
-#endif
-constexpr int kFp64RegWaves[12] = {JNE_FP64_REG_WAVES};
-
 // Philox calls per batch by dim (a multiple of the calls of one whole-step
 // group: 1, 1, 3, 1, 5, 3 at dims 1..6)
 #ifndef JNE_FP64_REG_CALLS
@@ -1023,65 +1017,6 @@ __global__ __launch_bounds__(64) void walk_eigen_jacobi(const double* __restrict
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// The forms of a moment launch.  One lane group per walk fills the GPU (the
-// waves resident at the kernel's occupancy) in whole rounds only; the walks of
-// the last, partial round are split over their blocks, as are all walks of a
-// batch too small for one lane group each.  With units = the walks' steps in
-// blocks of kBlockUnit, the split walks get
-//   one wave per block          up to kWaveForm units,
-//   one lane per component      up to kRowForm units (walk_moments_fp64, L = dim),
-//   the dim's own lane group    above.
-// The lines lie where two forms take the same time (T = 150 to 2,000; own
-// group / row / wave form, ms): dim 3, T = 240: 4,000 units 0.065 / 0.045 /
-// 0.044, 8,000 0.065 / 0.048 / 0.075, 30,000 0.068 / 0.067 / 0.24; dim 7:
-// 2,000 0.156 / 0.049 / 0.048, 30,000 0.171 / 0.127 / 0.42, 60,000 0.183 /
-// 0.205 / 0.81; dim 12: 2,000 0.110 / 0.060 / 0.078, 16,000 0.128 / 0.155 /
-// 0.46.  10,000 walks at T = 8,000, in turn and split: dim 1 0.607 and 0.112 ms,
-// dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
-constexpr uint32_t kSimds = 1024;
-#ifndef JNE_WAVE_FORM
-#define JNE_WAVE_FORM 3500, 4000, 5000, 4000, 4500, 4500, 2000, 1500, 1500, 1500, 1500, 1000
-#endif
-constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
-#ifndef JNE_ROW_FORM
-#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 52000, 24000, 0, 14000, 13000, 12000
-#endif
-constexpr uint32_t kRowForm[12] = {JNE_ROW_FORM};
-
-// Steps of m walks in blocks of 240.
-static uint64_t split_units(uint32_t T, uint32_t m) { return ((uint64_t)m * T + kBlockUnit - 1) / kBlockUnit; }
-
-// Walks of n whose blocks one lane group takes in turn (the rest are split).
-// Whole rounds of the GPU's waves are taken in turn, and a rest of 90% of one with
-// them.  For the others both times are estimated, in steps of a SIMD with all
-// its waves (one alone reaches 0.84 of that rate): in turn, the deepest SIMD's
-// waves of T steps (less what starts while the rounds before end); split, the
-// rest's steps spread evenly, but no less than the deepest SIMD's whole blocks,
-// and the sums' way through memory with their launches (130 steps behind whole
-// rounds; else 40 of the short steps below dim 7, nothing that shows above).  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8
-// steps): 65,536 walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536
-// 0.179 and 0.207, 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593,
-// 170,000 1.324 and 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 12, T =
-// 1,000, 16,384 0.368 and 0.481, 50,001 1.226 and 1.378.
-static uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
-  const uint32_t L = lanes_for_dim(d), wave = 64 / L;  // walks per wave
-  const uint32_t round = wave * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
-  const uint32_t rest = n % round, bn = block_steps(T), small = std::max(kWaveForm[d - 1], kRowForm[d - 1]);
-  if (block_count(T) == 1) return n > small ? n : 0;
-  if (split_units(T, rest) <= small) return n - rest;
-  if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
-  const double full = L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d);
-  const auto deep = [full](double w) {  // time of ceil(w) waves: 0.84 of the full rate with one, linear between
-    const double k = std::max(1.0, std::ceil(w));
-    return k >= full ? k : k / (1.0 - 0.16 * (full - k) / (full - 1.0));
-  };
-  const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
-  const bool first = rest == n;
-  const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
-  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 0.0);
-  return split < in_turn ? n - rest : n;
-}
-
 size_t fp64_part_doubles(int d, uint32_t T, uint32_t n) {
   return (size_t)block_count(T) * block_moment_count(d) * (n - fp64_turns(d, T, n));
 }
@@ -1120,6 +1055,9 @@ static hipError_t launch_moments_d(const uint32_t* seeds, const double* zin, uin
   };
   uint32_t turns = fp64_turns(D, T, n);
   if (part == nullptr || part_doubles < fp64_part_doubles(D, T, n)) turns = n;
+  if constexpr (D == 7) {
+    if (turns == n && fp64_turn_lanes(D, n) == 7) return go(IntTag<7>{}, BoolTag<false>{}, seeds, zin, n, acc, ld);
+  }
   hipError_t e = hipSuccess;
   if (turns > 0) e = go(IntTag<L>{}, BoolTag<false>{}, seeds, zin, turns, acc, ld);
   if (e != hipSuccess || turns == n) return e;

@@ -1,5 +1,6 @@
-"""The rule that splits a small mixed batch over its walks' segments, built for
-the host (CPU), over every length the entry points accept (2 to 2^30 steps)."""
+"""The rules by which the moment passes choose a form, built for the host (CPU):
+the split of a small mixed batch over its walks' segments, over every length the
+entry points accept (2 to 2^30 steps), and the FP64 pass's forms."""
 import ctypes
 import os
 import shutil
@@ -45,3 +46,13 @@ def test_scratch_is_bounded(rule):
 def test_small_batches_are_split(rule):
     assert rule.split_doubles(1, 256) == 0 and rule.split_doubles(1, 257) == 5 * 264
     assert rule.split_doubles(700, 10_000) == 700 * 157 * 264 and rule.split_doubles(701, 10_000) == 0
+
+
+def test_unsplit_small_batches_of_dim_7_run_in_lane_groups(rule):
+    """One lane per walk needs a wave per SIMD to be the better form at dim 7 (one walk of 1,000
+    steps: 0.71 ms, in a group of seven lanes 0.21)."""
+    for walks in (1, 9, 1000, 12_000, 50_000, 70_000, 90_000):
+        assert rule.turn_lanes(7, walks) == 7, walks
+    for walks in (60_000, 65_536, 131_072, 262_144):
+        assert rule.turn_lanes(7, walks) == 1, walks
+    assert [rule.turn_lanes(d, 100) for d in (1, 6, 8, 9, 10, 12)] == [1, 1, 2, 9, 5, 4]
