@@ -49,49 +49,71 @@ constexpr int kFp64RegWaves[12] = {JNE_FP64_REG_WAVES};
 // The forms of a moment launch.  One lane group per walk fills the GPU (the
 // waves resident at the kernel's occupancy) in whole rounds only; the walks of
 // the last, partial round are split over their blocks, as are all walks of a
-// batch too small for one lane group each.  With units = the walks' steps in
-// blocks of kBlockUnit, the split walks get
-//   one wave per block          up to kWaveForm units,
-//   one lane per component      up to kRowForm units (walk_moments_fp64, L = dim),
+// batch too small for one lane group each.  A split costs a second launch and
+// the sums' way through memory, the time of some steps of the walk.  So the
+// split walks run, with units = their blocks (a last, short one counted by its
+// steps, a walk of one block as one),
+//   one wave per block          up to wave (1 - wave_t / T) units,
+//   one lane per component      up to row (1 - row_t / T) units (walk_moments_fp64, L = dim),
 //   the dim's own lane group    above.
-// The lines lie where two forms take the same time (T = 150 to 2,000; own
-// group / row / wave form, ms): dim 3, T = 240: 4,000 units 0.065 / 0.045 /
-// 0.044, 8,000 0.065 / 0.048 / 0.075, 30,000 0.068 / 0.067 / 0.24; dim 7:
-// 2,000 0.156 / 0.049 / 0.048, 30,000 0.171 / 0.127 / 0.42, 60,000 0.183 /
-// 0.205 / 0.81; dim 12: 2,000 0.110 / 0.060 / 0.078, 16,000 0.128 / 0.155 /
-// 0.46.  10,000 walks at T = 8,000, in turn and split: dim 1 0.607 and 0.112 ms,
-// dim 5 3.62 and 0.59, dim 12 3.60 and 1.85.
+// The lines are fitted to the calls' times in every form at 18 lengths from 10
+// to 10^4 steps and 15 batches from 1 to 100,000 walks of each dim: the chosen
+// form is 0.2% slower than the fastest on average and 2 to 20% at its worst
+// place by dim.  us of whole calls of model 4, in turn / own group / row / wave:
+//   dim 3:  T = 100, 3,000 walks 46 / 54 / 38 / 34, 12,000 49 / 56 / 43 / 67,
+//           22,000 52 / 60 / 58 / 103; T = 1,000, 2,000 walks 250 / 90 / 58 / 68
+//   dim 7:  T = 240, 1,000 walks (in groups of seven lanes) 86 / 197 / 88 / 73,
+//           2,000 87 / 195 / 87 / 85; T = 1,000, 500 walks 221 / 211 / 104 / 102, 22,000
+//           403 / 345 / 350
+//   dim 12: T = 120, 1,000 walks 149 / 160 / 133 / 127, 12,000 154 / 173 / 163; T =
+//           1,000, 500 walks 462 / 233 / 164 / 170, 3,000 481 / 269 / 273
 constexpr uint32_t kSimds = 1024;
-#ifndef JNE_WAVE_FORM
-#define JNE_WAVE_FORM 3500, 4000, 5000, 4000, 4500, 4500, 2000, 1500, 1500, 1500, 1500, 1000
+struct FormLines {
+  uint32_t wave, wave_t, row, row_t;
+};
+#ifndef JNE_FORM_LINES
+#define JNE_FORM_LINES                                                                                     \
+  {3500, 80, 0, 0}, {4000, 30, 32000, 80}, {5000, 10, 29000, 30}, {4000, 10, 48000, 20},                  \
+      {5000, 10, 47000, 30}, {4500, 10, 40000, 10}, {2250, 40, 52000, 10}, {2250, 10, 24000, 10},          \
+      {3000, 45, 0, 0}, {1500, 10, 11500, 30}, {1500, 10, 13000, 10}, {1250, 10, 11000, 10}
 #endif
-constexpr uint32_t kWaveForm[12] = {JNE_WAVE_FORM};
-#ifndef JNE_ROW_FORM
-#define JNE_ROW_FORM 0, 25000, 29000, 45000, 45000, 45000, 52000, 24000, 0, 14000, 13000, 12000
-#endif
-constexpr uint32_t kRowForm[12] = {JNE_ROW_FORM};
+constexpr FormLines kFormLines[12] = {JNE_FORM_LINES};
 
-// Steps of m walks in blocks of 240.
-inline uint64_t split_units(uint32_t T, uint32_t m) { return ((uint64_t)m * T + kBlockUnit - 1) / kBlockUnit; }
+enum class SplitForm { wave, row, own };
+inline SplitForm split_form(int d, uint32_t T, uint32_t m) {
+  const FormLines& l = kFormLines[d - 1];
+  const double t = (double)T, units = m * std::max(1.0, t / block_steps(T));
+  if (units <= l.wave * (1.0 - l.wave_t / t)) return SplitForm::wave;
+  if (units <= l.row * (1.0 - l.row_t / t)) return SplitForm::row;
+  return SplitForm::own;
+}
 
 // Walks of n whose blocks one lane group takes in turn (the rest are split).
-// Whole rounds of the GPU's waves are taken in turn, and a rest of 90% of one with
-// them.  For the others both times are estimated, in steps of a SIMD with all
-// its waves (one alone reaches 0.84 of that rate): in turn, the deepest SIMD's
-// waves of T steps (less what starts while the rounds before end); split, the
-// rest's steps spread evenly, but no less than the deepest SIMD's whole blocks,
-// and the sums' way through memory with their launches (130 steps behind whole
-// rounds; else 40 of the short steps below dim 7, nothing that shows above).  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8
-// steps): 65,536 walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536
-// 0.179 and 0.207, 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593,
-// 170,000 1.324 and 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 12, T =
-// 1,000, 16,384 0.368 and 0.481, 50,001 1.226 and 1.378.
+// Walks of one block have nothing to split but the lanes' work.  Whole rounds of
+// the GPU's waves are taken in turn, and a rest of 90% of one with them.  For the
+// others both times are estimated, in steps of a SIMD with all its waves (one
+// alone reaches 0.84 of that rate): in turn, the deepest SIMD's waves of T steps
+// (less what starts while the rounds before end); split, the rest's steps spread
+// evenly, but no less than the deepest SIMD's whole blocks, and the sums' way
+// through memory with their launches (130 steps behind whole rounds; else 40 of
+// the short steps below dim 7, 20 above).  The rates and steps are fitted to the
+// times.  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8 steps): 65,536
+// walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536 0.179 and 0.207,
+// 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593, 170,000 1.324 and
+// 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 9, T = 264, 12,000 0.143 and
+// 0.135; dim 10, T = 241, 30,000 0.274 and 0.255; dim 12, T = 1,000, 16,384 0.368 and
+// 0.481, 50,001 1.226 and 1.378.
 inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   const uint32_t L = lanes_for_dim(d), wave = 64 / L;  // walks per wave
   const uint32_t round = wave * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
-  const uint32_t rest = n % round, bn = block_steps(T), small = std::max(kWaveForm[d - 1], kRowForm[d - 1]);
-  if (block_count(T) == 1) return n > small ? n : 0;
-  if (split_units(T, rest) <= small) return n - rest;
+  const uint32_t rest = n % round, bn = block_steps(T);
+  // dim 7 in turn has a lane group per walk (fp64_turn_lanes), what the row form is
+  // without its second launch, so its walks of one block and a little more are
+  // split for the wave form only (T = 241, 12,000 walks: 0.114 ms in turn, 0.121 row;
+  // T = 300: 0.127 and 0.121)
+  if (d == 7 && T <= 270) return split_form(d, T, n) == SplitForm::wave ? 0 : n;
+  if (block_count(T) == 1) return split_form(d, T, n) == SplitForm::own ? n : 0;
+  if (split_form(d, T, rest) != SplitForm::own) return n - rest;
   if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
   const double full = L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d);
   const auto deep = [full](double w) {  // time of ceil(w) waves: 0.84 of the full rate with one, linear between
@@ -101,7 +123,7 @@ inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
   const bool first = rest == n;
   const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
-  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 0.0);
+  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 20.0);
   return split < in_turn ? n - rest : n;
 }
 

@@ -1065,13 +1065,11 @@ static hipError_t launch_moments_d(const uint32_t* seeds, const double* zin, uin
   const uint32_t m = n - turns;
   const uint32_t* s = seeds ? seeds + turns : nullptr;
   const double* z = zin ? zin + (size_t)turns * T * D : nullptr;
-  const uint64_t units = split_units(T, m);
-  if (units <= kWaveForm[D - 1])
-    e = go(IntTag<0>{}, BoolTag<true>{}, s, z, m, part, m);
-  else if (units <= kRowForm[D - 1])
-    e = go(IntTag<D>{}, BoolTag<true>{}, s, z, m, part, m);
-  else
-    e = go(IntTag<L>{}, BoolTag<true>{}, s, z, m, part, m);
+  switch (split_form(D, T, m)) {
+    case SplitForm::wave: e = go(IntTag<0>{}, BoolTag<true>{}, s, z, m, part, m); break;
+    case SplitForm::row: e = go(IntTag<D>{}, BoolTag<true>{}, s, z, m, part, m); break;
+    case SplitForm::own: e = go(IntTag<L>{}, BoolTag<true>{}, s, z, m, part, m); break;
+  }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(walk_blocks_add<D>, dim3((m + 63) / 64, AddShape<D>::NH), dim3(64 * D), 0, st, T, m, part,
                      acc + turns, ld);

@@ -56,3 +56,23 @@ def test_unsplit_small_batches_of_dim_7_run_in_lane_groups(rule):
     for walks in (60_000, 65_536, 131_072, 262_144):
         assert rule.turn_lanes(7, walks) == 1, walks
     assert [rule.turn_lanes(d, 100) for d in (1, 6, 8, 9, 10, 12)] == [1, 1, 2, 9, 5, 4]
+
+
+@pytest.mark.parametrize("dim", range(1, 13))
+def test_short_walks_are_not_split(rule, dim):
+    """A split launch's second kernel and its sums cost the time of some steps: the shortest walks
+    are never split, and those of one block in small batches only."""
+    for walks in (1, 100, 3000, 12_000, 30_000, 65_000):
+        for steps in range(2, 11):
+            assert rule.turns(dim, steps, walks) == walks, (steps, walks)
+    for steps in (2 * dim + 4, 40, 60):
+        for walks in (30_000, 45_000, 100_000):
+            if not (dim in (4, 6) and walks == 30_000):  # 1 to 3% either way
+                assert rule.turns(dim, steps, walks) == walks, (steps, walks)
+
+
+def test_forms_go_by_the_blocks_of_a_walk(rule):
+    """A walk has at most 16 blocks: a few long walks are few waves."""
+    assert [rule.form(d, 10_000, 100) for d in (1, 5, 8, 10)] == [0, 0, 0, 0]
+    assert rule.form(5, 11_000_000, 1) == 0 and rule.form(8, 10_000, 1000) == 1
+    assert rule.turns(8, 10_000, 1000) == 0 and rule.turns(12, 300, 20_000) == 0
