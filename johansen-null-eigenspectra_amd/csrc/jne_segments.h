@@ -23,14 +23,22 @@ constexpr int kSplitSegs = 4;  // segments per wave: a carry period (4 CALLS is 
 constexpr uint32_t split_chunks(uint32_t T) { return (segment_count(T) + kSplitSegs - 1) / kSplitSegs; }
 
 // fp16x2 batches by seed whose waves leave the GPU mostly idle are split over
-// their walks' segments: a segment then also writes and reads its 2.1 KB, as
-// long as its share of a full GPU's time, so the line lies where the two forms
-// meet (waves; in turn / split, ms): dim 12, T = 1,000: 400 0.039 / 0.026, 800
-// 0.040 / 0.043; T = 10^4: 1 0.307 / 0.06, 400 0.325 / 0.161, 800 0.330 / 0.267,
-// 1,200 0.387 / 0.417; dim 7, T = 400: 400 0.0196 / 0.0188, 800 0.0204 / 0.0218.
+// their walks' segments.  A segment then also writes and reads its 2.1 KB, as
+// long as its share of a full GPU's time, and the launch has a second kernel, the
+// time of some segments: the line lies where the two forms meet, at fewer waves
+// the fewer segments a walk has.  Split over in turn, whole calls of dim 12: 5
+// segments 100 waves 1.00, 700 1.03; 8 segments 400 0.99, 700 1.05; 16 segments 600
+// 0.96, 800 1.03; 157 segments 1 0.33, 700 0.76, 900 0.97, 1,000 1.04; of dim 5: 5
+// segments 100 1.00, 700 1.04; 8 segments 700 0.98; 157 segments 1,000 0.80.
 #ifndef JNE_MFMA_SPLIT_WAVES
-#define JNE_MFMA_SPLIT_WAVES 700
+#define JNE_MFMA_SPLIT_WAVES 950u
+#define JNE_MFMA_SPLIT_WAVES_LESS 4000u
 #endif
+constexpr uint32_t split_waves(uint32_t segments) {
+  const uint32_t less = JNE_MFMA_SPLIT_WAVES_LESS / segments;
+  return segments > (uint32_t)kSplitSegs && JNE_MFMA_SPLIT_WAVES > less ? JNE_MFMA_SPLIT_WAVES - less : 0;
+}
+
 // The segments' sums grow with T (700 waves: 0.23 GB at T = 10^4, 23 GB at T =
 // 10^6) and stay with the context: a batch that needs more than this is not
 // split.  700 waves reach it at T = 11,585, one at T = 8.13 million.
@@ -40,7 +48,7 @@ static_assert(kMaxSplitBytes / sizeof(double) / kSegDoubles / kSplitSegs < 65535
 
 // Doubles of the segments' sums of a batch of `waves` waves (0: not split).
 constexpr size_t segment_split_doubles(uint32_t waves, uint32_t T) {
-  if (waves > JNE_MFMA_SPLIT_WAVES || segment_count(T) <= (uint32_t)kSplitSegs) return 0;
+  if (waves > split_waves(segment_count(T))) return 0;
   const size_t doubles = (size_t)waves * segment_count(T) * kSegDoubles;
   return doubles <= kMaxSplitBytes / sizeof(double) ? doubles : 0;
 }

@@ -44,8 +44,14 @@ def test_scratch_is_bounded(rule):
 
 
 def test_small_batches_are_split(rule):
+    """The second kernel of a split costs the time of some segments: batches of walks of few
+    segments are split only if they are small."""
     assert rule.split_doubles(1, 256) == 0 and rule.split_doubles(1, 257) == 5 * 264
-    assert rule.split_doubles(700, 10_000) == 700 * 157 * 264 and rule.split_doubles(701, 10_000) == 0
+    assert rule.split_doubles(100, 300) and not rule.split_doubles(400, 300)
+    assert rule.split_doubles(300, 448) and not rule.split_doubles(600, 448)
+    assert rule.split_doubles(650, 1000) and not rule.split_doubles(800, 1000)
+    assert rule.split_doubles(701, 4000) and rule.split_doubles(800, 10_000) == 800 * 157 * 264
+    assert rule.split_doubles(1000, 10_000) == 0
 
 
 def test_unsplit_small_batches_of_dim_7_run_in_lane_groups(rule):
