@@ -364,11 +364,18 @@ __device__ __forceinline__ void seg_det(double* g, double a, double dt, double d
   g[2] += ((a * a) * P0 + (2.0 * a + 1.0) * P1 + 2.0 * P2) * dt2;
 }
 
+// Target waves per SIMD, at least and at most.  At most JNE_MFMA_WAVES for fp32 at
+// the small dims with a wave per walk, whose registers and LDS leave room for a 17th
+// wave per CU: one SIMD of four then ran five, and the others waited for it (8,000
+// walks of 1,000 x 5: 242 us so, 225 with four).
+constexpr int min_waves(int prec) { return prec == JNE_PREC_FP32_KAHAN ? 2 : JNE_MFMA_WAVES; }
+constexpr int max_waves(int d, int prec) { return prec == JNE_PREC_MFMA_FP32 && d <= 8 ? JNE_MFMA_WAVES : 8; }
+
 // D: components of the wave (W walks of D / W each).  SPLIT: segments
 // kSplitSegs blockIdx.y .. + 3 of the wave's walks, to acc (the layout at kSegFloats).
 template <int D, int PREC, bool FROM_NORMALS, int W = 1, bool SPLIT = false>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(PREC == JNE_PREC_FP32_KAHAN ? 2 : JNE_MFMA_WAVES)))
+__attribute__((amdgpu_waves_per_eu(min_waves(PREC), max_waves(D, PREC))))
 void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restrict__ zin, uint32_t rng_stream,
                        uint32_t T, uint32_t n_walks, double* __restrict__ acc, size_t ld) {
   constexpr int DW = D / W;  // components of one walk
