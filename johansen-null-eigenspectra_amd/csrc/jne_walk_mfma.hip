@@ -397,9 +397,15 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   float(*const zbuf)[ZP] = xs;
   float(*const cbuf)[ZP] = xs + kRowC;
   double* const gram = reinterpret_cast<double*>(rows_raw);
-  // sums of the scan blocks, block p of component i at [SP - 1 + p][i]: the SP - 1
-  // rows before a lane's own are those of the blocks before it and zeros
-  __shared__ __align__(16) double vecs[(2 * SP + 10) * D];  // one array: no padding between its parts
+  // sums of the scan blocks, block p of component i at [EP + p][i].  With fewer than
+  // eight scan lanes the EP = SP - 1 rows before a lane's own are those of the
+  // blocks before it and zeros, read again as its offset.  With eight (dims 5, 7
+  // and 8) a lane selects from the sums it has read: seven more LDS reads cost a
+  // wave alone 3-5% and the batches of up to a wave or two per SIMD with it (dim 8,
+  // T = 1,000, bf16x3: 5,000 walks 158 to 149 us, 1 walk 72 to 70; dim 5, fp16x2: 701
+  // walks 61.5 to 59, 100,000 walks 1.232 to 1.202 ms).
+  constexpr int EP = SP < 8 ? SP - 1 : 0;
+  __shared__ __align__(16) double vecs[(SP + EP + 11) * D];  // one array: no padding between its parts
   double(*const eps_part)[D] = reinterpret_cast<double(*)[D]>(vecs);
   // (not with the three-way bf16 split, whose operands leave no registers for it)
   constexpr bool kCarry = Sh::CARRY && !FROM_NORMALS && PREC != JNE_PREC_MFMA_BF16X3 && PREC != JNE_PREC_FP32_KAHAN;
@@ -411,7 +417,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   // walks at T = 10,000, dim 9: 14.7 to 14.0 ms)
   static_assert(!kCarry || Sh::CALLS * 4 <= D * ZP, "a segment's calls fit the c rows");
   float4* const zcall = reinterpret_cast<float4*>(&xs[kRowC][0]);
-  double* const seg_eps = vecs + (2 * SP - 1) * D;
+  double* const seg_eps = vecs + (SP + EP) * D;
   double* const b0s = seg_eps + D;  // B at the segment start (FP64)
   // per component j of a segment: b = B0 + s m (the state the centred c rows
   // are relative to), P = n b + s sig, Q = s sig, E = s eps, so that the
@@ -507,7 +513,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
   const int si = l % D, sp = l / D;
   const bool scan_lane = l < SP * D;
 
-  for (int e = l; e < (SP - 1) * D; e += 64) eps_part[e / D][e % D] = 0.0;
+  for (int e = l; e < EP * D; e += 64) eps_part[e / D][e % D] = 0.0;
   if (l < D) b0s[l] = 0.0;
   if (l < 3 * D) mb[l] = 0.0;
   // walk constants: uniform, held in scalar registers
@@ -624,7 +630,7 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
         }
         e = j ? e + (double)zb[j] : (double)zb[j];  // (no 0.0 + first term: one add fewer)
       });
-      eps_part[SP - 1 + sp][si] = e;
+      eps_part[EP + sp][si] = e;
     }
     __syncthreads();
 
@@ -633,16 +639,24 @@ void walk_moments_mfma(const uint32_t* __restrict__ seeds, const double* __restr
     // square, so the FP32 accumulation rounds less, and b_t = (B0 + s m) + s c_t.
     // Steps at or beyond T get c = 0 (their z are 0), so they add nothing.
     if (scan_lane) {
-      double e = eps_part[SP - 1][si];
+      double ep[SP];
 #pragma unroll
-      for (int p = 1; p < SP; ++p) e += eps_part[SP - 1 + p][si];
+      for (int p = 0; p < SP; ++p) ep[p] = eps_part[EP + p][si];
+      double e = ep[0];
+#pragma unroll
+      for (int p = 1; p < SP; ++p) e += ep[p];
       float m;
       const double bm = seg_state(SPLIT ? 0.0 : b0s[si], s, e, m);
       // running sum in FP64 (exact but for FP64 rounding): each c_t is then
       // rounded to FP32 once
       double c = -(double)m;
 #pragma unroll
-      for (int p = 0; p < SP - 1; ++p) c += eps_part[sp + p][si];
+      for (int p = 0; p < SP - 1; ++p) {
+        if constexpr (EP > 0)
+          c += eps_part[sp + p][si];
+        else
+          c += p < sp ? ep[p] : 0.0;
+      }
       float* const crow = &cbuf[si][sp * BS];
       block([&](int j) {
         crow[j] = (!tail || ts + (uint32_t)(sp * BS + j) < T) ? (float)c : 0.0f;
