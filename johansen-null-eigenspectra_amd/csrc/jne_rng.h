@@ -16,10 +16,11 @@
 // the stream is therefore bit-identical on any IEEE-754 host that performs
 // the same operations.  Three steps below are written in forms that reach the
 // same values with fewer instructions (the exponent split, the logarithm at
-// twice the scale, the quadrant turn); tests/test_transform_forms.py compares
-// them with the plain forms over every radius input the stream can produce
-// and the angle words near the quadrant edges, where a sign of zero could
-// differ.
+// twice the scale, the quadrant turn); tests/test_device_stream_forms.py builds
+// this header for the host and compares them with the plain forms over every
+// radius input the stream can produce and the angle words near the quadrant
+// edges, where a sign of zero could differ.  The square root is compared on the
+// GPU, at every radius word (jne_rng_check.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -98,10 +99,10 @@ __device__ __forceinline__ float two_ln(float u) {
 // Correctly rounded sqrt(y) for y = -0 or y = -two_ln(u1) of the stream:
 // g = y rsq(y) and one Newton step, g + (y - g^2) rsq(y)/2 (Markstein's final
 // step), whose error is about 1.5 times the square of v_rsq_f32's.  That does
-// not prove the last bit by itself: it was compared, on the GPU, with the
-// neighbour-residual form (v_sqrt_f32, then the neighbour whose residual has
-// the right sign) and with sqrt in double for every radius word (all 2^32):
-// no difference.  6 instructions instead of 9, without the half-rate compares
+// not prove the last bit by itself: jne_rng_check.hip compares it with what a
+// correctly rounded root is at every radius word (all 2^32), on the GPU: no
+// difference.  6 instructions instead of the 9 of v_sqrt_f32 and a step to the
+// neighbour whose residual has the right sign, without the half-rate compares
 // and selects (an instruction's issue measured 2.6 SIMD cycles at the full and
 // 4.4 at the half rate, 8.4 for v_sqrt_f32 and v_rsq_f32): with the exponent
 // split above, the stream alone went from 428 to 404 SIMD cycles per Philox
