@@ -43,15 +43,19 @@ extern "C" {
 #define JNE_PREC_MFMA_BF16X2 3 /* MFMA, bf16 hi+lo operands, fp32 accumulate */
 #define JNE_PREC_MFMA_BF16X3 4 /* MFMA, bf16 hi+mid+lo operands, fp32 accumulate */
 #define JNE_PREC_MFMA_FP32 5   /* MFMA, fp32 operands, fp32 accumulate */
-#define JNE_PREC_AUTO 6        /* per (dim, steps), the faster of FP64 and MFMA_FP16X2 */
+#define JNE_PREC_AUTO 6        /* FP64 or MFMA_FP16X2 by (dim, steps), see below */
 /* The MFMA modes keep the state B and the per-64-step segment terms in FP64
  * and put only within-segment corrections on the matrix cores.  Both paths
- * draw the same normals, whose generation bounds them both; measured on
- * MI355X the MFMA pass is faster for dim 12 from 200 steps, dims 10-11 from
- * 300, dim 9 from 500, dim 8 from 1,000 and dim 7 from 3,000 steps, so
- * JNE_PREC_AUTO runs MFMA_FP16X2
- * there and FP64 elsewhere (FP64 results meet the mixed-path tolerance
- * trivially). */
+ * draw the same normals, whose generation bounds them both.  JNE_PREC_AUTO
+ * runs MFMA_FP16X2 for dim 12 from 200 steps, dims 10-11 from 300, dim 9 from
+ * 500, dim 8 from 1,000 and dim 7 from 3,000 steps, and FP64 elsewhere (FP64
+ * results meet the mixed-path tolerance trivially).  The rule was drawn where
+ * the MFMA pass was the faster one and stays as it is, because which pass runs
+ * is part of a call's results.  The FP64 pass has become faster since: on
+ * MI355X it now leads at dim 7 (1.3x to 1.4x from 3,000 steps), at dim 8 (1.02x
+ * to 1.09x) and at dim 12 with 200 steps (1.14x), where a caller who wants the
+ * faster pass asks for JNE_PREC_FP64.  At dims 9-12 the MFMA pass leads from 500
+ * steps (1.14x to 1.29x at 10,000). */
 
 /* Dims 1..JNE_MAX_DIM run on the device.  The reduced-precision moment
  * passes (the MFMA modes and JNE_PREC_FP32_KAHAN) cover dims
@@ -104,7 +108,16 @@ int jne_eigenvalues_by_seed(jne_ctx *ctx, int model, int dim, uint32_t steps, ui
  * returns without synchronising.  Non-positive-definite walks yield NaN rows;
  * no host-side check is made.  The context's device scratch is shared by its
  * calls: a call on another stream than the previous call first waits (on the
- * device) for the previous call's use of it. */
+ * device) for the previous call's use of it.  It grows to the largest need of
+ * the calls made and stays until jne_destroy: the moments and eigen matrices of
+ * up to 2^18 walks at a time (8 (2.5 dim^2 + 6.5 dim + 1) bytes per walk up to dim
+ * 12, 8 (2 dim^2 + 6 dim) of up to about 1 GiB above), and, for batches whose
+ * walks are split to fill the GPU, partial sums of at most 1.5 GiB (FP64) or
+ * 256 MiB (MFMA_FP16X2).  A batch is not split where that memory is not to be had,
+ * nor while the stream is being captured into a graph (the graph would keep a
+ * pointer to memory that a later call may replace): the same bits, but a small
+ * batch then takes its walks' serial time.  jne_eigenvalues_by_seed_device_noalloc
+ * splits under capture too, as far as its fixed scratch has room. */
 int jne_eigenvalues_by_seed_device(jne_ctx *ctx, int model, int dim, uint32_t steps, uint32_t rng_stream,
                                    const uint32_t *d_seeds, size_t n, int precision, double *d_out,
                                    void *hip_stream);
@@ -171,8 +184,8 @@ int jne_walk_normals_device(jne_ctx *ctx, int dim, uint32_t steps, uint32_t rng_
 /* Percentiles p[0..np) (1 <= np <= 8, each in [0, 1]) of the device array
  * d_values[0..n), n < 2^31, into the host array out[np]: rank p*(n-1),
  * linear interpolation between the neighbouring order statistics, the same
- * values as jne_percentiles, found on the device by bucket selection (a sort
- * only when ties crowd the selected buckets).  Synchronous on hip_stream
+ * values as jne_percentiles, found on the device by bucket selection (by radix
+ * select when ties or outliers crowd the selected buckets).  Synchronous on hip_stream
  * (see JNE_STREAM_CONTEXT); n = 0 gives NaN as jne_percentiles.  The
  * device counterpart of get_percentile_value (src/simulation_analyzers.rs:4-18),
  * used by the query server; NaN values are JNE_ERR_NUMERIC. */
@@ -302,10 +315,13 @@ int jne_run_simulation_models(jne_ctx *ctx, const int *models, int n_models, int
  * Walk w (0-based) of a query is walk seed w+1 with Philox key word `seed`,
  * so a query's result depends only on (model, dim, steps, runs, seed,
  * precision): the same alone and in any mix of concurrent queries.
- * Queries are admitted in arrival order when their device footprint
- * (16 bytes per walk) fits the HBM budget; admitted queries share `lanes`
+ * Queries are admitted in arrival order when their per-walk statistics
+ * (16 bytes per walk) fit the HBM budget; admitted queries share `lanes`
  * launch streams chunk by chunk (continuous batching), a free stream taking
- * the next chunk of the query with the least work left.  The quantiles are
+ * the next chunk of the query with the least work left.  Outside the budget
+ * each lane has a context of its own with the scratch of chunks of up to 65,536
+ * walks (see jne_eigenvalues_by_seed_device), grown by the chunks it runs: up to
+ * 1.3 GB after queries of dims 1..12, up to 2.3 GB after some of dim 32 too.  The quantiles are
  * selected on the device (bucket selection of the per-walk statistics, as
  * jne_percentiles_device); only the six values come back to the host.
  * ------------------------------------------------------------------------ */

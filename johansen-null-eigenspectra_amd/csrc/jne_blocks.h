@@ -14,9 +14,10 @@
 //   sum (t+1)^2 b   += B sum (t+1)^2 + te^2 S - 2 te A1 + 2 A2 + A1
 //   B               += E
 //
-// A1 and A2 are the running sums of S and A1 (each added before its source is
-// advanced): A1 = sum m c, A2 = sum m (m - 1)/2 c with m = te - (t+1), so the
-// kernels form no powers of t.  The moments of the increments follow from the
+// A1 = sum m c and A2 = sum m (m - 1)/2 c with m = te - (t+1).  The kernels of dims
+// 1..12 form them as the running sums of S and A1 (each added before its source is
+// advanced), with no powers of t; those of the wide dims, whose lanes take every
+// fourth step, with the weights m and m (m - 1)/2.  The moments of the increments follow from the
 // others by summation by parts: sum (t+1) z = T B_T - sum b and
 // sum (t+1)^2 z = T^2 B_T - 2 sum (t+1) b + sum b.  Everything is unscaled
 // until the end, where e = s z and b scale by s = sqrt(1/T).

@@ -258,12 +258,17 @@ hipError_t timed_launch(jne_ctx* ctx, int kernel, uint64_t walks, hipStream_t st
 }
 
 // Enqueue the walk path for n walks (device pointers) on stream st.
-// JNE_PREC_AUTO: the MFMA pass where it measured faster than the FP64 pass
-// (walks/s of the whole path, model 4, T = 100..10^4): dim 12 from 200 steps,
-// dims 10-11 from 300, dim 9 from 500, dim 8 from 1,000 and dim 7 from 3,000;
-// short walks carry the MFMA pass's per-walk setup.  At dims 1-6 the FP64 pass
-// keeps each walk in one lane's registers and runs 1.2-1.45x the MFMA pass
-// (which packs 12 / dim walks per wave at 1, 2, 3, 4 and 6).
+// JNE_PREC_AUTO: the MFMA pass for dim 12 from 200 steps, dims 10-11 from 300,
+// dim 9 from 500, dim 8 from 1,000 and dim 7 from 3,000; short walks carry its
+// per-walk setup.  The lines were drawn where the two passes met (walks/s of the
+// whole path, model 4, 262,144 walks) before the FP64 pass took blocks of steps,
+// and stay, because which pass runs is part of a call's results.  Measured since,
+// FP64 / MFMA in M walks/s: dim 7, T = 3,000 37.3 / 28.2, 10,000 11.9 / 8.7; dim 8,
+// 1,000 83.7 / 76.5, 10,000 9.1 / 8.4; dim 9, 300 168 / 159, 500 110 / 112, 1,000 57.8
+// / 63.9; dim 10, 200 200 / 179, 300 139 / 152; dim 11, 200 168 / 157, 300 118 / 135;
+// dim 12, 200 172 / 150, 300 122 / 135, 10,000 5.0 / 6.3.  At dims 1-6 the FP64 pass
+// keeps each walk in one lane's registers and leads by 1.2x or more (dim 6: 1.2-1.4x)
+// over the MFMA pass, which packs 12 / dim walks per wave at 1, 2, 3, 4 and 6.
 bool auto_uses_mfma(int dim, uint32_t steps) {
   if (dim > JNE_MAX_MIXED_DIM) return false;
   if (dim == 12) return steps >= 200;
@@ -306,10 +311,12 @@ int launch_walks(jne_ctx* ctx, const int* models, int n_models, int dim, uint32_
     const uint32_t* s = d_seeds ? d_seeds + off : nullptr;
     const double* z = d_z ? d_z + off * (size_t)steps * dim : nullptr;
     auto moments = [&] {
-      if (dim > jne::kMaxDim) 
+      if (dim > jne::kMaxDim)
         return jne::launch_walk_moments_wide(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
-      if (precision == JNE_PREC_FP64) return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
-      return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
+      if (precision == JNE_PREC_FP64)
+        return jne::launch_walk_moments_fp64(dim, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles, st);
+      return jne::launch_walk_moments_mfma(dim, precision, s, z, rng_stream, steps, cn, acc, cn, part, part_doubles,
+                                           st);
     };
     if (timed)
       JNE_HIP_CHECK(ctx, timed_launch(ctx, JNE_KERNEL_MOMENTS, cn, st, moments));

@@ -22,7 +22,7 @@
 //
 // 10^6 values: 127 to 63 us a call.  Before, 1,024 workgroups met in atomics on
 // one min and max (27 us, now 6 with a min and max per workgroup), 512 added
-// their 8,192 counts (25 us, now 61 groups in 8), the select walked its scans
+// their 8,192 counts (25 us, now 62 groups in 8), the select walked its scans
 // in one thread (26 us, now 8) and a copy brought the results back.  Ending a
 // pass in its last workgroup instead of a launch was slower: the fence that
 // makes the others' writes visible cost 70 us.
@@ -79,7 +79,8 @@ struct QsArgs {
 };
 
 // Workgroups of a pass over an array: up to kMaxGroups, for the histogram (whose
-// LDS copy each group adds to the array's) of at least 16,384 values each.
+// LDS copy each group adds to the array's) of up to about 16,384 values each until
+// kMaxGroups take more.
 constexpr unsigned kMaxGroups = 256;
 unsigned pass_groups(uint64_t n, uint64_t per) {
   const uint64_t g = (n + per - 1) / per;

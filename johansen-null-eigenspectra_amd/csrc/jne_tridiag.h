@@ -218,8 +218,9 @@ JNE_TRI_HD double sturm_scale(double* d, double* e2, int n, double& lo, double& 
 // leading minors of T - x, p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, which
 // take three FP64 operations each where the ratios p_i / p_{i-1} take a
 // reciprocal (the same backward error, a few ulp of |T|).  A term grows at most
-// 5-fold, and two terms shrink at most 2^-201-fold, so eight steps from a pair of
-// size one neither overflow nor underflow.
+// 5-fold (|d_i - x| <= 5 with the padding, whose e_i^2 are zero; below n, |d_i - x|
+// and e_i^2 are at most 2 and 1), and two terms shrink at most 2^-201-fold, so eight
+// steps from a pair of size one neither overflow nor underflow.
 template <int NMAX>
 JNE_TRI_HD int sturm_count(const double* d, const double* e2, int n, double x) {
   double p0 = 1.0, p1 = d[0] - x;
@@ -250,7 +251,8 @@ JNE_TRI_HD int sturm_count(const double* d, const double* e2, int n, double x) {
 
 // Eigenvalue k (0-based, ascending) of T by `iters` halvings of [lo, hi] (the
 // one-lane form; the wave-parallel solve runs the same counts at several
-// points per round).
+// points per round).  Math and the unnamed pivmin are for counts by ratios; these
+// counts need neither.
 // From the Gershgorin interval (width <= 2 |T|), 54 halvings leave a width of
 // at most 2^-53 |T|.
 template <int NMAX, class Math>
