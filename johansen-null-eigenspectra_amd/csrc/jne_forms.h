@@ -80,12 +80,16 @@ struct FormLines {
 constexpr FormLines kFormLines[12] = {JNE_FORM_LINES};
 
 enum class SplitForm { wave, row, own };
+inline double split_units(uint32_t T, uint32_t m) { return m * std::max(1.0, (double)T / block_steps(T)); }
+inline double wave_line(int d, uint32_t T) { return kFormLines[d - 1].wave * (1.0 - kFormLines[d - 1].wave_t / (double)T); }
+inline double row_line(int d, uint32_t T) { return kFormLines[d - 1].row * (1.0 - kFormLines[d - 1].row_t / (double)T); }
 inline SplitForm split_form(int d, uint32_t T, uint32_t m) {
-  const FormLines& l = kFormLines[d - 1];
-  const double t = (double)T, units = m * std::max(1.0, t / block_steps(T));
-  if (units <= l.wave * (1.0 - l.wave_t / t)) return SplitForm::wave;
-  if (units <= l.row * (1.0 - l.row_t / t)) return SplitForm::row;
-  return SplitForm::own;
+  const double units = split_units(T, m);
+  return units <= wave_line(d, T) ? SplitForm::wave : units <= row_line(d, T) ? SplitForm::row : SplitForm::own;
+}
+// m walks' part of what the row and wave forms take
+inline double form_load(int d, uint32_t T, uint32_t m) {
+  return split_units(T, m) / std::max(wave_line(d, T), row_line(d, T));
 }
 
 // Walks of n whose blocks one lane group takes in turn (the rest are split).
@@ -103,6 +107,11 @@ inline SplitForm split_form(int d, uint32_t T, uint32_t m) {
 // 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 9, T = 264, 12,000 0.143 and
 // 0.135; dim 10, T = 241, 30,000 0.274 and 0.255; dim 12, T = 1,000, 16,384 0.368 and
 // 0.481, 50,001 1.226 and 1.378.
+// A rest small enough for the row or wave form is split up to dim 8; at dims 9-12,
+// whose own groups need fewer walks to fill the GPU, it is split where the form's
+// time, which grows with its units, is under the time in turn (split and in turn,
+// ms: dim 11, T = 241, 45,000 walks 0.452 and 0.418, 67,236 0.571 and 0.594; dim 10, T
+// = 300, 45,000 0.400 and 0.382; dim 12, T = 1,000, 100,000 2.41 and 2.60).
 inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   const uint32_t L = lanes_for_dim(d), wave = 64 / L;  // walks per wave
   const uint32_t round = wave * kSimds * (L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d));
@@ -113,7 +122,9 @@ inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   // T = 300: 0.127 and 0.121)
   if (d == 7 && T <= 270) return split_form(d, T, n) == SplitForm::wave ? 0 : n;
   if (block_count(T) == 1) return split_form(d, T, n) == SplitForm::own ? n : 0;
-  if (split_form(d, T, rest) != SplitForm::own) return n - rest;
+  const bool first = rest == n;
+  const SplitForm form = split_form(d, T, rest);
+  if (form != SplitForm::own && (first || rest == 0 || d <= 8)) return n - rest;
   if ((uint64_t)rest * 100 >= (uint64_t)round * 90) return n;
   const double full = L == 1 ? kFp64RegWaves[d - 1] : waves_for_dim(d);
   const auto deep = [full](double w) {  // time of ceil(w) waves: 0.84 of the full rate with one, linear between
@@ -121,9 +132,11 @@ inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
     return k >= full ? k : k / (1.0 - 0.16 * (full - k) / (full - 1.0));
   };
   const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
-  const bool first = rest == n;
   const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
-  const double split = std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 20.0);
+  const double split =
+      form != SplitForm::own
+          ? bn * (full > 2.0 ? 0.5 + 0.8 * form_load(d, T, rest) : 0.1 + 0.5 * form_load(d, T, rest)) + 115.0
+          : std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 20.0);
   return split < in_turn ? n - rest : n;
 }
 

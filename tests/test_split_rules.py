@@ -82,3 +82,12 @@ def test_forms_go_by_the_blocks_of_a_walk(rule):
     assert [rule.form(d, 10_000, 100) for d in (1, 5, 8, 10)] == [0, 0, 0, 0]
     assert rule.form(5, 11_000_000, 1) == 0 and rule.form(8, 10_000, 1000) == 1
     assert rule.turns(8, 10_000, 1000) == 0 and rule.turns(12, 300, 20_000) == 0
+
+
+def test_a_rest_is_split_where_that_is_faster(rule):
+    """Dims 9-12 behind whole rounds of the GPU: a rest that the row form would take is left in turn
+    where the two blocks of a walk just above 240 steps gain less than the split costs."""
+    for dim, steps, walks in ((11, 241, 45_000), (11, 255, 75_000), (12, 241, 75_000), (10, 241, 45_000), (10, 300, 45_000)):
+        assert rule.turns(dim, steps, walks) == walks, (dim, steps, walks)
+    assert rule.turns(11, 1000, 100_000) == 98_304 and rule.turns(12, 1000, 100_000) == 98_304
+    assert rule.turns(8, 241, 75_000) == 65_536 and rule.turns(5, 241, 140_000) == 131_072
