@@ -74,7 +74,7 @@ struct FormLines {
 #ifndef JNE_FORM_LINES
 #define JNE_FORM_LINES                                                                                     \
   {3500, 80, 0, 0}, {4000, 30, 32000, 80}, {5000, 10, 29000, 30}, {4000, 10, 48000, 20},                  \
-      {5000, 10, 47000, 30}, {4500, 10, 40000, 10}, {2250, 40, 52000, 10}, {2250, 10, 24000, 10},          \
+      {5000, 10, 47000, 30}, {4500, 10, 40000, 10}, {2250, 40, 54000, 10}, {2250, 10, 24000, 10},          \
       {3000, 45, 0, 0}, {1500, 10, 11500, 30}, {1500, 10, 13000, 10}, {1250, 10, 11000, 10}
 #endif
 constexpr FormLines kFormLines[12] = {JNE_FORM_LINES};
@@ -92,6 +92,18 @@ inline double form_load(int d, uint32_t T, uint32_t m) {
   return split_units(T, m) / std::max(wave_line(d, T), row_line(d, T));
 }
 
+// Lanes per walk of a launch of n walks that is not split.  A lane per walk is
+// the better form at dim 7 once a wave per SIMD is nearly full, and again when
+// two are; fewer walks leave their chains exposed and run in groups of seven
+// lanes (ms in one lane / seven): T = 1,000: 1 walk 0.712 / 0.209, 12,000 0.736 /
+// 0.311, 55,000 0.796 / 0.700, 60,000 0.798 / 0.793, 65,000 0.802 / 0.871, 70,000
+// 1.209 / 0.909, 100,000 1.236 / 1.212; T = 240: 55,000 0.219 / 0.218, 70,000 0.336
+// / 0.278, 100,000 0.345 / 0.359.
+inline int fp64_turn_lanes(int d, uint32_t n) {
+  if (d == 7 && (n <= 55000 || (n > 64 * kSimds && n <= 95000))) return 7;
+  return lanes_for_dim(d);
+}
+
 // Walks of n whose blocks one lane group takes in turn (the rest are split).
 // Walks of one block have nothing to split but the lanes' work.  Whole rounds of
 // the GPU's waves are taken in turn, and a rest of 90% of one with them.  For the
@@ -100,13 +112,14 @@ inline double form_load(int d, uint32_t T, uint32_t m) {
 // (less what starts while the rounds before end); split, the rest's steps spread
 // evenly, but no less than the deepest SIMD's whole blocks, and the sums' way
 // through memory with their launches (130 steps behind whole rounds; else 40 of
-// the short steps below dim 7, 20 above).  The rates and steps are fitted to the
+// the short steps below dim 7, 35 at dim 7, 20 above).  The rates and steps are fitted to the
 // times.  Split and in turn, ms: dim 6, T = 248 (blocks of 240 and 8 steps): 65,536
 // walks 0.168 and 0.162, 170,000 0.409 and 0.365; T = 333: 65,536 0.179 and 0.207,
 // 170,000 0.491 and 0.477; T = 1,000: 65,536 0.485 and 0.593, 170,000 1.324 and
 // 1.399; dim 2, T = 248, 90,000 0.075 and 0.067; dim 9, T = 264, 12,000 0.143 and
 // 0.135; dim 10, T = 241, 30,000 0.274 and 0.255; dim 12, T = 1,000, 16,384 0.368 and
-// 0.481, 50,001 1.226 and 1.378.
+// 0.481, 50,001 1.226 and 1.378; dim 7 (in turn in groups of seven lanes), T = 480,
+// 36,000 0.329 and 0.273, 50,000 0.337 and 0.363.
 // A rest small enough for the row or wave form is split up to dim 8; at dims 9-12,
 // whose own groups need fewer walks to fill the GPU, it is split where the form's
 // time, which grows with its units, is under the time in turn (split and in turn,
@@ -120,7 +133,7 @@ inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
   // without its second launch, so its walks of one block and a little more are
   // split for the wave form only (T = 241, 12,000 walks: 0.114 ms in turn, 0.121 row;
   // T = 300: 0.127 and 0.121)
-  if (d == 7 && T <= 270) return split_form(d, T, n) == SplitForm::wave ? 0 : n;
+  if (d == 7 && T <= 270 && n < round) return split_form(d, T, n) == SplitForm::wave ? 0 : n;
   if (block_count(T) == 1) return split_form(d, T, n) == SplitForm::own ? n : 0;
   const bool first = rest == n;
   const SplitForm form = split_form(d, T, rest);
@@ -132,24 +145,15 @@ inline uint32_t fp64_turns(int d, uint32_t T, uint32_t n) {
     return k >= full ? k : k / (1.0 - 0.16 * (full - k) / (full - 1.0));
   };
   const double w = (double)((rest + wave - 1) / wave) / kSimds, t = (double)T;
-  const double in_turn = first ? t * deep(w) : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
+  // dim 7's groups of seven lanes: nine walks per wave, four waves per SIMD
+  const double in_turn = first && d == 7 && fp64_turn_lanes(d, n) == 7 ? t * (0.2 + 0.147 * std::ceil(n / (9.0 * kSimds)))
+                         : first ? t * deep(w)
+                                 : t * ((full > 2.0 ? deep(w) : std::ceil(w)) - 0.145);
   const double split =
       form != SplitForm::own
           ? bn * (full > 2.0 ? 0.5 + 0.8 * form_load(d, T, rest) : 0.1 + 0.5 * form_load(d, T, rest)) + 115.0
-          : std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : 20.0);
+          : std::max(t * w, bn * deep(w * (T / bn))) + (!first ? 130.0 : d < 7 ? 40.0 : d == 7 ? 35.0 : 20.0);
   return split < in_turn ? n - rest : n;
-}
-
-// Lanes per walk of a launch of n walks that is not split.  A lane per walk is
-// the better form at dim 7 once a wave per SIMD is nearly full, and again when
-// two are; fewer walks leave their chains exposed and run in groups of seven
-// lanes (ms in one lane / seven): T = 1,000: 1 walk 0.712 / 0.209, 12,000 0.736 /
-// 0.311, 55,000 0.796 / 0.700, 60,000 0.798 / 0.793, 65,000 0.802 / 0.871, 70,000
-// 1.209 / 0.909, 100,000 1.236 / 1.212; T = 240: 55,000 0.219 / 0.218, 70,000 0.336
-// / 0.278, 100,000 0.345 / 0.359.
-inline int fp64_turn_lanes(int d, uint32_t n) {
-  if (d == 7 && (n <= 55000 || (n > 64 * kSimds && n <= 95000))) return 7;
-  return lanes_for_dim(d);
 }
 
 }  // namespace jne

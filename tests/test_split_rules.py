@@ -91,3 +91,10 @@ def test_a_rest_is_split_where_that_is_faster(rule):
         assert rule.turns(dim, steps, walks) == walks, (dim, steps, walks)
     assert rule.turns(11, 1000, 100_000) == 98_304 and rule.turns(12, 1000, 100_000) == 98_304
     assert rule.turns(8, 241, 75_000) == 65_536 and rule.turns(5, 241, 140_000) == 131_072
+
+
+def test_dim_7_is_split_where_that_beats_its_lane_groups(rule):
+    for steps, walks in ((400, 36_000), (480, 36_000), (480, 45_000), (480, 70_000)):
+        assert rule.turns(7, steps, walks) == walks, (steps, walks)
+    for steps, walks in ((480, 50_000), (480, 30_000), (1000, 36_000), (1000, 55_000), (333, 50_001)):
+        assert rule.turns(7, steps, walks) == 0, (steps, walks)
